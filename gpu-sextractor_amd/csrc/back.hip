@@ -4,9 +4,9 @@
  *
  * Kernels:
  *   k_meshstat   backstat (back.c:214-290).  The double sums of pix and pix^2 are
- *                sequential in raster order inside the mesh, as back.c does, so one lane
- *                runs each sum's chain; three wavefronts of the workgroup stream the mesh
- *                rows through a double-buffered LDS ring meanwhile.
+ *                sequential in raster order inside the mesh, as in back.c; the mesh is cut
+ *                into runs, every lane finds what its run adds to the sequential sum, bit
+ *                for bit, and one wavefront walks the runs.
  *   k_meshmode   one workgroup per mesh: histogram in LDS (back.c:297-341), then the
  *                clipped-mode iteration of backguess (back.c:347-426) on one wavefront.
  *                Inside the iteration every sum is an exact integer (< 2^53), so the
@@ -31,6 +31,7 @@
 #include <vector>
 
 #include "sxg_internal.h"
+#include "sxg_wave.h"
 
 #define QUANTIF_NSIGMA 5
 #define QUANTIF_AMIN 4
@@ -81,255 +82,376 @@ __device__ inline void meshstat_pass2_end(const MeshAcc &a, MeshStat &o)
     o.qzero = (float)(mean - QUANTIF_NSIGMA * sigma);
 }
 
+#define MS_LDS_BYTES (144 * 1024)
+/* the largest mesh (pixels) of the one-, two- and four-wavefront kernels */
+#define MS_PX1 2048
+#define MS_PX2 8192
+#define MS_PX4 20000
+
 /*
- * One workgroup per band of up to MS_MPB meshes along x.  The sums of back.c are two
- * sequential double chains per mesh (pix and pix*pix in raster order); they cannot be
- * reordered (the squares carry up to 48 significant bits, so their double sum rounds),
- * but nothing else has to sit on the chain: wavefronts 1..3 stream the band's rows
- * through a double-buffered LDS ring and store, per pixel, t = (included ? pix : +0)
- * and t2 = (included ? pix*pix : -0) as doubles; in wavefront 0, lane m adds the t of
- * mesh m and lane MS_MPB + m its t2 (counting the non-negative ones), one double add per
- * pixel and lane.  Adding +0 to the first sum and -0 to the second is an exact identity
- * (both start at +0 and stay >= +0 in round-to-nearest).
+ * The sums of back.c are sequential double sums of pix and of pix*pix in raster order.
+ * A chain of dependent adds costs 8 cycles an element and leaves the chip idle, so each
+ * mesh is cut into runs of consecutive pixels, one lane each, and every lane finds what
+ * its run adds to the sequential sum, bit for bit:
+ *
+ *   - While a partial sum S stays in one binade [2^e, 2^(e+1)) it is k*u with u its ulp
+ *     and k an integer, and adding x gives u*RNE(k + x/u): the increment depends on x and
+ *     on k mod 2 only (the parity decides the ties).  So a lane adds its run with ordinary
+ *     FP64 adds to two stand-ins for S, one of either parity, taken from a prefix sum A
+ *     that is close to S: B0 (A with its last mantissa bit cleared) and B1 = B0 + u.  The
+ *     differences d0, d1 of the ends from the starts are exact, and the sequential sum
+ *     after the run is S + (last bit of S ? d1 : d0), exact as well.  d0 and d1 are equal,
+ *     or a tie came up in the run: then they differ by u and both ends have the same last
+ *     bit, so one more tie picks the right one: y1 = (d0 + d1) / 2 is halfway between the
+ *     two ends, of which the even one is taken; where the end has to be the odd one, y1
+ *     and y2 = u put it one ulp lower and back: S = (S + y1) + y2.  S + y2 is exact, and so
+ *     is y2 plus the next run's y1, a multiple of u/2 below 2^52 u: a run costs the walk
+ *     one dependent add.
+ *   - |A - S| <= 2 n 2^-53 sum|x| (the rounding of two recursive sums, Higham, Accuracy and
+ *     Stability of Numerical Algorithms, 2nd ed., eq. 4.4); the run's bounds are widened by
+ *     delta = 8 times n 2^-53 sum|x|, and a run whose bounds do not lie in one binade, or are
+ *     not finite, zero or subnormal, is flagged: its pixels are added one by one.  A sum of
+ *     positive terms crosses log2(runs) + 1 binades after its first run, so few runs are.
+ *   - Where sum|pix| <= 2^53 times the unit of the smallest pixel's last bit, every partial
+ *     sum is a multiple of that unit that a double holds: the order does not matter and the
+ *     sum of pix is taken in any (true of almost all frames).
+ *
+ * The mesh sits in LDS between the two passes (run t at t*KS, KS a multiple of four floats
+ * and KS/4 odd: a lane's float4 reads are conflict-free), so the frame is read once; the
+ * runs' places past the last pixel hold NaN, which no pass takes.  G: a
+ * mesh that does not fit stays in global memory.  One workgroup of NW wavefronts per mesh;
+ * wavefront 0 walks the runs' increments.
+ *
+ * Bound: VALU instructions (about 20 a pixel and pass), then the walk (3 us a pass at two
+ * wavefronts).  A 64 x 64 mesh takes 12 us; measured against the sequential chains fed from
+ * an LDS ring (8,192 dependent adds a mesh): 1024^2 105 -> 15 us, 4096^2 119 -> 63 us (256
+ * CUs, 16 meshes each, seven at a time by LDS), 2011 x 1533 (rows not aligned) 343 -> 21 us,
+ * 8192 x 4096 with weights and 128 x 128 meshes 806 -> 140 us.
  */
-#define MS_MPB 16
-#define MS_THREADS 256
-/* loads of a loader thread in flight together */
-#define MS_U 4
-/* dynamic LDS of a workgroup, the ring: more rows per batch (a larger ring) measured no
-   faster, and on a CU it leaves less room for other frames' kernels */
-#define MS_LDS_BYTES (128 * 1024)
-
-/* meshes whose rows do not fit the LDS ring: one lane per mesh reading global memory */
-__global__ void __launch_bounds__(64) k_meshstat_direct(const float *__restrict__ img,
-                                                        const float *__restrict__ wmap, int W,
-                                                        int H, int bs, int nbx, int nmesh,
-                                                        MeshStat *ms)
+__host__ __device__ inline int ms_run(int npx, int runs)   /* pixels of a run: K */
 {
-    const int mi = blockIdx.x * 64 + threadIdx.x;
-    if (mi >= nmesh) return;
-    const int x0 = (mi % nbx) * bs, y0 = (mi / nbx) * bs;
-    const int bw = min(bs, W - x0), bh = min(bs, H - y0);
-    MeshAcc acc;
-    MeshStat o;
-    float lcut = 0.0f, hcut = 0.0f;
-    bool bad = false;
-    for (int pass = 0; pass < 2 && !(pass == 1 && bad); pass++) {
-        for (int y = 0; y < bh; y++) {
-            const size_t ro = (size_t)(y0 + y) * W + x0;
-            for (int x = 0; x < bw; x++) {
-                const double pix = (wmap && !(wmap[ro + x] > 0.0f)) ? (float)-SXG_BIG : img[ro + x];
-                if (pass == 0 ? pix > -SXG_BIG : (pix <= hcut && pix >= lcut)) {
-                    acc.mean += pix;
-                    acc.sigma += pix * pix;
-                    acc.npix++;
-                }
-            }
-        }
-        if (pass == 0) {
-            meshstat_pass1_end(acc, bw, bh, o, lcut, hcut, bad);
-            acc = MeshAcc();
-        } else {
-            meshstat_pass2_end(acc, o);
-        }
-    }
-    ms[mi] = o;
+    return ((npx + runs - 1) / runs + 3) & ~3;
 }
-/* LDS segment of one mesh row in doubles: column c of the mesh sits at
-   (c & 3) * ms_q(bs) + (c >> 2), so the loader lanes, which take four adjacent columns
-   each, store to consecutive doubles; the segment length is odd, so the 16 chain lanes
-   of an array, which read the same column of 16 meshes, start on distinct bank pairs */
-__host__ __device__ inline int ms_q(int bs) { return (bs + 3) >> 2; }
-__host__ __device__ inline int ms_seg(int bs) { return (4 * ms_q(bs)) | 1; }
+__host__ __device__ inline int ms_stride(int K) { return (K >> 2) & 1 ? K : K + 4; }
 
-__global__ void __launch_bounds__(MS_THREADS) k_meshstat(const float *__restrict__ img,
-                                                         const float *__restrict__ wmap, int W,
-                                                         int H, int bs, int nbx, int mpb, int R,
-                                                         MeshStat *ms)
+/* lo and hi (lo <= hi) are normal numbers of one sign and binade */
+__device__ inline bool ms_binade(double lo, double hi)
 {
-    extern __shared__ __align__(16) double ring[];
-    __shared__ float s_lcut[MS_MPB], s_hcut[MS_MPB];
-    __shared__ int s_cnt[MS_MPB];
-    const int tid = threadIdx.x, wid = tid >> 6, lane = tid & 63;
-    const int mx0 = blockIdx.x * mpb, my = blockIdx.y;
-    const int nm = min(mpb, nbx - mx0);
-    const int x0 = mx0 * bs, y0 = my * bs;
-    const int bandw = min(W, x0 + nm * bs) - x0;
-    const int bh = min(bs, H - y0);
-    const int seg = ms_seg(bs), q = ms_q(bs);
-    const int bufsz = R * mpb * seg;            /* doubles per buffer and array */
-    const int nbatch = (bh + R - 1) / R;
-    /* mesh of a band column: a shift when the mesh size is a power of two */
-    const int bsh = (bs & (bs - 1)) == 0 ? __builtin_ctz(bs) : -1;
-    /* the chain lane's mesh and array (0: t, 1: t2) */
-    const int m = lane < mpb ? lane : lane - mpb;
-    const int arr = lane < mpb ? 0 : 1;
-    const bool chain = wid == 0 && lane < 2 * mpb && m < nm;
-    const int bw = min(bs, W - (x0 + m * bs));
-    MeshStat o;
-    float lcut = 0.0f, hcut = 0.0f;
-    bool bad = false;
-    const bool vec4 = ((bs | W) & 3) == 0;
-    /* wavefronts 1..3: rows [b*R, b*R + nr) of the band into buffer half h, and the
-       number of included pixels of each mesh */
-    auto load = [&](int pass, int b, int h) {
-        double *bt = ring + (size_t)(2 * h) * bufsz, *bt2 = bt + bufsz;
-        const int r0 = b * R, nr = min(R, bh - r0);
-        const int lt = tid - 64, LT = MS_THREADS - 64;
-        auto incl = [&](double pix, int mm) {
-            return pass == 0 ? (pix > -SXG_BIG)
-                             : ((pix <= (double)s_hcut[mm]) & (pix >= (double)s_lcut[mm]));
-        };
-        if (vec4) {
-            /* all the batch's loads of a thread in flight before any store */
-            const int q4 = bandw >> 2, tot = nr * q4;
-            const int qsh = (q4 & (q4 - 1)) == 0 ? __builtin_ctz(q4) : -1;
-            for (int e0 = lt; e0 < tot; e0 += MS_U * LT) {
-                float4 v[MS_U];
+    const int a = __double2hiint(lo) >> 20, b = __double2hiint(hi) >> 20;
+    return a == b && (a & 0x7ff) != 0 && (a & 0x7ff) != 0x7ff;
+}
+
+template <int NW, bool G>
+__global__ void __launch_bounds__(64 * NW) k_meshstat(const float *__restrict__ img,
+                                                      const float *__restrict__ wmap, int W,
+                                                      int H, int bs, int nbx, MeshStat *ms)
+{
+    constexpr int R = 64 * NW;
+    extern __shared__ __align__(16) float px[];
+    __shared__ double s_y1[R], s_y2[R + 1];  /* y1 of run t, y2 of run t - 1 */
+    __shared__ unsigned long long s_flag[NW];
+    __shared__ double s_s1[NW], s_s2[NW];
+    __shared__ float s_fa[NW];
+    __shared__ unsigned s_min[NW];
+    __shared__ int s_cnt[NW];
+    __shared__ double s_res;
+    __shared__ float s_cut[2];
+    __shared__ int s_bad;
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int m = blockIdx.x, x0 = (m % nbx) * bs, y0 = (m / nbx) * bs;
+    const int bw = min(bs, W - x0), bh = min(bs, H - y0), npx = bw * bh;
+    const int K = ms_run(npx, R), KS = ms_stride(K);
+    const int len = min(max(npx - tid * K, 0), K);      /* pixels of this lane's run */
+    const float big = (float)-SXG_BIG;
+    const float *const base = img + (size_t)y0 * W + x0;
+    const float *const wbase = wmap ? wmap + (size_t)y0 * W + x0 : nullptr;
+    /* pixels of non-positive weight are left out: -BIG */
+    auto weigh = [&](float v, size_t o) { return wmap && !(wbase[o] > 0.0f) ? big : v; };
+    if constexpr (!G) {
+        /* pixel i of the mesh at i + (i / K) * (KS - K) */
+        const unsigned mk = 0xffffffffu / (unsigned)K + 1u;   /* i / K, i*K < 2^32 */
+        const int pad = KS - K;
+        if (((bw | W | bs) & 3) == 0) {
+            constexpr int U = 8;
+            const int q4 = bw >> 2, tot = q4 * bh;
+            const unsigned mq = 0xffffffffu / (unsigned)q4 + 1u;
+            for (int e0 = tid; e0 < tot; e0 += U * R) {
+                float4 v[U];
+                size_t of[U];
+                int at[U];
 #pragma unroll
-                for (int u = 0; u < MS_U; u++) {
-                    const int e = e0 + u * LT;
-                    if (e < tot) {
-                        const int r = qsh >= 0 ? e >> qsh : e / q4, c = 4 * (e - r * q4);
-                        const size_t ofs = (size_t)(y0 + r0 + r) * W + x0 + c;
-                        v[u] = *reinterpret_cast<const float4 *>(img + ofs);
-                        if (wmap) {
-                            /* pixels of non-positive weight are left out: -BIG */
-                            const float4 wv = *reinterpret_cast<const float4 *>(wmap + ofs);
-                            const float nb = (float)-SXG_BIG;
-                            if (!(wv.x > 0.0f)) v[u].x = nb;
-                            if (!(wv.y > 0.0f)) v[u].y = nb;
-                            if (!(wv.z > 0.0f)) v[u].z = nb;
-                            if (!(wv.w > 0.0f)) v[u].w = nb;
-                        }
+                for (int u = 0; u < U; u++) {
+                    const int e = min(e0 + u * R, tot - 1);
+                    const int y = q4 == 1 ? e : (int)__umulhi((unsigned)e, mq);
+                    const size_t o = (size_t)y * W + 4 * (e - y * q4);
+                    v[u] = *reinterpret_cast<const float4 *>(base + o);
+                    of[u] = o;
+                    at[u] = 4 * e + (int)__umulhi(4u * e, mk) * pad;
+                }
+                if (wmap) {
+                    float4 wv[U];
+#pragma unroll
+                    for (int u = 0; u < U; u++)
+                        wv[u] = *reinterpret_cast<const float4 *>(wbase + of[u]);
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        if (!(wv[u].x > 0.0f)) v[u].x = big;
+                        if (!(wv[u].y > 0.0f)) v[u].y = big;
+                        if (!(wv[u].z > 0.0f)) v[u].z = big;
+                        if (!(wv[u].w > 0.0f)) v[u].w = big;
                     }
                 }
 #pragma unroll
-                for (int u = 0; u < MS_U; u++) {
-                    const int e = e0 + u * LT;
-                    if (e < tot) {
-                        const int r = qsh >= 0 ? e >> qsh : e / q4, c = 4 * (e - r * q4);
-                        const int mm = bsh >= 0 ? c >> bsh : c / bs, off = c - mm * bs;
-                        const double p0 = v[u].x, p1 = v[u].y, p2 = v[u].z, p3 = v[u].w;
-                        const bool i0 = incl(p0, mm), i1 = incl(p1, mm), i2 = incl(p2, mm),
-                                   i3 = incl(p3, mm);
-                        /* off is a multiple of 4: its four columns at off/4 + j*q */
-                        const int idx = (r * mpb + mm) * seg + (off >> 2);
-                        double *d = bt + idx, *d2 = bt2 + idx;
-                        d[0] = i0 ? p0 : 0.0;
-                        d[q] = i1 ? p1 : 0.0;
-                        d[2 * q] = i2 ? p2 : 0.0;
-                        d[3 * q] = i3 ? p3 : 0.0;
-                        d2[0] = i0 ? p0 * p0 : -0.0;
-                        d2[q] = i1 ? p1 * p1 : -0.0;
-                        d2[2 * q] = i2 ? p2 * p2 : -0.0;
-                        d2[3 * q] = i3 ? p3 * p3 : -0.0;
-                        const int k = (int)i0 + (int)i1 + (int)i2 + (int)i3;
-                        if (k) atomicAdd(&s_cnt[mm], k);
-                    }
+                for (int u = 0; u < U; u++)
+                    if (e0 + u * R < tot) *reinterpret_cast<float4 *>(px + at[u]) = v[u];
+            }
+        } else {
+            constexpr int U = 16;
+            const unsigned mw = 0xffffffffu / (unsigned)bw + 1u;
+            for (int e0 = tid; e0 < npx; e0 += U * R) {
+                float v[U];
+                size_t of[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int e = min(e0 + u * R, npx - 1);
+                    const int y = bw == 1 ? e : (int)__umulhi((unsigned)e, mw);
+                    of[u] = (size_t)y * W + (e - y * bw);
+                    v[u] = base[of[u]];
+                }
+                if (wmap) {
+                    float wv[U];
+#pragma unroll
+                    for (int u = 0; u < U; u++) wv[u] = wbase[of[u]];
+#pragma unroll
+                    for (int u = 0; u < U; u++)
+                        if (!(wv[u] > 0.0f)) v[u] = big;
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int e = e0 + u * R;
+                    if (e < npx) px[e + (int)__umulhi((unsigned)e, mk) * pad] = v[u];
+                }
+            }
+        }
+        for (int i = npx + tid; i < R * K; i += R)
+            px[i + (int)__umulhi((unsigned)i, mk) * pad] = NAN;
+        __syncthreads();
+    }
+    /* pixel j of run t (NaN past the mesh's last pixel) */
+    auto pix1 = [&](int t, int j) -> float {
+        const int i = t * K + j;
+        if (i >= npx) return NAN;
+        if constexpr (G) {
+            const size_t o = (size_t)(i / bw) * W + i % bw;
+            return weigh(base[o], o);
+        } else {
+            return px[t * KS + j];
+        }
+    };
+    /* the pixels that take part: those above -BIG, then those between the cuts */
+    float lcut = ord2f(f2ord(big) + 1), hcut = INFINITY;
+    auto sel = [&](float v, bool &in) {
+        in = v >= lcut && v <= hcut;
+        return in ? v : 0.0f;
+    };
+    /* f(the pixel or 0, takes part) over this lane's run */
+    auto each = [&](auto f) {
+        if constexpr (G) {
+            int y = (tid * K) / bw, x = tid * K - y * bw;
+            for (int j = 0; j < len; j++) {
+                const size_t ofs = (size_t)y * W + x;
+                bool in;
+                const float q = sel(weigh(base[ofs], ofs), in);
+                f(q, in);
+                if (++x == bw) {
+                    x = 0;
+                    y++;
                 }
             }
         } else {
-            const int tot = nr * bandw;
-            for (int e0 = lt; e0 < tot; e0 += MS_U * LT) {
-                float v[MS_U];
-#pragma unroll
-                for (int u = 0; u < MS_U; u++) {
-                    const int e = e0 + u * LT;
-                    if (e < tot) {
-                        const int r = e / bandw, c = e - r * bandw;
-                        const size_t ofs = (size_t)(y0 + r0 + r) * W + x0 + c;
-                        v[u] = (wmap && !(wmap[ofs] > 0.0f)) ? (float)-SXG_BIG : img[ofs];
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < MS_U; u++) {
-                    const int e = e0 + u * LT;
-                    if (e < tot) {
-                        const int r = e / bandw, c = e - r * bandw;
-                        const int mm = bsh >= 0 ? c >> bsh : c / bs, off = c - mm * bs;
-                        const double pix = v[u];
-                        const bool in = incl(pix, mm);
-                        const int idx = (r * mpb + mm) * seg + (off & 3) * q + (off >> 2);
-                        bt[idx] = in ? pix : 0.0;
-                        bt2[idx] = in ? pix * pix : -0.0;
-                        if (in) atomicAdd(&s_cnt[mm], 1);
-                    }
-                }
+            const float4 *rp = reinterpret_cast<const float4 *>(px + tid * KS);
+#pragma unroll 4
+            for (int j = 0; j < K; j += 4) {
+                const float4 v = rp[j >> 2];
+                bool i0, i1, i2, i3;
+                const float q0 = sel(v.x, i0), q1 = sel(v.y, i1), q2 = sel(v.z, i2),
+                            q3 = sel(v.w, i3);
+                f(q0, i0);
+                f(q1, i1);
+                f(q2, i2);
+                f(q3, i3);
             }
         }
     };
+    MeshStat o;
     for (int pass = 0; pass < 2; pass++) {
-        double acc = 0.0;
-        if (tid < MS_MPB) s_cnt[tid] = 0;
+        double s1 = 0.0, s2 = 0.0;
+        float fa = 0.0f;
+        /* bits of the smallest non-zero |pixel|, twice, less one */
+        unsigned um = 0xffffffffu;
+        int cnt = 0;
+        each([&](float q, bool in) {
+            const double p = q;
+            s1 += p;
+            s2 += p * p;
+            fa += fabsf(q);
+            um = min(um, 2u * (unsigned)__float_as_int(q) - 1u);
+            cnt += in;
+        });
+        const int mycnt = cnt;
+        double x2 = s2;                /* inclusive prefix in the wavefront */
+        for (int d = 1; d < 64; d <<= 1) {
+            const double t = __shfl_up(x2, d);
+            if (lane >= d) x2 += t;
+            s1 += __shfl_xor(s1, d);
+            fa += __shfl_xor(fa, d);
+        }
+        cnt = sxw_sum(cnt);
+        um = (unsigned)sxw_min((int)(um ^ 0x80000000u)) ^ 0x80000000u;
+        if (lane == 63) {
+            s_s1[wid] = s1;
+            s_s2[wid] = x2;
+            s_fa[wid] = fa;
+            s_min[wid] = um;
+            s_cnt[wid] = cnt;
+        }
         __syncthreads();
-        if (wid != 0) load(pass, 0, 0);
-        __syncthreads();
-        for (int b = 0; b < nbatch; b++) {
-            if (wid != 0) {
-                if (b + 1 < nbatch) load(pass, b + 1, (b + 1) & 1);
-            } else if (chain) {
-                /* the lane's chain: one double add per pixel in column order (column c
-                   of a row at (c & 3) * q + (c >> 2)) */
-                const double *src = ring + (size_t)(2 * (b & 1) + arr) * bufsz + m * seg;
-                const int nr = min(R, bh - b * R), rstride = mpb * seg;
-                if ((bw & 31) == 0 && ((nr * (bw >> 5)) & 1) == 0) {
-                    /* an even number of chunks of 32 columns, in two register buffers
-                       used in turn: the reads of the next chunk are in flight while this
-                       one is added.  Every load is unconditional (the pointer wraps to
-                       the batch's first chunk after its last), so no control-flow merge
-                       makes the compiler wait for both buffers at once; no copy between
-                       the buffers either, which would wait for the newer reads */
-                    const int cpr = bw >> 5, K = nr * cpr;
-                    const double *cp = src;
-                    int cc = 0, rr = 0;
-                    auto ld = [&](double (&d)[32]) {
+        double t1 = 0.0, t2 = 0.0, b2 = 0.0;
+        fa = 0.0f;
+        cnt = 0;
 #pragma unroll
-                        for (int u = 0; u < 32; u++) d[u] = cp[(u & 3) * q + (u >> 2)];
-                        const bool eor = ++cc == cpr;
-                        cc = eor ? 0 : cc;
-                        rr += eor ? 1 : 0;
-                        const bool eob = rr == nr;
-                        rr = eob ? 0 : rr;
-                        cp = eob ? src : (eor ? cp + (rstride - (cpr - 1) * 8) : cp + 8);
-                    };
-                    double A[32], B[32];
-                    ld(A);
-                    for (int k = 0; k < K; k += 2) {
-                        ld(B);
+        for (int w = 0; w < NW; w++) {
+            if (w == wid) b2 = t2;
+            t1 += s_s1[w];
+            t2 += s_s2[w];
+            fa += s_fa[w];
+            um = min(um, s_min[w]);
+            cnt += s_cnt[w];
+        }
+        /* wavefront 0: the sequential sum from the runs' increments, sixteen runs at a time
+           (the rows of the wavefront do the same); term: the summand of a pixel */
+        auto walk = [&](auto term) {
+            const int l16 = lane & 15;
+            double S = 0.0;
+#pragma unroll 1
+            for (int w = 0; w < NW; w++) {
+                const unsigned long long f = s_flag[w];
+                const unsigned flo = (unsigned)__builtin_amdgcn_readfirstlane((int)f);
+                const unsigned fhi = (unsigned)__builtin_amdgcn_readfirstlane((int)(f >> 32));
+                double z[4];
 #pragma unroll
-                        for (int u = 0; u < 32; u++) acc += A[u];
-                        ld(A);
+                for (int g = 0; g < 4; g++)
+                    z[g] = s_y1[w * 64 + g * 16 + l16] + s_y2[w * 64 + g * 16 + l16];
 #pragma unroll
-                        for (int u = 0; u < 32; u++) acc += B[u];
+                for (int g = 0; g < 4; g++) {
+                    const int t0 = w * 64 + g * 16;
+                    unsigned fl = ((g < 2 ? flo : fhi) >> (16 * (g & 1))) & 0xffffu;
+                    int done = 0;      /* runs of the sixteen in S */
+#pragma unroll 1
+                    while (fl) {
+                        /* up to the next flagged run (its y1, y2 are 0), then its pixels
+                           one by one */
+                        const int r = __builtin_ctz(fl);
+                        fl &= fl - 1;
+                        S = sxw_row_fold(S, l16 >= done && l16 <= r ? z[g] : 0.0);
+                        for (int j = 0; j < K; j += 16) {
+                            bool in;
+                            const float v = j + l16 < K ? pix1(t0 + r, j + l16) : NAN;
+                            S = sxw_row_fold(S, term((double)sel(v, in)));
+                        }
+                        done = r + 1;
                     }
-                } else {
-                    for (int r = 0; r < nr; r++) {
-                        const double *row = src + r * rstride;
-                        for (int x = 0; x < bw; x++) acc += row[(x & 3) * q + (x >> 2)];
-                    }
+                    S = sxw_row_fold(S, l16 >= done ? z[g] : 0.0);
                 }
             }
+            return S + s_y2[R];
+        };
+        /* every lane: its run's increments and flag.  A: the prefix before the run, [A -
+           neg, A + pos]: what the run can reach, abs: sum|x| of the mesh */
+        auto increments = [&](double A, double neg, double pos, double abs, auto term) {
+            const double delta = abs * (double)npx * 0x1p-50;
+            const bool flag = mycnt > 0 && !ms_binade(A - neg - delta, A + pos + delta);
+            double y1 = 0.0, y2 = 0.0;
+            if (mycnt > 0 && !flag) {
+                const double B0 = __hiloint2double(__double2hiint(A), __double2loint(A) & ~1);
+                const double B1 = __hiloint2double(__double2hiint(A), __double2loint(A) | 1);
+                double a0 = B0, a1 = B1;
+                each([&](float q, bool) {
+                    const double x = term((double)q);
+                    a0 += x;
+                    a1 += x;
+                });
+                const double d0 = a0 - B0, d1 = a1 - B1;
+                const bool odd = d0 != d1 && (__double2loint(a0) & 1);
+                y2 = odd ? B1 - B0 : 0.0;
+                y1 = (d0 + d1) * 0.5 - y2;
+            }
+            s_y1[tid] = y1;
+            s_y2[tid + 1] = y2;
+            if (tid == 0) s_y2[0] = 0.0;
+            const unsigned long long b = __ballot(flag);
+            if (lane == 0) s_flag[wid] = b;
+        };
+        auto square = [](double p) { return p * p; };
+        auto same = [](double p) { return p; };
+        increments(b2 + x2 - s2, 0.0, s2, t2, square);
+        __syncthreads();
+        /* the unit of the last mantissa bit of the smallest pixel */
+        const int ue = max((int)((um + 1u) >> 24), 1) - 150;
+        const bool any = um == 0xffffffffu || (double)fa * (1.001 + K * 0x1p-22) <= ldexp(1.0, 53 + ue);
+        MeshAcc a;
+        a.npix = cnt;
+        a.mean = t1;
+        if (wid == 0) a.sigma = walk(square);
+        if (!any) {
+            /* the sum of pix along its order too: prefix, and the parts of either sign */
             __syncthreads();
+            double ps = 0.0, ng = 0.0;
+            each([&](float q, bool) {
+                ps += q > 0.0f ? (double)q : 0.0;
+                ng += q < 0.0f ? -(double)q : 0.0;
+            });
+            double xs = ps - ng, ab = ps + ng;
+            const double own = xs;
+            for (int d = 1; d < 64; d <<= 1) {
+                const double t = __shfl_up(xs, d);
+                if (lane >= d) xs += t;
+                ab += __shfl_xor(ab, d);
+            }
+            if (lane == 63) {
+                s_s1[wid] = xs;
+                s_s2[wid] = ab;
+            }
+            __syncthreads();
+            double before = 0.0, tab = 0.0;
+#pragma unroll
+            for (int w = 0; w < NW; w++) {
+                if (w < wid) before += s_s1[w];
+                tab += s_s2[w];
+            }
+            increments(before + xs - own, ng, ps, tab, same);
+            __syncthreads();
+            if (wid == 0) a.mean = walk(same);
         }
-        /* mesh m: the pix sum from lane m, the pix^2 sum from lane mpb+m */
-        const double sq = __shfl(acc, lane + mpb);
-        if (wid == 0 && lane < nm) {
-            MeshAcc a;
-            a.mean = acc;
-            a.sigma = sq;
-            a.npix = s_cnt[lane];
+        if (tid == 0) {
             if (pass == 0) {
+                bool bad;
                 meshstat_pass1_end(a, bw, bh, o, lcut, hcut, bad);
-                s_lcut[lane] = lcut;
-                s_hcut[lane] = hcut;
-            } else if (!bad) {
+                s_cut[0] = lcut;
+                s_cut[1] = hcut;
+                s_bad = bad;
+            } else {
                 meshstat_pass2_end(a, o);
             }
         }
         __syncthreads();
+        if (pass == 0) {
+            if (s_bad) break;
+            lcut = s_cut[0];
+            hcut = s_cut[1];
+        }
     }
-    if (wid == 0 && lane < nm) ms[my * nbx + mx0 + lane] = o;
+    if (tid == 0) ms[m] = o;
 }
 
 /* --------------------------------------------------------------- backguess ---- */
@@ -1129,33 +1251,41 @@ bool sxg_back_run(const BackGeom &g, const BackBufs &b, const float *src, float 
     while (n2 < nmesh) n2 <<= 1;
     if (timed) sxg_kt_begin(SXG_KT_MESHSTAT);
     {
-        /* meshes per workgroup and rows per batch: two buffers of R rows of mpb padded
-           segments of t and t2 (doubles), each within 64 KB */
-        const size_t segbytes = (size_t)ms_seg(bs) * 2 * sizeof(double);
-        const int mpb = (int)std::min<size_t>(MS_MPB, (64 * 1024) / segbytes);
-        if (mpb >= 1) {
-            /* the LDS limit is an attribute of the function: raised once, to the most
-               any launch asks for */
-            static const bool attr = [] {
-                return hipFuncSetAttribute(reinterpret_cast<const void *>(&k_meshstat),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           MS_LDS_BYTES) == hipSuccess;
-            }();
-            if (!attr) {
-                sxg_set_error("back_estimate: cannot raise the LDS limit of k_meshstat");
-                return false;
-            }
-            const size_t rowbytes = mpb * segbytes;
-            const long rows = sxg_option(SXG_OPT_MESH_ROWS);
-            int R = (int)std::max<size_t>(1, std::min<size_t>(8, (64 * 1024) / rowbytes));
-            if (rows > 0 && rows < R) R = (int)rows;
-            const size_t lds = 2 * R * rowbytes;
-            hipLaunchKernelGGL(k_meshstat, dim3(sxg_div_up(nbx, mpb), nby), dim3(MS_THREADS), lds,
-                               st, src, wmap, W, H, bs, nbx, mpb, R, b.ms);
-        } else {
-            hipLaunchKernelGGL(k_meshstat_direct, dim3(sxg_div_up(nmesh, 64)), dim3(64), 0, st,
-                               src, wmap, W, H, bs, nbx, nmesh, b.ms);
+        /* wavefronts per mesh by its pixels: runs of 16 to 80 pixels.  Longer ones cost the
+           flagged runs' one-by-one adds, shorter ones the walk.  Measured at 4096^2: meshes
+           of 64 with 1, 2, 4 wavefronts 74, 63, 76 us, meshes of 128 with 2, 4, 8
+           wavefronts 92, 69, 93 us.  A mesh beyond the LDS stays in global memory */
+        const long px = (long)std::min(bs, W) * std::min(bs, H);
+        auto bytes = [&](int nw) {
+            return sizeof(float) * 64 * (size_t)nw * ms_stride(ms_run((int)px, 64 * nw));
+        };
+        auto launch = [&](auto kern, int nw, size_t lds) {
+            hipLaunchKernelGGL(kern, dim3(nmesh), dim3(64 * nw), lds, st, src, wmap, W, H, bs,
+                               nbx, b.ms);
+        };
+        /* the LDS limit is an attribute of the function: raised once, to the most any
+           launch asks for */
+        static const bool attr =
+            hipFuncSetAttribute(reinterpret_cast<const void *>(&k_meshstat<4, false>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                MS_LDS_BYTES) == hipSuccess &&
+            hipFuncSetAttribute(reinterpret_cast<const void *>(&k_meshstat<8, false>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                MS_LDS_BYTES) == hipSuccess;
+        if (!attr) {
+            sxg_set_error("back_estimate: cannot raise the LDS limit of k_meshstat");
+            return false;
         }
+        if (px <= MS_PX1)
+            launch(&k_meshstat<1, false>, 1, bytes(1));
+        else if (px <= MS_PX2)
+            launch(&k_meshstat<2, false>, 2, bytes(2));
+        else if (px <= MS_PX4)
+            launch(&k_meshstat<4, false>, 4, bytes(4));
+        else if (bytes(8) <= MS_LDS_BYTES)
+            launch(&k_meshstat<8, false>, 8, bytes(8));
+        else
+            launch(&k_meshstat<16, true>, 16, 0);
     }
     if (timed) sxg_kt_end(SXG_KT_MESHSTAT);
     if (timed) sxg_kt_begin(SXG_KT_MESHMODE);

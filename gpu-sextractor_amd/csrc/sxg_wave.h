@@ -84,6 +84,27 @@ template <class Op> __device__ inline float sxw_dpp_allf(float v, Op op)
     return op(op(a, b), op(c, d));
 }
 
+/*
+ * S + x_0 + x_1 + ... + x_15 in that order, x_j the value of lane j of the row of 16 lanes
+ * (S: the same in every lane of a row, and the result too; each row its own sum).  One
+ * v_fmac_f64 with a row broadcast per value: fma(x, 1, S) rounds once, as S + x does.  A
+ * dependent chain of them issues every 4.3 cycles, against 10 to 15 for adds fed from LDS
+ * reads (a read costs its wavefront 12 cycles) and 13 for readlanes (2.4 GHz, one
+ * wavefront).  Every lane must be active; s_nop: a VALU result needs two wait states before
+ * a DPP read.
+ */
+#define SXW_RF(n) "v_fmac_f64_dpp %0, %1, %2 row_newbcast:" #n " row_mask:0xf bank_mask:0xf\n"
+__device__ inline double sxw_row_fold(double S, double x)
+{
+    const double one = 1.0;
+    asm("s_nop 1\n" SXW_RF(0) SXW_RF(1) SXW_RF(2) SXW_RF(3) SXW_RF(4) SXW_RF(5) SXW_RF(6)
+        SXW_RF(7) SXW_RF(8) SXW_RF(9) SXW_RF(10) SXW_RF(11) SXW_RF(12) SXW_RF(13) SXW_RF(14)
+        SXW_RF(15)
+        : "+v"(S)
+        : "v"(x), "v"(one));
+    return S;
+}
+
 /* keep the five largest values seen by this lane, t[0] >= ... >= t[4] (-inf = empty) */
 struct SxwTop5 {
     float t[5];

@@ -438,10 +438,8 @@ int sxg_kernel_times(int id, double *total_ms, int *launches);
      SXG_OPT_DEB_ORDER_FULL the global-memory objects are launched largest first when there
                             are at most this many of them (default 4096); beyond, only the
                             level-parallel ones are ordered, the others follow in any order
-     SXG_OPT_MESH_ROWS      frame rows per batch of the mesh-statistics kernel's LDS ring
-                            (0, default: as many as fit in 64 KB per buffer, at most 8; else
-                            1..8): fewer rows hold less LDS while its chains run, which
-                            leaves room on each CU for other frames' kernels
+     SXG_OPT_MESH_ROWS      0..8, without effect (it sized an LDS ring of the mesh statistics
+                            that is no longer there); kept for callers that set it
      SXG_OPT_FUSED_FILTER   1 (default): the whole-frame runs (sxg_process_resident and the
                             batches) subtract the background spline, convolve and write the
                             detection parents in one kernel for frames of a width that is a
