@@ -107,7 +107,7 @@ SINGLE_KERNELS = {
     "conv": ("k_convolve<K>", lambda N, i: 8 * N),
     "analyse": ("k_analyse", lambda N, i: 12 * i["npix_raw"] + 176 * i["nobj"]),
     "deb_tree0": ("k_deb_tree_lds<256, 0>", lambda N, i: 12 * i["deb_class_pixels"][0]),
-    "deb_tree1": ("k_deb_tree_lds<1024, 1>", lambda N, i: 12 * i["deb_class_pixels"][1]),
+    "deb_tree1": ("k_deb_tree_lds<512, 1>", lambda N, i: 12 * i["deb_class_pixels"][1]),
     "deb_tree2": ("k_deb_tree_lds<1024, 2>", lambda N, i: 12 * i["deb_class_pixels"][2]),
 }
 

@@ -560,19 +560,16 @@ static void graph_release()
 /* capacity of a count seen in calibration: the margin, and a few units of slack */
 static FramePlan plan_from(const FramePlan &seen, int margin)
 {
-    static const int64_t slack[PL_N] = {4096, 64, 1024, 256, 16, 8, 4, 4, 2, 65536, 1024,
-                                        0, 0, 0, 128};
+    static const int64_t slack[PL_N] = {4096, 64, 1024, 256, 16, 8, 4, 4, 0, 0, 0, 128};
     FramePlan pl;
     for (int k = 0; k < PL_N; k++) {
         if (k >= PL_LDS0 && k <= PL_LDS2) continue;
         pl.cap[k] = seen.cap[k] + seen.cap[k] * margin / 100 + slack[k];
     }
-    /* the level-parallel objects are one grid row each (at most 65535) */
-    pl.cap[PL_BIG] = std::min<int64_t>(pl.cap[PL_BIG], 65535);
-    /* LDS of a class's workgroups: the class's budget (the kernel is launched with the
-       smaller of the two), except that class 2 asks for 76 KiB when its largest tree
-       seen, with the margin, fits there: two of its 1024-lane workgroups then share a
-       CU */
+    /* LDS of a class's workgroups: what the class's largest object may need (the kernel is
+       launched with the smaller of the two), except that class 2 asks for 76 KiB when its
+       largest object seen, with the margin, fits there: two of its 1024-lane workgroups
+       then share a CU */
     for (int c = 0; c < 3; c++) pl.cap[PL_LDS0 + c] = 0x7fffffff;
     const int64_t need2 = seen.cap[PL_LDS2] + seen.cap[PL_LDS2] * margin / 100;
     if (need2 <= 76 * 1024) pl.cap[PL_LDS2] = 76 * 1024;

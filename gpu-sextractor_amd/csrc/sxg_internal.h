@@ -156,9 +156,6 @@ enum PlanCap {
     PL_NPIX,      /* pixels of raw objects */
     PL_NTOT,      /* node capacity of the deblending trees */
     PL_C0, PL_C1, PL_C2, PL_C3,     /* raw objects per deblending size class */
-    PL_BIG,       /* class-3 objects built level-parallel */
-    PL_NPL,       /* pixel-levels of those */
-    PL_NREC,      /* node records of those */
     PL_LDS0, PL_LDS1, PL_LDS2,      /* LDS bytes of the tree workgroups of classes 0..2 */
     PL_NOBJ,      /* deblended objects */
     PL_N
@@ -170,15 +167,13 @@ struct FramePlan {
 struct PlanDev {
     int nfg, nraw, npix, nobj, nsurv;
     int ovf;          /* bit k: the count of PlanCap k exceeded its capacity; bit 30: the
-                         detection threshold is not positive; bit 29: deblending levels
-                         inconsistent */
+                         detection threshold is not positive */
     int pad[2];
     float dthresh, thresh, backmean, backsig;
     /* deblending work (sxg_frame_info's deb_pixels, deb_labels, deb_class_pixels) */
     long long deb_pixels, deb_labels, class_pixels[4];
 };
 #define SXG_PLAN_BADTHRESH 30
-#define SXG_PLAN_DEBLEVELS 29
 /* n, or the device count *nd when a planned run passes one */
 __device__ inline int sxg_dn(const int *nd, int n) { return nd ? *nd : n; }
 

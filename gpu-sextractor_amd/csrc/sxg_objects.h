@@ -7,8 +7,6 @@
 #include "sxg_internal.h"
 
 #define COMP_KEPT 1
-#define COMP_SIG 2
-#define COMP_OKA 4
 
 /* deblending-tree node as the object kernels see it, stored in the raw object's region
    of the table in the reference's order (level, then raster order of the first pixel):

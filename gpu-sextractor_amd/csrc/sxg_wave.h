@@ -105,6 +105,27 @@ __device__ inline double sxw_row_fold(double S, double x)
     return S;
 }
 
+/* the same for floats */
+#define SXW_RA(n) "v_add_f32_dpp %0, %1, %0 row_newbcast:" #n " row_mask:0xf bank_mask:0xf\n"
+__device__ inline float sxw_row_fold(float S, float x)
+{
+    asm("s_nop 1\n" SXW_RA(0) SXW_RA(1) SXW_RA(2) SXW_RA(3) SXW_RA(4) SXW_RA(5) SXW_RA(6)
+        SXW_RA(7) SXW_RA(8) SXW_RA(9) SXW_RA(10) SXW_RA(11) SXW_RA(12) SXW_RA(13) SXW_RA(14)
+        SXW_RA(15)
+        : "+v"(S)
+        : "v"(x));
+    return S;
+}
+
+/* S + the values of all 64 lanes in lane order, the same in every lane */
+__device__ inline float sxw_fold64(float S, float x)
+{
+    S = sxw_rl(sxw_row_fold(S, x), 0);
+    S = sxw_rl(sxw_row_fold(S, x), 16);
+    S = sxw_rl(sxw_row_fold(S, x), 32);
+    return sxw_rl(sxw_row_fold(S, x), 48);
+}
+
 /* keep the five largest values seen by this lane, t[0] >= ... >= t[4] (-inf = empty) */
 struct SxwTop5 {
     float t[5];

@@ -259,8 +259,8 @@ typedef struct {
     /* photometry work of the last endobject_gpu call: the aperture pixels summed (inside
        the APER outer radius, inside both AUTO ellipses) */
     int64_t phot_pixels;
-    /* pixels of the multi-peak raw objects in each deblending size class (0: 256-lane LDS
-       trees, 1 and 2: 1024-lane LDS trees, 3: global-memory trees) */
+    /* pixels of the multi-peak raw objects in each deblending size class (0, 1, 2: trees in
+       LDS with 256, 512 and 1024 lanes, 3: global-memory trees) */
     int64_t deb_class_pixels[4];
 } sxg_frame_info;
 int sxg_get_frame_info(sxg_frame_info *info);
@@ -409,8 +409,8 @@ enum sxg_kernel_id {
     SXG_KT_DEB_LEVELS, SXG_KT_DEB_OBJECTS, SXG_KT_ANALYSE, SXG_KT_CLEAN, SXG_KT_SEG,
     SXG_KT_DEB_LMAX, SXG_KT_OBJ_SORT, SXG_KT_PHOT,
     /* the deblending tree kernels one by one, each timed on the stream it runs on: size
-       classes 0, 1, 2 (k_deb_tree_lds), the one-workgroup global-memory trees
-       (k_deb_tree_glb) and the level-parallel chain (k_deb_glb_prep/levels/tree) */
+       classes 0, 1, 2 (k_deb_tree_lds) and the global-memory trees (k_deb_tree_glb);
+       SXG_KT_DEB_LVPAR times nothing any more */
     SXG_KT_DEB_TREE0, SXG_KT_DEB_TREE1, SXG_KT_DEB_TREE2, SXG_KT_DEB_TREE_GLB, SXG_KT_DEB_LVPAR,
     SXG_NKT
 };
@@ -421,23 +421,17 @@ int sxg_kernel_times(int id, double *total_ms, int *launches);
    choose which kernel variant handles which work.
      SXG_OPT_DEB_LDS_TINY   raw objects (with two or more local maxima) up to this many
                             pixels are deblended by 256-lane workgroups in LDS (default 512)
-     SXG_OPT_DEB_LDS_SMALL  up to this many by 1024-lane workgroups in LDS (default 1024)
+     SXG_OPT_DEB_LDS_SMALL  up to this many by 512-lane workgroups in LDS (default 1024)
      SXG_OPT_DEB_LDS_LARGE  up to this many by 1024-lane workgroups in LDS (default 6144,
                             at most 6400); larger ones use global scratch memory
-     SXG_OPT_DEB_TABLE      deblending-tree nodes an LDS workgroup can hold (0: 192, 512
-                            and 1024 for the three classes; at most 2048, and what the
-                            class's pixels leave of the LDS); a raw object whose tree may
-                            need more is built in global memory
+     SXG_OPT_DEB_TABLE      0..2048, without effect (it sized a node table in LDS that is no
+                            longer there); kept for callers that set it
      SXG_OPT_SIDE_STREAMS   1 (default): the deblending size classes of a frame run side by
                             side on streams of their own; 0: all on the context's stream
-     SXG_OPT_DEB_GLB_LEVELS the raw objects built in global memory with at least this many
-                            pixels (default 12288; at most 2^30) get the components of all
-                            their levels from one workgroup per level, in parallel; the
-                            others, and all of them at 0, one growing union-find per tree,
-                            level after level
+     SXG_OPT_DEB_GLB_LEVELS 0..2^30, without effect (it chose between two builds of the largest
+                            trees; there is one now); kept for callers that set it
      SXG_OPT_DEB_ORDER_FULL the global-memory objects are launched largest first when there
-                            are at most this many of them (default 4096); beyond, only the
-                            level-parallel ones are ordered, the others follow in any order
+                            are at most this many of them (default 4096), else in any order
      SXG_OPT_MESH_ROWS      0..8, without effect (it sized an LDS ring of the mesh statistics
                             that is no longer there); kept for callers that set it
      SXG_OPT_FUSED_FILTER   1 (default): the whole-frame runs (sxg_process_resident and the
