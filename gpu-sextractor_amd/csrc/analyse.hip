@@ -10,13 +10,20 @@
  * the reference's EXT_MINAREA = 5, cudatypes.h:62), the 8 isophotal areas and the FWHM
  * log fit; the SATUR flag of endobject (:2873-2874).
  *
- * Layout: one 64-lane wavefront per object over its contiguous, raster-ordered range of
- * the object pixel list (opix/objoff, built after deblending).  Lanes compute the
- * per-pixel terms of a chunk of 64 pixels in parallel; extrema, counts and the
- * first-maximum position are wavefront reductions; the floating-point sums are folded in
- * raster order by transposed folds (sxg_wave.h: lane s adds the terms of sum s), so each
- * sum is the reference's sequential sum bit for bit.
+ * Layout: one object per row of 16 lanes, per wavefront or per workgroup by its size
+ * (SxwTeam), over its contiguous, raster-ordered range of the object pixel list
+ * (opix/objoff, built after deblending).  Lanes compute the per-pixel terms; extrema, counts
+ * and the first-maximum position are reductions; the floating-point sums are folded in raster
+ * order (SxwSums), so each sum is the reference's sequential sum bit for bit.
+ *
+ * Bound: instruction issue (the moments, powers, roots and quotients of an object are some
+ * thousand instructions however few its pixels: four small objects share them in a
+ * wavefront), then the sequential sums of the largest object.  A wavefront per object
+ * whatever its size before: crowded 4096^2 109 -> 70 us, 8192 x 4096 67 -> 33, 2048^2 with
+ * saturated stars 78 -> 36 (its largest objects), 1024^2 17 -> 17.
  */
+#include <algorithm>
+
 #include "sxg_internal.h"
 #include "sxg_objects.h"
 #include "sxg_wave.h"
@@ -38,20 +45,31 @@ struct AnaArgs {
     const PlanDev *pd;      /* planned run: nobj, backsig, thresh and dthresh on the device */
 };
 
-/* objects of at least ANA_BIG pixels are analysed first: their sequential sums are the
-   longest, so they start at once and the small objects fill the machine around them */
-#define ANA_BIG 256
+/* objects of at least ANA_BIG pixels take a workgroup each, of at least ANA_MID a wavefront,
+   smaller ones a row of 16 lanes.  Measured (crowded 4096^2, dense 2048^2, 1024^2, in us): 256
+   and 32: 72, 124, 17; 512 and 32: 70, 111, 17; 512 and 64: 68, 102, 20 (a row takes 16
+   pixels a step: the latency of a small frame); 1024 and 64: 68, 106, 20 */
+#ifndef ANA_BIG
+#define ANA_BIG 512
+#define ANA_MID 32
+#endif
 
+/* the objects by size: order[0, nbig) the big ones, order[nbig + nmid, nobj) the small ones,
+   order[cap, cap + nmid) those between; cnt: their numbers */
 __global__ void __launch_bounds__(256) k_obj_order(const int *objoff, int nobj, int *cnt,
                                                    int *order, const PlanDev *pd)
 {
     const int obj = blockIdx.x * 256 + threadIdx.x;
+    const int cap = nobj;
     if (pd) nobj = pd->nobj;
     if (obj >= nobj) return;
-    if (objoff[obj + 1] - objoff[obj] >= ANA_BIG)
+    const int n = objoff[obj + 1] - objoff[obj];
+    if (n >= ANA_BIG)
         order[atomicAdd(&cnt[0], 1)] = obj;
+    else if (n >= ANA_MID)
+        order[cap + atomicAdd(&cnt[1], 1)] = obj;
     else
-        order[nobj - 1 - atomicAdd(&cnt[1], 1)] = obj;
+        order[nobj - 1 - atomicAdd(&cnt[2], 1)] = obj;
 }
 
 /* back.c:685-732 */
@@ -78,20 +96,16 @@ __device__ inline float back_at(const float *b, int x, int y, int nx, int ny, in
     return (float)((1 - dy) * (cdx * b0 + dx * b1) + dy * (dx * b2 + cdx * b3));
 }
 
-__global__ void __launch_bounds__(256) k_analyse(AnaArgs A)
+/* one object, by a row of 16 lanes, a wavefront or the workgroup; rows: the LDS of its sums */
+template <SxwSize Z>
+__device__ __forceinline__ void ana_object(const AnaArgs &A, const int obj, double *rows)
 {
-    __shared__ double s_rows[4][11 * SXW_ROW];
-    __shared__ float s_frows[4][SXW_ROW];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const int slot = blockIdx.x * 4 + wid;
-    if (slot >= (A.pd ? A.pd->nobj : A.nobj)) return;
-    const int obj = A.order[slot];
+    typedef SxwTeam<Z> Team;
+    const int id = Team::first();
     /* the frame's noise and thresholds (from the device in a planned run) */
     const float backsig = A.pd ? A.pd->backsig : A.backsig;
     const float athresh = A.pd ? A.pd->thresh : A.thresh;
     const float adthresh = A.pd ? A.pd->dthresh : A.dthresh;
-    double *rows = s_rows[wid];
-    float *frows = s_frows[wid];
     const int W = A.W, H = A.H;
     ObjCols o = A.o;
     const int g0 = A.objoff[obj], npx = A.objoff[obj + 1] - g0;
@@ -110,7 +124,7 @@ __global__ void __launch_bounds__(256) k_analyse(AnaArgs A)
         float peak = (float)-SXG_BIG, cpeak = (float)-SXG_BIG;
         int xmin = 2 * SXG_MAXPICSIZE, ymin = 2 * SXG_MAXPICSIZE, xmax = 0, ymax = 0;
 #pragma unroll 4
-        for (int k = lane; k < npx; k += 64) {
+        for (int k = id; k < npx; k += Team::STEP) {
             const int p = P[k];
             const int y = p / W, x = p - y * W;
             peak = fmaxf(peak, A.sub[p]);
@@ -120,27 +134,26 @@ __global__ void __launch_bounds__(256) k_analyse(AnaArgs A)
             ymin = min(ymin, y);
             ymax = max(ymax, y);
         }
-        peak = sxw_max(peak);
-        cpeak = sxw_max(cpeak);
-        xmin = sxw_min(xmin);
-        xmax = sxw_max(xmax);
-        ymin = sxw_min(ymin);
-        ymax = sxw_max(ymax);
+        peak = Team::max(peak);
+        cpeak = Team::max(cpeak);
+        xmin = Team::min(xmin);
+        xmax = Team::max(xmax);
+        ymin = Team::min(ymin);
+        ymax = Team::max(ymax);
         if (xmin == 0 || xmax == W - 1 || ymin == 0 || ymax == H - 1) flag |= SXG_OBJ_TRUNC;
         const double dthresh = (double)odth;
         const double dthresh2 = (dthresh + peak) / 2.0;
-        double acc = 0.0;
-        float racc = 0.0f;
+        SxwSums<6, 1, Z> sums;
         int area2 = 0, dnpix = 0;
         /* the next chunk's pixels are read while this chunk is folded */
-        int np_ = lane < npx ? P[lane] : 0;
-        float nsub = lane < npx ? A.sub[np_] : 0.0f, ncd = lane < npx ? A.cd[np_] : 0.0f;
-        for (int base = 0; base < npx; base += 64) {
-            const int k = base + lane;
+        int np_ = id < npx ? P[id] : 0;
+        float nsub = id < npx ? A.sub[np_] : 0.0f, ncd = id < npx ? A.cd[np_] : 0.0f;
+        for (int base = 0; base < npx; base += Team::STEP) {
+            const int k = base + id;
             const int pc = np_;
             const float csub = nsub, ccd = ncd;
-            if (k + 64 < npx) {
-                np_ = P[k + 64];
+            if (k + Team::STEP < npx) {
+                np_ = P[k + Team::STEP];
                 nsub = A.sub[np_];
                 ncd = A.cd[np_];
             }
@@ -160,14 +173,15 @@ __global__ void __launch_bounds__(256) k_analyse(AnaArgs A)
                 txy = cval * x * y;
             }
             const double t6[6] = {val, tx, ty, txx, tyy, txy};
-            const float tf[1] = {cval};
-            sxw_fold2<6, 1>(rows, frows, t6, tf, k < npx, acc, racc);
+            const float tf[2] = {cval, 0.0f};
+            sums.add(rows, t6, tf, k < npx);
         }
-        const float rv = sxw_rl(racc, 6);
-        const double tv = sxw_rl(acc, 0), mx = sxw_rl(acc, 1), my = sxw_rl(acc, 2);
-        const double mx2 = sxw_rl(acc, 3), my2 = sxw_rl(acc, 4), mxy = sxw_rl(acc, 5);
-        area2 = sxw_sum(area2);
-        dnpix = sxw_sum(dnpix);
+        sums.end(rows);
+        const float rv = sums.f[0];
+        const double tv = sums.d[0], mx = sums.d[1], my = sums.d[2];
+        const double mx2 = sums.d[3], my2 = sums.d[4], mxy = sums.d[5];
+        area2 = Team::sum(area2);
+        dnpix = Team::sum(dnpix);
         Moments m;
         sxg_moments(mx, my, mx2, my2, mxy, rv, (flag & SXG_OBJ_MERGED) != 0, o.mx[obj], o.my[obj],
                     xmin, ymin, area2, dnpix, dthresh, dthresh2, m);
@@ -176,7 +190,7 @@ __global__ void __launch_bounds__(256) k_analyse(AnaArgs A)
         fdflux = rv;
         oa = m.a;
         ob = m.b;
-        if (lane == 0) {
+        if (id == 0) {
             o.fdflux[obj] = rv;
             o.fdpeak[obj] = cpeak;
             o.dpeak[obj] = peak;
@@ -207,7 +221,7 @@ __global__ void __launch_bounds__(256) k_analyse(AnaArgs A)
     SxwTop5 top;
     top.init();
 #pragma unroll 4
-    for (int k = lane; k < npx; k += 64) {
+    for (int k = id; k < npx; k += Team::STEP) {
         const int p = P[k];
         const float pix = A.sub[p];
         pk = fmaxf(pk, pix);
@@ -222,38 +236,48 @@ __global__ void __launch_bounds__(256) k_analyse(AnaArgs A)
         if (pix > athr) area++;
         if (cleanflag) top.add(cdpix - odth);
     }
-    pk = sxw_max(pk);
-    othr = sxw_minf(othr);
-    area = sxw_sum(area);
+    pk = Team::max(pk);
+    othr = Team::min(othr);
+    area = Team::sum(area);
     int peakx = 0, peaky = 0;
     if (A.peakflag) {
-        const float cmax = sxw_max(cdpeak);
-        const int pp = sxw_min(cdpeak == cmax ? peakp : 0x7fffffff);
+        const float cmax = Team::max(cdpeak);
+        const int pp = Team::min(cdpeak == cmax ? peakp : 0x7fffffff);
         peakx = pp % W + 1;
         peaky = pp / W + 1;
     }
-    const float mthresh = cleanflag ? top.fifth() : 0.0f;
+    const float mthresh = cleanflag ? Team::fifth(top) : 0.0f;
     const float thr_o = othr - dbkg, pk_o = pk - dbkg;
+    /* lane i of the row computes threshold i */
     float threshs[SXG_NISO];
-    if (pk_o > 0.0 && thr_o > 0.0)
-        for (int i = 0; i < SXG_NISO; i++)
-            threshs[i] = (float)(thr_o * sx_pow((double)pk_o / thr_o, (double)i / SXG_NISO));
-    else
-        for (int i = 0; i < SXG_NISO; i++) threshs[i] = 0.0f;
+    {
+        const int i = threadIdx.x & (SXG_NISO - 1);
+        float t = 0.0f;
+        if (pk_o > 0.0 && thr_o > 0.0)
+            t = (float)(thr_o * sx_pow((double)pk_o / thr_o, (double)i / SXG_NISO));
+        threshs[0] = sxw_row_bcast<0>(t);
+        threshs[1] = sxw_row_bcast<1>(t);
+        threshs[2] = sxw_row_bcast<2>(t);
+        threshs[3] = sxw_row_bcast<3>(t);
+        threshs[4] = sxw_row_bcast<4>(t);
+        threshs[5] = sxw_row_bcast<5>(t);
+        threshs[6] = sxw_row_bcast<6>(t);
+        threshs[7] = sxw_row_bcast<7>(t);
+    }
     int iso[SXG_NISO] = {0, 0, 0, 0, 0, 0, 0, 0};
     float thresh0 = (float)(pk_o / 5.0);
     if (thresh0 < thr_o) thresh0 = thr_o;
     const double sat = (double)(A.satur_level - dbkg);
-    double eacc = 0.0;
+    SxwSums<11, 0, Z> sums;
     /* the next chunk's pixels are read while this chunk is folded */
-    int np_ = lane < npx ? P[lane] : 0;
-    float nsub = lane < npx ? A.sub[np_] : 0.0f, ncd = lane < npx ? A.cd[np_] : 0.0f;
-    for (int base = 0; base < npx; base += 64) {
-        const int k = base + lane;
+    int np_ = id < npx ? P[id] : 0;
+    float nsub = id < npx ? A.sub[np_] : 0.0f, ncd = id < npx ? A.cd[np_] : 0.0f;
+    for (int base = 0; base < npx; base += Team::STEP) {
+        const int k = base + id;
         const int pc = np_;
         const float csub = nsub, ccd = ncd;
-        if (k + 64 < npx) {
-            np_ = P[k + 64];
+        if (k + Team::STEP < npx) {
+            np_ = P[k + Team::STEP];
             nsub = A.sub[np_];
             ncd = A.cd[np_];
         }
@@ -299,10 +323,12 @@ __global__ void __launch_bounds__(256) k_analyse(AnaArgs A)
         /* tv, sigtv, esum, emx2, emy2, emxy (the error sums only with errflag), then the
            FWHM fit sums */
         const double t11[11] = {pix, var2, err, ex2, ey2, exy, ts, tsx, tsxx, tsy, tsxy};
-        sxw_fold<11, double>(rows, t11, k < npx, eacc);
+        const float none[1] = {0.0f};
+        sums.add(rows, t11, none, k < npx);
     }
-    double tv = sxw_rl(eacc, 0), sigtv = sxw_rl(eacc, 1);
-    const double emx2 = sxw_rl(eacc, 3), emy2 = sxw_rl(eacc, 4), emxy = sxw_rl(eacc, 5);
+    sums.end(rows);
+    double tv = sums.d[0], sigtv = sums.d[1];
+    const double emx2 = sums.d[3], emy2 = sums.d[4], emxy = sums.d[5];
     double pmx2 = 0.0, pmy2 = 0.0, pmxy = 0.0;
     if (A.errflag) {
         const double flux2 = (float)(fdflux * fdflux);
@@ -312,10 +338,10 @@ __global__ void __launch_bounds__(256) k_analyse(AnaArgs A)
     }
     tv -= npx * dbkg;
     if (!A.gainflag && A.gain > 0.0 && tv > 0.0) sigtv += tv / A.gain;
-    const double s = sxw_rl(eacc, 6), sx = sxw_rl(eacc, 7), sxx = sxw_rl(eacc, 8);
-    const double sy = sxw_rl(eacc, 9), sxy = sxw_rl(eacc, 10);
+    const double s = sums.d[6], sx = sums.d[7], sxx = sums.d[8];
+    const double sy = sums.d[9], sxy = sums.d[10];
 #pragma unroll
-    for (int i = 0; i < SXG_NISO; i++) iso[i] = sxw_sum(iso[i]);
+    for (int i = 0; i < SXG_NISO; i++) iso[i] = Team::sum(iso[i]);
     float fwhm = 0.0f;
     if (A.fwhmflag && thresh0 > 0.0) {
         const double d = s * sxx - sx * sx;
@@ -327,7 +353,7 @@ __global__ void __launch_bounds__(256) k_analyse(AnaArgs A)
         }
     }
     if (pk_o + bkg >= A.satur_level) flag |= SXG_OBJ_SATUR;
-    if (lane != 0) return;
+    if (id != 0) return;
     o.fdnpix[obj] = npx;
     o.dthresh[obj] = odth;   /* the detection threshold from here on */
     o.mthresh[obj] = mthresh;
@@ -350,9 +376,35 @@ __global__ void __launch_bounds__(256) k_analyse(AnaArgs A)
     o.flag[obj] = flag;
 }
 
+/* by size: the largest a workgroup each, the next four, the small ones sixteen to a
+   workgroup (k_obj_order; the grid is an upper bound, the host does not know the numbers) */
+__global__ void __launch_bounds__(256) k_analyse(AnaArgs A)
+{
+    __shared__ double s_rows[sxw_brows(11, 0)];
+    static_assert(sxw_brows(11, 0) >= 4 * sxw_wrows(11, 0), "four wavefronts' rows");
+    const int nobj = A.pd ? A.pd->nobj : A.nobj;
+    const int nbig = A.order[2 * A.nobj], nmid = A.order[2 * A.nobj + 1];
+    const int *const mid = A.order + A.nobj;
+    int b = blockIdx.x;
+    if (b < nbig) {
+        ana_object<SXW_GROUP>(A, A.order[b], s_rows);
+        return;
+    }
+    b -= nbig;
+    if (4 * b < nmid) {
+        const int wid = threadIdx.x >> 6;
+        if (4 * b + wid < nmid)
+            ana_object<SXW_WAVE>(A, mid[4 * b + wid], s_rows + wid * sxw_wrows(11, 0));
+        return;
+    }
+    b -= (nmid + 3) / 4;
+    const int slot = nbig + nmid + b * 16 + (threadIdx.x >> 4);
+    if (slot < nobj) ana_object<SXW_ROWS>(A, A.order[slot], s_rows);
+}
+
 __global__ void k_ana_zero2(int *p)
 {
-    if (threadIdx.x < 2) p[threadIdx.x] = 0;
+    if (threadIdx.x < 3) p[threadIdx.x] = 0;
 }
 
 extern "C" void analyse_gpu(double flagobj_poserr_mx2, int flagobj_peakx, int flagobj_iso_0,
@@ -405,18 +457,22 @@ extern "C" void analyse_gpu(double flagobj_poserr_mx2, int flagobj_peakx, int fl
     A.rawt0 = ro.t0;
     if (!sxg_obj_view(A.o)) return;
     S.clean_enabled = prefs_clean_flag != 0;
-    int *order = sxg_take<int>("ana.order", (size_t)numobj + 2);
+    int *order = sxg_take<int>("ana.order", 2 * (size_t)numobj + 3);
     if (!order) return;
     A.order = order;
     /* a planned run: numobj is a capacity, the count and thresholds are on the device */
     A.pd = S.plan ? S.pdev : nullptr;
     sxg_stage_begin(ST_ANALYSE);
-    /* the two counters of k_obj_order (a fill kernel: no memset node in a graph) */
-    hipLaunchKernelGGL(k_ana_zero2, dim3(1), dim3(64), 0, S.stream, order + numobj);
+    /* the counters of k_obj_order (a fill kernel: no memset node in a graph) */
+    hipLaunchKernelGGL(k_ana_zero2, dim3(1), dim3(64), 0, S.stream, order + 2 * numobj);
     hipLaunchKernelGGL(k_obj_order, dim3(sxg_div_up(numobj, 256)), dim3(256), 0, S.stream,
-                       S.objoff, numobj, order + numobj, order, A.pd);
+                       S.objoff, numobj, order + 2 * (size_t)numobj, order, A.pd);
     sxg_kt_begin(SXG_KT_ANALYSE);
-    hipLaunchKernelGGL(k_analyse, dim3(sxg_div_up(numobj, 4)), dim3(256), 0, S.stream, A);
+    const int grid = (int)(S.npix_raw / ANA_BIG) + 1 +
+                     sxg_div_up(std::min<long>(numobj, S.npix_raw / ANA_MID), 4) + 1 +
+                     sxg_div_up(numobj, 16);
+    hipLaunchKernelGGL(k_analyse, dim3(grid), dim3(256), 0,
+                       S.stream, A);
     sxg_kt_end(SXG_KT_ANALYSE);
     sxg_stage_end(ST_ANALYSE);
     /* no host output: the next entry points run on the same stream */

@@ -28,6 +28,7 @@ __device__ inline double sxw_rl(double v, int j)
     return __hiloint2double(hi, lo);
 }
 
+template <int N> struct SxwInt { static constexpr int value = N; };
 template <class Op> __device__ inline float sxw_dpp_allf(float v, Op op);
 struct SxwMaxF { __device__ float operator()(float a, float b) const { return fmaxf(a, b); } };
 struct SxwMinF { __device__ float operator()(float a, float b) const { return fminf(a, b); } };
@@ -143,11 +144,10 @@ struct SxwTop5 {
             v = lo;
         }
     }
-    /* the fifth largest value over the wavefront (needs >= 5 values in total) */
-    __device__ float fifth()
+    /* the five largest values over the wavefront, in descending order (-inf: none) */
+    __device__ void five(float (&r)[5])
     {
         const int lane = threadIdx.x & 63;
-        float res = 0.0f;
 #pragma unroll
         for (int round = 0; round < 5; round++) {
             const float m = sxw_max(t[0]);
@@ -157,10 +157,11 @@ struct SxwTop5 {
                 for (int i = 0; i < 4; i++) t[i] = t[i + 1];
                 t[4] = -INFINITY;
             }
-            res = m;
+            r[round] = m;
         }
-        return res;
     }
+    /* the same over the row of 16 lanes */
+    __device__ void row_five(float (&r)[5]);
 };
 
 /*
@@ -241,3 +242,198 @@ __device__ inline void sxw_fold2(double *drows, float *frows, const double (&td)
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+/*
+ * The same over a workgroup of four wavefronts, for the objects whose sums are the longest:
+ * 256 pixels a step, one per thread.  All four compute terms, then each adds three of the
+ * sums, a row of 16 lanes each (sxw_row_fold), so the longest chain is 256 adds of 4.3
+ * cycles for 256 pixels instead of 16 to 33 cycles a pixel (LDS reads and adds of one
+ * wavefront).  A pixel left out adds +0, an identity (a sum that starts at +0 is never -0).
+ * ND double sums (up to 9, or 12 without float sums: wavefront w has 3w .. 3w + 2), NF float
+ * sums (up to 4, wavefront 3).  rows: sxw_brows(ND, NF) doubles.  All 256 threads call it.
+ */
+#define SXW_BROW 272   /* row stride in elements: two rows of lanes on all banks */
+constexpr int sxw_brows(int nd, int nf) { return nd * SXW_BROW + (nf * SXW_BROW + 1) / 2; }
+
+template <int ND, int NF>
+__device__ inline void sxw_bfold(double *rows, const double (&td)[ND], const float (&tf)[NF + 1],
+                                 bool member, double &dacc, float &facc)
+{
+    static_assert(ND <= (NF ? 9 : 12) && NF <= 4, "three sums a wavefront");
+    const int tid = threadIdx.x, wid = tid >> 6, row = (tid >> 4) & 3, l16 = tid & 15;
+    float *frows = reinterpret_cast<float *>(rows + ND * SXW_BROW);
+#pragma unroll
+    for (int s = 0; s < ND; s++) rows[s * SXW_BROW + tid] = member ? td[s] : 0.0;
+#pragma unroll
+    for (int s = 0; s < NF; s++) frows[s * SXW_BROW + tid] = member ? tf[s] : 0.0f;
+    __syncthreads();
+    if (NF && wid == 3) {
+        const float *p = frows + min(row, NF > 0 ? NF - 1 : 0) * SXW_BROW + l16;
+#pragma unroll
+        for (int c = 0; c < 16; c++) facc = sxw_row_fold(facc, p[16 * c]);
+    } else if (3 * wid < ND) {
+        const double *p = rows + min(3 * wid + row, ND - 1) * SXW_BROW + l16;
+#pragma unroll
+        for (int c = 0; c < 16; c++) dacc = sxw_row_fold(dacc, p[16 * c]);
+    }
+    __syncthreads();
+}
+
+/* the sums of sxw_bfold, to every thread */
+template <int ND, int NF>
+__device__ inline void sxw_bfold_end(double *rows, double dacc, float facc, double (&d)[ND],
+                                     float (&f)[NF + 1])
+{
+    const int tid = threadIdx.x, wid = tid >> 6, row = (tid >> 4) & 3, l16 = tid & 15;
+    float *frows = reinterpret_cast<float *>(rows + ND);
+    if (l16 == 0 && row < 3 && 3 * wid + row < ND) rows[3 * wid + row] = dacc;
+    if (NF && l16 == 0 && wid == 3 && row < NF) frows[row] = facc;
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < ND; s++) d[s] = rows[s];
+#pragma unroll
+    for (int s = 0; s < NF; s++) f[s] = frows[s];
+    __syncthreads();
+}
+
+/* value of v in lane J of the row of 16 */
+template <int J> __device__ inline float sxw_row_bcast(float v)
+{
+    const int i = __float_as_int(v);
+    return __int_as_float(__builtin_amdgcn_update_dpp(i, i, 0x150 + J, 0xF, 0xF, false));
+}
+/* op over the 16 lanes of a row, the result in every lane of it */
+template <class V, class Op> __device__ inline V sxw_row_all(V v, Op op)
+{
+    static_assert(sizeof(V) == 4, "one register");
+    auto mv = [](V x, auto ctrl) {
+        const int i = __builtin_bit_cast(int, x);
+        return __builtin_bit_cast(
+            V, __builtin_amdgcn_update_dpp(i, i, decltype(ctrl)::value, 0xF, 0xF, false));
+    };
+    v = op(v, mv(v, SxwInt<0xB1>{}));
+    v = op(v, mv(v, SxwInt<0x4E>{}));
+    v = op(v, mv(v, SxwInt<0x141>{}));
+    return op(v, mv(v, SxwInt<0x140>{}));
+}
+
+__device__ inline void SxwTop5::row_five(float (&r)[5])
+{
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int round = 0; round < 5; round++) {
+        const float m = sxw_row_all(t[0], SxwMaxF{});
+        const unsigned b = (unsigned)(__ballot(t[0] == m) >> (lane & 48)) & 0xffffu;
+        if ((lane & 15) == __builtin_ctz(b)) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) t[i] = t[i + 1];
+            t[4] = -INFINITY;
+        }
+        r[round] = m;
+    }
+}
+
+/*
+ * One object by a row of 16 lanes (SXW_ROWS: the many small ones; four share a wavefront,
+ * and with it every instruction of the per-object arithmetic), by a wavefront (SXW_WAVE) or
+ * by a workgroup of four (SXW_GROUP): the pixel index a thread starts at, the step, and
+ * reductions over all of its threads.  Rows may be in different places of the program; the
+ * lanes of a row are not.
+ */
+enum SxwSize { SXW_ROWS, SXW_WAVE, SXW_GROUP };
+
+template <SxwSize Z> struct SxwTeam {
+    static constexpr int STEP = Z == SXW_GROUP ? 256 : Z == SXW_WAVE ? 64 : 16;
+    __device__ static int first() { return threadIdx.x & (STEP - 1); }
+    template <class V, class Op> __device__ static V all(V v, Op op)
+    {
+        v = sxw_row_all(v, op);
+        if constexpr (Z == SXW_WAVE) {
+            const int i = __builtin_bit_cast(int, v);
+            auto rl = [&](int j) {
+                return __builtin_bit_cast(V, __builtin_amdgcn_readlane(i, j));
+            };
+            v = op(op(rl(0), rl(16)), op(rl(32), rl(48)));
+        }
+        if constexpr (Z == SXW_GROUP) {
+            __shared__ V s[16];
+            if ((threadIdx.x & 15) == 0) s[threadIdx.x >> 4] = v;
+            __syncthreads();
+            v = sxw_row_all(s[threadIdx.x & 15], op);
+            __syncthreads();
+        }
+        return v;
+    }
+    __device__ static float max(float v) { return all(v, SxwMaxF{}); }
+    __device__ static float min(float v) { return all(v, SxwMinF{}); }
+    __device__ static int max(int v) { return all(v, SxwMax{}); }
+    __device__ static int min(int v) { return all(v, SxwMin{}); }
+    __device__ static int sum(int v) { return all(v, SxwAdd{}); }
+    /* the fifth largest value (needs at least five) */
+    __device__ static float fifth(SxwTop5 &t)
+    {
+        float r[5];
+        if constexpr (Z == SXW_WAVE) {
+            t.five(r);
+            return r[4];
+        }
+        t.row_five(r);
+        if constexpr (Z == SXW_GROUP) {
+            __shared__ float s[16][5];
+            if ((threadIdx.x & 15) == 0)
+                for (int i = 0; i < 5; i++) s[threadIdx.x >> 4][i] = r[i];
+            __syncthreads();
+            for (int i = 0; i < 5; i++) t.t[i] = s[threadIdx.x & 15][i];
+            __syncthreads();
+            t.row_five(r);
+        }
+        return r[4];
+    }
+};
+
+/* the ordered sums of an object: ND double and NF float ones; rows: LDS, for a workgroup
+   sxw_brows(ND, NF) doubles, for a wavefront its own sxw_wrows(ND, NF), none for a row */
+constexpr int sxw_wrows(int nd, int nf) { return nd * SXW_ROW + (nf * SXW_ROW + 1) / 2; }
+template <int ND, int NF, SxwSize Z> struct SxwSums {
+    double d[ND];
+    float f[NF + 1];
+    __device__ SxwSums()
+    {
+#pragma unroll
+        for (int s = 0; s < ND; s++) d[s] = 0.0;
+#pragma unroll
+        for (int s = 0; s <= NF; s++) f[s] = 0.0f;
+    }
+    __device__ void add(double *rows, const double (&td)[ND], const float (&tf)[NF + 1],
+                        bool member)
+    {
+        if constexpr (Z == SXW_GROUP) {
+            sxw_bfold<ND, NF>(rows, td, tf, member, d[0], f[0]);
+        } else if constexpr (Z == SXW_WAVE && NF > 0) {
+            float t[NF];
+#pragma unroll
+            for (int s = 0; s < NF; s++) t[s] = tf[s];
+            sxw_fold2<ND, NF>(rows, reinterpret_cast<float *>(rows + ND * SXW_ROW), td, t, member,
+                              d[0], f[0]);
+        } else if constexpr (Z == SXW_WAVE) {
+            sxw_fold<ND, double>(rows, td, member, d[0]);
+        } else {
+#pragma unroll
+            for (int s = 0; s < ND; s++) d[s] = sxw_row_fold(d[s], member ? td[s] : 0.0);
+#pragma unroll
+            for (int s = 0; s < NF; s++) f[s] = sxw_row_fold(f[s], member ? tf[s] : 0.0f);
+        }
+    }
+    __device__ void end(double *rows)
+    {
+        if constexpr (Z == SXW_GROUP) {
+            sxw_bfold_end<ND, NF>(rows, d[0], f[0], d, f);
+        } else if constexpr (Z == SXW_WAVE) {
+            const double a = d[0];
+            const float b = f[0];
+#pragma unroll
+            for (int s = 0; s < ND; s++) d[s] = sxw_rl(a, s);
+#pragma unroll
+            for (int s = 0; s < NF; s++) f[s] = sxw_rl(b, ND + s);
+        }
+    }
+};
