@@ -64,12 +64,15 @@ __global__ void __launch_bounds__(256) k_obj_order(const int *objoff, int nobj, 
     if (pd) nobj = pd->nobj;
     if (obj >= nobj) return;
     const int n = objoff[obj + 1] - objoff[obj];
+    const int big = sxw_place(&cnt[0], n >= ANA_BIG);
+    const int mid = sxw_place(&cnt[1], n >= ANA_MID && n < ANA_BIG);
+    const int low = sxw_place(&cnt[2], n < ANA_MID);
     if (n >= ANA_BIG)
-        order[atomicAdd(&cnt[0], 1)] = obj;
+        order[big] = obj;
     else if (n >= ANA_MID)
-        order[cap + atomicAdd(&cnt[1], 1)] = obj;
+        order[cap + mid] = obj;
     else
-        order[nobj - 1 - atomicAdd(&cnt[2], 1)] = obj;
+        order[nobj - 1 - low] = obj;
 }
 
 /* back.c:685-732 */

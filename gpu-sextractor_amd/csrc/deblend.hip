@@ -818,7 +818,7 @@ __device__ __forceinline__ void deb_tree(const DebArgs &a, const int r, const in
     if (!(deb_ld<false>(&s_top) & D::NOTA)) {
         /* no split: the raw object is kept as it is */
         if (tid == 0) {
-            C[0] = {0, fp[0], COMP_KEPT};
+            C[0] = {0, fp[0], 0, n - 1};
             a.rootnc[r] = 1;
             a.rootkept[r] = 1;
         }
@@ -879,13 +879,22 @@ __device__ __forceinline__ void deb_tree(const DebArgs &a, const int r, const in
         }
         if (j < nk) {
             deb_st<G>(&slot[j], rank);
-            C[rank] = {D::lev(key), fp[(int)(key & D::IM)], COMP_KEPT};
+            const int lo = (int)(key & D::IM);
+            C[rank] = {D::lev(key), fp[lo], lo, lo};
         }
     }
     deb_sync<G || PG>();
-    for (int k = tid; k < n; k += NT) {
-        const IT s = deb_ld<G>(&list[k]);
-        a.kcomp[off + k] = s == (IT)-1 ? -1 : deb_ld<G>(&slot[s]);
+    /* the last pixel of each kept node: from the last of every run of its pixels */
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    for (int b0 = 0; b0 < n; b0 += NT) {
+        const int k = b0 + tid;
+        const IT s = k < n ? deb_ld<G>(&list[k]) : (IT)-1;
+        const int c = s == (IT)-1 ? -1 : deb_ld<G>(&slot[s]);
+        const int next = __shfl_down(c, 1);
+        if (k >= n) continue;
+        a.kcomp[off + k] = c;
+        if (c >= 0 && (lane == 63 || k == n - 1 || next != c)) atomicMax(&C[c].hi, k);
     }
     if (tid == 0) {
         a.rootnc[r] = nk;
@@ -978,88 +987,78 @@ struct ObjArgs {
     const int *order;       /* objects in launch order: those of large raw objects first */
 };
 
-/* objects whose raw object has at least PRE_BIG pixels are preanalysed first (each scans
-   its raw object's list) */
-#define PRE_BIG 256
+/* nodes whose entries lo .. hi are at least PRE_BIG take a workgroup each, at least PRE_MID a
+   wavefront, the others a row of 16 lanes */
+#ifndef PRE_BIG
+#define PRE_BIG 512
+#define PRE_MID 32
+#endif
 
 /* the objects: the device count of a planned run */
 __device__ inline int obj_n(const ObjArgs &A) { return A.d.pd ? A.d.pd->nobj : A.nobj; }
 
+/* the objects by size: order[0, nbig) the big ones, order[nbig + nmid, nobj) the small ones,
+   order[cap, cap + nmid) those between; cnt: their numbers */
 __global__ void __launch_bounds__(256) k_pre_order(ObjArgs A, int *cnt, int *order)
 {
     const int obj = blockIdx.x * 256 + threadIdx.x;
     const int nobj = obj_n(A);
     if (obj >= nobj) return;
-    if (A.d.cnt[A.objraw[obj]] >= PRE_BIG)
-        order[atomicAdd(&cnt[0], 1)] = obj;
+    const Comp c = A.d.comps[A.d.compoff[A.objraw[obj]] + A.objcomp[obj]];
+    const int n = c.hi - c.lo + 1;
+    const int big = sxw_place(&cnt[0], n >= PRE_BIG);
+    const int mid = sxw_place(&cnt[1], n >= PRE_MID && n < PRE_BIG);
+    const int low = sxw_place(&cnt[2], n < PRE_MID);
+    if (n >= PRE_BIG)
+        order[big] = obj;
+    else if (n >= PRE_MID)
+        order[A.nobj + mid] = obj;
     else
-        order[nobj - 1 - atomicAdd(&cnt[1], 1)] = obj;
+        order[nobj - 1 - low] = obj;
 }
 
 /* objects of each raw object, in component-table order (one wavefront per raw object) */
-__global__ void __launch_bounds__(256) k_deb_objlist(ObjArgs A, int *zero2)
+__global__ void __launch_bounds__(256) k_deb_objlist(ObjArgs A, int *zero3)
 {
-    /* the two counters of k_pre_order start at zero (no fill launch) */
-    if (blockIdx.x == 0 && threadIdx.x < 2) zero2[threadIdx.x] = 0;
+    /* the counters of k_pre_order start at zero (no fill launch) */
+    if (blockIdx.x == 0 && threadIdx.x < 3) zero3[threadIdx.x] = 0;
     const int lane = threadIdx.x & 63;
     const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (r >= deb_nraw(A.d)) return;
     const int nc = A.d.rootnc[r], base = A.objbase[r];
-    Comp *C = A.d.comps + A.d.compoff[r];
-    if (A.d.lstar[r] == 0) {
-        /* a single local maximum: the raw object is the object */
-        if (lane == 0) {
-            Comp c0;
-            c0.level = 0;
-            c0.first = A.d.first[r];
-            c0.flags = COMP_KEPT;
-            C[0] = c0;
-            A.objraw[base] = r;
-            A.objcomp[base] = 0;
-        }
-        return;
-    }
-    const unsigned long long below = sxw_lanes_below(lane);
-    int done = 0;
-    for (int c0 = 0; c0 < nc; c0 += 64) {
-        const int c = c0 + lane;
-        const bool kept = c < nc && (C[c].flags & COMP_KEPT);
-        const unsigned long long b = __ballot(kept);
-        if (kept) {
-            const int j = base + done + __popcll(b & below);
-            A.objraw[j] = r;
-            A.objcomp[j] = c;
-        }
-        done += __popcll(b);
+    /* a single local maximum: the raw object is the object */
+    if (A.d.lstar[r] == 0 && lane == 0)
+        A.d.comps[A.d.compoff[r]] = {0, A.d.first[r], 0, A.d.cnt[r] - 1};
+    for (int c = lane; c < nc; c += 64) {
+        A.objraw[base + c] = r;
+        A.objcomp[base + c] = c;
     }
 }
 
 
 /*
- * FULL preanalysis of each kept component over its level pixels (one wavefront per
- * object); the component's pixels get the object index.
+ * FULL preanalysis of each kept node over its level pixels, by a row of 16 lanes, a wavefront
+ * or a workgroup (SxwTeam); the node's pixels get the object index.  Bound: the sequential
+ * sums of the largest nodes (7 cycles a pixel), then the latency of the loads.  A node reads
+ * its own stretch of the raw object's list only.  Measured (a wavefront per node over the whole raw object before): crowded
+ * 4096^2 95 -> 45 us, dense 2048^2 253 -> 74, 2048^2 with saturated stars 68 -> 24.
  */
-__global__ void __launch_bounds__(256) k_deb_pre(ObjArgs A)
+template <SxwSize Z>
+__device__ __forceinline__ void pre_object(const ObjArgs &A, const int obj, double *rows)
 {
-    __shared__ double s_rows[4][6 * SXW_ROW];
-    __shared__ float s_frows[4][SXW_ROW];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const int slot = blockIdx.x * 4 + wid;
-    if (slot >= obj_n(A)) return;
-    const int obj = A.order[slot];
-    double *rows = s_rows[wid];
-    float *frows = s_frows[wid];
+    typedef SxwTeam<Z> Team;
+    const int id = Team::first();
     const DebArgs &d = A.d;
     const int r = A.objraw[obj], c = A.objcomp[obj];
-    const Comp *C = d.comps + d.compoff[r];
-    const int L = C[c].level;
-    const int n = d.cnt[r], off = d.off[r], W = d.W, H = d.H;
+    const Comp C = d.comps[d.compoff[r] + c];
+    const int L = C.level;
+    const int n = C.hi - C.lo + 1, off = d.off[r] + C.lo, W = d.W, H = d.H;
     const int *lv = L > 0 ? d.kcomp + off : nullptr;
     /* extent, peaks, count (reductions); the node's pixels get the object index */
     float peak = (float)-SXG_BIG, cpeak = (float)-SXG_BIG;
     int xmin = 2 * SXG_MAXPICSIZE, ymin = 2 * SXG_MAXPICSIZE, xmax = 0, ymax = 0, cnt = 0;
 #pragma unroll 4
-    for (int k = lane; k < n; k += 64) {
+    for (int k = id; k < n; k += Team::STEP) {
         if (lv && lv[k] != c) continue;
         const int p = d.fpia[off + k];
         const int y = p / W, x = p - y * W;
@@ -1072,32 +1071,31 @@ __global__ void __launch_bounds__(256) k_deb_pre(ObjArgs A)
         ymax = max(ymax, y);
         cnt++;
     }
-    peak = sxw_max(peak);
-    cpeak = sxw_max(cpeak);
-    xmin = sxw_min(xmin);
-    xmax = sxw_max(xmax);
-    ymin = sxw_min(ymin);
-    ymax = sxw_max(ymax);
-    cnt = sxw_sum(cnt);
+    peak = Team::max(peak);
+    cpeak = Team::max(cpeak);
+    xmin = Team::min(xmin);
+    ymin = Team::min(ymin);
+    xmax = Team::max(xmax);
+    ymax = Team::max(ymax);
+    cnt = Team::sum(cnt);
     int flag = L > 0 ? SXG_OBJ_MERGED : 0;
     if (xmin == 0 || xmax == W - 1 || ymin == 0 || ymax == H - 1) flag |= SXG_OBJ_TRUNC;
     const double dthresh = (double)d.thr[(size_t)r * d.nthresh + L];
     const double dthresh2 = (dthresh + peak) / 2.0;
     /* one fold pass: rv, the raster-order float sum of cd, and the moments, double sums
-       of float terms in raster order (independent chains, one lane each) */
-    double acc = 0.0;
-    float racc = 0.0f;
+       of float terms in raster order */
+    SxwSums<6, 1, Z> sums;
     int area2 = 0, dnpix = 0;
     /* the next chunk's membership and pixel are read while this chunk is folded */
-    bool nin = lane < n && (!lv || lv[lane] == c);
-    int npix_ = lane < n ? d.fpia[off + lane] : 0;
-    for (int base = 0; base < n; base += 64) {
-        const int k = base + lane;
+    bool nin = id < n && (!lv || lv[id] == c);
+    int npix_ = id < n ? d.fpia[off + id] : 0;
+    for (int base = 0; base < n; base += Team::STEP) {
+        const int k = base + id;
         const bool in = nin;
         const int pc = npix_;
-        if (k + 64 < n) {
-            nin = !lv || lv[k + 64] == c;
-            npix_ = d.fpia[off + k + 64];
+        if (k + Team::STEP < n) {
+            nin = !lv || lv[k + Team::STEP] == c;
+            npix_ = d.fpia[off + k + Team::STEP];
         } else {
             nin = false;
         }
@@ -1116,22 +1114,21 @@ __global__ void __launch_bounds__(256) k_deb_pre(ObjArgs A)
             txy = cval * x * y;
         }
         const double t6[6] = {val, tx, ty, txx, tyy, txy};
-        const float tf[1] = {cval};
-        sxw_fold2<6, 1>(rows, frows, t6, tf, in, acc, racc);
+        const float tf[2] = {cval, 0.0f};
+        sums.add(rows, t6, tf, in);
     }
-    const float rv = sxw_rl(racc, 6);
-    const double tv = sxw_rl(acc, 0), mx = sxw_rl(acc, 1), my = sxw_rl(acc, 2);
-    const double mx2 = sxw_rl(acc, 3), my2 = sxw_rl(acc, 4), mxy = sxw_rl(acc, 5);
-    area2 = sxw_sum(area2);
-    dnpix = sxw_sum(dnpix);
-    if (lane != 0) return;
+    sums.end(rows);
+    const float rv = sums.f[0];
+    area2 = Team::sum(area2);
+    dnpix = Team::sum(dnpix);
+    if (id != 0) return;
     Moments m;
-    sxg_moments(mx, my, mx2, my2, mxy, rv, false, 0.0, 0.0, xmin, ymin, area2, dnpix, dthresh,
-                dthresh2, m);
+    sxg_moments(sums.d[1], sums.d[2], sums.d[3], sums.d[4], sums.d[5], rv, false, 0.0, 0.0, xmin,
+                ymin, area2, dnpix, dthresh, dthresh2, m);
     ObjCols &o = const_cast<ObjCols &>(A.o);
     o.level[obj] = L;
     o.root[obj] = r;
-    o.firstpix[obj] = C[c].first;
+    o.firstpix[obj] = C.first;
     o.flag[obj] = flag;
     o.fdnpix[obj] = cnt;
     o.dnpix[obj] = dnpix;
@@ -1139,18 +1136,45 @@ __global__ void __launch_bounds__(256) k_deb_pre(ObjArgs A)
     o.fdflux[obj] = rv;
     o.fdpeak[obj] = cpeak;
     o.dpeak[obj] = peak;
-    o.dflux[obj] = (float)tv;
+    o.dflux[obj] = (float)sums.d[0];
     o.dthresh[obj] = (float)dthresh;
     sxg_store_moments(o, obj, m);
 }
 
+/* by size (k_pre_order; the grid is an upper bound, the host does not know the numbers) */
+__global__ void __launch_bounds__(256) k_deb_pre(ObjArgs A)
+{
+    __shared__ double s_rows[std::max(4 * sxw_wrows(6, 1), sxw_brows(6, 1))];
+    const int nobj = obj_n(A);
+    const int nbig = A.order[2 * A.nobj], nmid = A.order[2 * A.nobj + 1];
+    int b = blockIdx.x;
+    if (b < nbig) {
+        pre_object<SXW_GROUP>(A, A.order[b], s_rows);
+        return;
+    }
+    b -= nbig;
+    if (4 * b < nmid) {
+        const int wid = threadIdx.x >> 6;
+        if (4 * b + wid < nmid)
+            pre_object<SXW_WAVE>(A, A.order[A.nobj + 4 * b + wid],
+                                 s_rows + wid * sxw_wrows(6, 1));
+        return;
+    }
+    b -= (nmid + 3) / 4;
+    const int slot = nbig + nmid + b * 16 + (threadIdx.x >> 4);
+    if (slot < nobj) pre_object<SXW_ROWS>(A, A.order[slot], s_rows);
+}
+
 /* gatherup: every unassigned pixel goes to the nearest kept object of its raw object
    in the ellipse metric (first minimum in object order); then the sort keys */
-__global__ void __launch_bounds__(256) k_deb_gather(ObjArgs A, int *objcnt, long nz)
+__global__ void __launch_bounds__(256) k_deb_gather(ObjArgs A, int *objcnt, int2 *objspan, long nz)
 {
     const long g = (long)blockIdx.x * 256 + threadIdx.x;
-    /* the per-object pixel counts of k_deb_objcount start at zero (no fill launch) */
-    if (g < nz) objcnt[g] = 0;
+    /* the per-object pixel counts and spans of k_deb_objcount start empty (no fill launch) */
+    if (g < nz) {
+        objcnt[g] = 0;
+        objspan[g] = {0x7fffffff, -1};
+    }
     if (g >= deb_P0(A.d)) return;
     const int p = A.d.fpia[g];
     const int r = A.d.rawkey[g];
@@ -1182,9 +1206,10 @@ __global__ void __launch_bounds__(256) k_deb_gather(ObjArgs A, int *objcnt, long
     A.oval[g] = p;
 }
 
-/* pixels per object; lanes with the same object (long runs: the list is grouped by raw
-   object) add their count once */
-__global__ void __launch_bounds__(256) k_deb_objcount(ObjArgs A, int *objcnt)
+/* pixels per object, and for those of split raw objects the first and last list entry of
+   each; lanes with the same object (long runs: the list is grouped by raw object) add their
+   count once */
+__global__ void __launch_bounds__(256) k_deb_objcount(ObjArgs A, int *objcnt, int2 *objspan)
 {
     const long g = (long)blockIdx.x * 256 + threadIdx.x;
     const int lane = threadIdx.x & 63;
@@ -1195,7 +1220,13 @@ __global__ void __launch_bounds__(256) k_deb_objcount(ObjArgs A, int *objcnt)
         const int leader = __builtin_ctzll(pending);
         const int k = __shfl(key, leader);
         const unsigned long long grp = __ballot(act && key == k);
-        if (lane == leader) atomicAdd(&objcnt[k], __popcll(grp));
+        if (lane == leader) {
+            atomicAdd(&objcnt[k], __popcll(grp));
+            if (A.d.rootkept[A.d.rawkey[g]] >= 2) {
+                atomicMin(&objspan[k].x, (int)g);
+                atomicMax(&objspan[k].y, (int)g + 63 - __builtin_clzll(grp) - leader);
+            }
+        }
         if (act && key == k) act = false;
         pending &= ~grp;
     }
@@ -1204,10 +1235,11 @@ __global__ void __launch_bounds__(256) k_deb_objcount(ObjArgs A, int *objcnt)
 /*
  * The raw pixels regrouped by object, stably (each object's pixels in the raster order
  * of its raw object's list), from the object offsets: a raw object kept as one object
- * moves as one block (k_obj_place1, a lane per pixel); a raw object split into several,
- * one wavefront each (k_obj_place_multi), walks its list 64 entries at a time with the
- * next free position of each of its objects in LDS: the lanes of one object take
- * consecutive positions in lane order, and the chunks follow the list's order.
+ * moves as one block (k_obj_place1, a lane per pixel); each object of a split one has a
+ * wavefront (k_obj_place_multi) that picks its pixels from the stretch of the list between
+ * its first and last, 64 entries at a time.  Bound: latency of the longest stretch's reads.
+ * One wavefront per split raw object, which placed all of its objects, took 26 us in a
+ * crowded 4096^2 and 255 us in a dense 2048^2 frame (18,000 entries); now 11 and 27 us.
  */
 __global__ void __launch_bounds__(256) k_obj_place1(ObjArgs A, const int *__restrict__ objoff,
                                                     int *opix)
@@ -1219,69 +1251,34 @@ __global__ void __launch_bounds__(256) k_obj_place1(ObjArgs A, const int *__rest
     opix[objoff[A.okey[g]] + (int)(g - A.d.off[r])] = A.d.fpia[g];
 }
 
-/* positions kept in LDS per wavefront: objects of one raw object per window */
-#define OP_WIN 1024
-/* list chunks of 64 entries read ahead of the one being placed */
+/* list chunks of 64 entries read together */
 #define OP_AHEAD 4
 __global__ void __launch_bounds__(256) k_obj_place_multi(ObjArgs A,
                                                          const int *__restrict__ objoff,
+                                                         const int2 *__restrict__ objspan,
                                                          int *opix)
 {
-    __shared__ int s_next[4][OP_WIN];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const int r = blockIdx.x * 4 + wid;
-    if (r >= deb_nraw(A.d)) return;
-    const int nk = A.d.rootkept[r];
-    if (nk < 2) return;
-    const int base = A.objbase[r], off = A.d.off[r], n = A.d.cnt[r];
+    const int lane = threadIdx.x & 63;
+    const int obj = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (obj >= obj_n(A)) return;
+    const int2 span = objspan[obj];
+    if (span.y < span.x) return;       /* not part of a split raw object */
     const unsigned long long below = sxw_lanes_below(lane);
-    int *nxt = s_next[wid];
-    for (int w0 = 0; w0 < nk; w0 += OP_WIN) {
-        const int wn = min(OP_WIN, nk - w0);
-        for (int j = lane; j < wn; j += 64) nxt[j] = objoff[base + w0 + j];
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        /* chunk c's object ids and pixels, OP_AHEAD chunks in flight */
-        int qk[OP_AHEAD], qp[OP_AHEAD];
+    int at = objoff[obj];
+    for (int k0 = span.x; k0 <= span.y; k0 += 64 * OP_AHEAD) {
+        bool in[OP_AHEAD];
+        int pix[OP_AHEAD];
 #pragma unroll
         for (int u = 0; u < OP_AHEAD; u++) {
-            const int k = u * 64 + lane;
-            qk[u] = k < n ? A.okey[off + k] : -1;
-            qp[u] = k < n ? A.d.fpia[off + k] : 0;
+            const int k = min(k0 + u * 64 + lane, span.y);
+            in[u] = A.okey[k] == obj && k0 + u * 64 + lane <= span.y;
+            pix[u] = A.d.fpia[k];
         }
-        for (int c0 = 0; c0 < n; c0 += 64 * OP_AHEAD) {
 #pragma unroll
-            for (int u = 0; u < OP_AHEAD; u++) {
-                const int c = c0 + u * 64;
-                if (c >= n) break;
-                const int key = qk[u], pix = qp[u];
-                /* the same slot's chunk of the next round */
-                const int kn = c + 64 * OP_AHEAD + lane;
-                qk[u] = kn < n ? A.okey[off + kn] : -1;
-                qp[u] = kn < n ? A.d.fpia[off + kn] : 0;
-                const int j = key - base - w0;
-                bool act = c + lane < n && j >= 0 && j < wn;
-                unsigned long long pending = __ballot(act);
-                while (pending) {
-                    const int lead = __builtin_ctzll(pending);
-                    const int jl = __shfl(j, lead);
-                    const unsigned long long grp = __ballot(act && j == jl);
-                    const int start = nxt[jl];
-                    if (act && j == jl) {
-                        opix[start + __popcll(grp & below)] = pix;
-                        act = false;
-                    }
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                    if (lane == lead) nxt[jl] = start + __popcll(grp);
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                    pending &= ~grp;
-                }
-            }
+        for (int u = 0; u < OP_AHEAD; u++) {
+            const unsigned long long b = __ballot(in[u]);
+            if (in[u]) opix[at + __popcll(b & below)] = pix[u];
+            at += __popcll(b);
         }
     }
 }
@@ -1575,40 +1572,48 @@ extern "C" int parcel_out(float basethresh, int n_thresh, int deb_minarea, size_
         A.objraw = sxg_take<int>("obj.raw", nobj);
         A.objcomp = sxg_take<int>("obj.comp", nobj);
         int *k0 = sxg_take<int>("opix.k0", P0), *v0 = sxg_take<int>("opix.v0", P0);
-        int *k1 = sxg_take<int>("opix.k1", P0), *v1 = sxg_take<int>("opix.v1", P0);
-        int *hist = sxg_take<int>("opix.hist", 256 * (size_t)(sxg_div_up(P0 + 1, 4096) + 1) + 64);
+        int *v1 = sxg_take<int>("opix.v1", P0);
+        int2 *objspan = sxg_take<int2>("obj.pixspan", (size_t)nobj + 1);
         int *objcnt = sxg_take<int>("obj.pixcount", (size_t)nobj + 1);
         int *objoff = sxg_take<int>("obj.pixoff", (size_t)nobj + 1);
-        if (!A.objraw || !A.objcomp || !k0 || !v0 || !k1 || !v1 || !hist || !objcnt || !objoff)
+        if (!A.objraw || !A.objcomp || !k0 || !v0 || !v1 || !objspan || !objcnt || !objoff)
             return -1;
         A.okey = k0;
         A.oval = v0;
         const int gp = sxg_div_up(P0, 256);
         sxg_kt_begin(SXG_KT_DEB_OBJECTS);
-        int *order = sxg_take<int>("pre.order", (size_t)nobj + 2);
+        int *order = sxg_take<int>("pre.order", 2 * (size_t)nobj + 3);
         if (!order) return -1;
         hipLaunchKernelGGL(k_deb_objlist, dim3(sxg_div_up(nraw, 4)), dim3(256), 0, st, A,
-                           order + nobj);
+                           order + 2 * (size_t)nobj);
         hipLaunchKernelGGL(k_pre_order, dim3(sxg_div_up(nobj, 256)), dim3(256), 0, st, A,
-                           order + nobj, order);
+                           order + 2 * (size_t)nobj, order);
         A.order = order;
-        hipLaunchKernelGGL(k_deb_pre, dim3(sxg_div_up(nobj, 4)), dim3(256), 0, st, A);
+        /* workgroups: one an object at the most; fewer where the counts are exact: an object
+           that is a whole raw object has the length of its pixels (the pixels bound how many
+           are long), and a raw object with s > 1 kept nodes adds s - 1 <= 2 (nobj - nraw) in
+           all to the objects, so at most 2 (nobj - nraw) are parts */
+        const long parts = pl ? nobj : 2 * ((long)nobj - nraw);
+        const long bigs = std::min<long>(nobj, P0 / PRE_BIG + parts);
+        const long mids = std::min<long>(nobj, P0 / PRE_MID + parts);
+        const int grid = (int)std::min<long>(nobj + 2, bigs + mids / 4 + nobj / 16 + 3);
+        hipLaunchKernelGGL(k_deb_pre, dim3(grid), dim3(256), 0, st, A);
         /* planned: the counts past the device's nobj stay zero, so the scan over the
            capacity puts the total at objoff[nobj] as well; the gather kernel clears them */
         const long nz = pl ? (long)nobj + 1 : (long)nobj;
         hipLaunchKernelGGL(k_deb_gather, dim3(sxg_div_up(std::max<long>(P0, nz), 256)), dim3(256),
-                           0, st, A, objcnt, nz);
+                           0, st, A, objcnt, objspan, nz);
         sxg_kt_end(SXG_KT_DEB_OBJECTS);
         /* raw pixels regrouped by object (stable: raster order inside each object) */
         sxg_kt_begin(SXG_KT_OBJ_SORT);
-        hipLaunchKernelGGL(k_deb_objcount, dim3(gp), dim3(256), 0, st, A, objcnt);
+        hipLaunchKernelGGL(k_deb_objcount, dim3(gp), dim3(256), 0, st, A, objcnt, objspan);
         if (pl)
             sxg_scan_excl(objcnt, objoff, nobj + 1, nullptr, st);
         else
             sxg_scan_excl(objcnt, objoff, nobj, objoff + nobj, st);
         hipLaunchKernelGGL(k_obj_place1, dim3(gp), dim3(256), 0, st, A, (const int *)objoff, v1);
-        hipLaunchKernelGGL(k_obj_place_multi, dim3(sxg_div_up(nraw, 4)), dim3(256), 0, st, A,
-                           (const int *)objoff, v1);
+        hipLaunchKernelGGL(k_obj_place_multi, dim3(sxg_div_up(nobj, 4)), dim3(256), 0, st, A,
+                           (const int *)objoff, (const int2 *)objspan, v1);
         sxg_kt_end(SXG_KT_OBJ_SORT);
         S.opix = v1;
         S.objoff = objoff;

@@ -6,13 +6,12 @@
 #pragma once
 #include "sxg_internal.h"
 
-#define COMP_KEPT 1
-
-/* deblending-tree node as the object kernels see it, stored in the raw object's region
-   of the table in the reference's order (level, then raster order of the first pixel):
-   level, first (raster index of its first pixel), flags & COMP_KEPT */
+/* kept node of a deblending tree as the object kernels see it, stored in the raw object's
+   region of the table in the reference's order (level, then raster order of the first
+   pixel): level, first (raster index of its first pixel), and the raw-object list entries lo
+   .. hi between its first and last pixel */
 struct Comp {
-    int level, first, flags;
+    int level, first, lo, hi;
 };
 
 /* per-object columns (structure of arrays, object order) */

@@ -15,6 +15,19 @@ __device__ inline unsigned long long sxw_lanes_below(int lane)
     return lane == 0 ? 0ull : (~0ull >> (64 - lane));
 }
 
+/* a place from the counter for every lane with `take` (lane order), one atomic for the
+   wavefront; every lane of it that is active calls */
+__device__ inline int sxw_place(int *counter, bool take)
+{
+    const int lane = threadIdx.x & 63;
+    const unsigned long long b = __ballot(take);
+    if (!b) return 0;
+    const int lead = __builtin_ctzll(b);
+    int base = 0;
+    if (lane == lead) base = atomicAdd(counter, __popcll(b));
+    return __shfl(base, lead) + __popcll(b & sxw_lanes_below(lane));
+}
+
 /* value of v in lane j (j uniform across the wavefront) */
 __device__ inline float sxw_rl(float v, int j)
 {
