@@ -1438,8 +1438,7 @@ void sxg_back_estimate_from(const float *src, int back_size, float backfthresh, 
         return;
     if (!S.plan) {
         float hv[2];
-        SXG_HIP(hipMemcpyAsync(hv, b.outv, sizeof(hv), hipMemcpyDeviceToHost, S.stream));
-        SXG_HIP(hipStreamSynchronize(S.stream));
+        if (!sxg_read_back({{b.outv, hv, 2}})) return;
         S.backmean = hv[0];
         S.backsig = hv[1];
     }

@@ -183,6 +183,7 @@ extern "C" void run_clean(int *masterIndex, double clean_param, int clean_stacks
     double *amp = sxg_take<double>("clean.amp", n), *alpha = sxg_take<double>("clean.alpha", n);
     CleanBox *box = sxg_take<CleanBox>("clean.box", (size_t)sxg_div_up(n > 0 ? n : 1, 64));
     if (!amp || !alpha || !box) return;
+    S.ranked = S.counted = false;
     sxg_stage_begin(ST_CLEAN);
     if (n > 0) {
         hipLaunchKernelGGL(k_clean_prep, dim3(sxg_div_up(n, 256)), dim3(256), 0, S.stream, o, n,
@@ -248,7 +249,7 @@ __global__ void __launch_bounds__(256) k_seg_scatter(const int *fpia, long P0, c
 
 /* the survivors of CLEAN: keep[i], rank[i] (catalogue NUMBER - 1 of a survivor) and their
    number in tot[0] (in a planned run the device's nsurv), all on the device (queued on
-   the context's stream) */
+   the context's stream): once per CLEAN, for the map and the rows alike */
 static bool survivor_ranks(const ObjCols &o, int *&keep, int *&rank, int *&tot)
 {
     SxgState &S = sxg_state();
@@ -256,10 +257,12 @@ static bool survivor_ranks(const ObjCols &o, int *&keep, int *&rank, int *&tot)
     rank = sxg_take<int>("out.rank", S.nobj);
     tot = S.plan ? &S.pdev->nsurv : sxg_take<int>("out.total", 4);
     if (!keep || !rank || !tot) return false;
+    if (S.ranked && !S.plan) return true;
     const int *nd = S.plan ? &S.pdev->nobj : nullptr;
     hipLaunchKernelGGL(k_keepflag, dim3(sxg_div_up(S.nobj, 256)), dim3(256), 0, S.stream,
                        o.master, S.nobj, keep, nd);
     sxg_scan_excl(keep, rank, S.nobj, tot, S.stream, nd);
+    S.ranked = !S.plan;
     return true;
 }
 
@@ -296,11 +299,12 @@ static int *build_map(int mode, int *dst = nullptr)
                        mode, (const int *)(S.plan ? &S.pdev->npix : nullptr));
     sxg_kt_end(SXG_KT_SEG);
     /* a planned run leaves the survivor count on the device */
-    if (mode == 0 && !S.plan) {
+    if (mode == 0 && !S.plan && !S.counted) {
         int ns = 0;
-        if (hipMemcpyAsync(&ns, tot, sizeof(int), hipMemcpyDeviceToHost, S.stream) == hipSuccess &&
-            hipStreamSynchronize(S.stream) == hipSuccess)
+        if (sxg_read_back({{tot, &ns, 1}}, true)) {
             S.nsurv = ns;
+            S.counted = true;
+        }
     }
     return map;
 }
@@ -393,15 +397,16 @@ extern "C" int sxg_get_catalog(sxg_isorow *out, int cap)
         sxg_set_error("sxg_get_catalog: call after run_clean, with an output buffer");
         return -1;
     }
-    if (S.nobj > 0) {
-        /* the number of survivors, read back once */
+    if (S.nobj > 0 && S.ranked && S.counted) {
+        /* the number of survivors came with the segmentation map */
+    } else if (S.nobj > 0) {
         ObjCols o;
         int *keep = nullptr, *rank = nullptr, *tot = nullptr;
         if (!sxg_obj_view(o) || !survivor_ranks(o, keep, rank, tot)) return -1;
         int ns = 0;
-        SXG_HIP_RET(hipMemcpyAsync(&ns, tot, sizeof(int), hipMemcpyDeviceToHost, S.stream), -1);
-        SXG_HIP_RET(hipStreamSynchronize(S.stream), -1);
+        if (!sxg_read_back({{tot, &ns, 1}})) return -1;
         S.nsurv = ns;
+        S.counted = true;
     } else {
         S.nsurv = 0;
     }

@@ -1447,10 +1447,8 @@ extern "C" int parcel_out(float basethresh, int n_thresh, int deb_minarea, size_
             hipLaunchKernelGGL(k_deb_plan_guard, dim3(1), dim3(64), 0, st, dwork, pd, ccount,
                                dtot, (long long)pl->cap[PL_NTOT], gc);
         } else {
-            SXG_HIP_RET(hipMemcpyAsync(cc, ccount, sizeof(cc), hipMemcpyDeviceToHost, st), -1);
-            SXG_HIP_RET(hipMemcpyAsync(&ntot, dtot, sizeof(int), hipMemcpyDeviceToHost, st), -1);
-            SXG_HIP_RET(hipMemcpyAsync(dw, dwork, sizeof(dw), hipMemcpyDeviceToHost, st), -1);
-            SXG_HIP_RET(hipStreamSynchronize(st), -1);
+            if (!sxg_read_back({{ccount, cc, DEB_NCOUNT}, {dtot, &ntot, 1}, {dwork, dw, 6}}))
+                return -1;
             if (dw[2] > (unsigned long long)0x7fffffff) {
                 sxg_set_error("parcel_out: deblending trees exceed 2^31 nodes in one frame");
                 return -1;
@@ -1551,8 +1549,7 @@ extern "C" int parcel_out(float basethresh, int n_thresh, int deb_minarea, size_
                                (const unsigned long long *)dwork, (const int *)ccount, pd);
         } else {
             sxg_scan_excl(rootkept, objbase, nraw, dtot, st);
-            SXG_HIP_RET(hipMemcpyAsync(&nobj, dtot, sizeof(int), hipMemcpyDeviceToHost, st), -1);
-            SXG_HIP_RET(hipStreamSynchronize(st), -1);
+            if (!sxg_read_back({{dtot, &nobj, 1}})) return -1;
             S.seen.cap[PL_NOBJ] = nobj;
         }
     } else if (pl) {
@@ -1561,6 +1558,7 @@ extern "C" int parcel_out(float basethresh, int n_thresh, int deb_minarea, size_
         for (int k = PL_NTOT; k <= PL_NOBJ; k++) S.seen.cap[k] = 0;
     }
     S.nobj = nobj;
+    S.ranked = S.counted = false;
     S.opix = nullptr;
     S.objoff = nullptr;
     ObjCols oc;

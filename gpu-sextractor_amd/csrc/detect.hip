@@ -245,15 +245,13 @@ __global__ void __launch_bounds__(256) k_det_rootflag(const int *__restrict__ rk
 
 __global__ void __launch_bounds__(256) k_det_rawinfo(const int *__restrict__ rawpos, int nraw,
                                                      const int *__restrict__ fg, int W,
-                                                     RootStat rs,
-                                                     int *rawid_of_pos, RawObj ro, float t,
+                                                     RootStat rs, RawObj ro, float t,
                                                      int perpix, const int *nd, const float *td)
 {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= sxg_dn(nd, nraw)) return;
     if (td) t = *td;
     const int k = rawpos[i];
-    rawid_of_pos[k] = i;
     ro.first[i] = fg[k];
     ro.count[i] = rs.cnt[k];
     ro.fdpeak[i] = ord2f(rs.peak[k]);
@@ -264,6 +262,15 @@ __global__ void __launch_bounds__(256) k_det_rawinfo(const int *__restrict__ raw
     ro.t0[i] = perpix ? ord2f(rs.t0[k]) : t;
 }
 
+
+/* the raw object number at each kept component's root entry */
+__global__ void __launch_bounds__(256) k_det_rawid(const int *__restrict__ rawpos,
+                                                   const int *__restrict__ nraw,
+                                                   int *rawid_of_pos)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < *nraw) rawid_of_pos[rawpos[i]] = i;
+}
 
 /* object id of each detected pixel (or -1 when its component is too small) */
 __global__ void __launch_bounds__(256) k_det_pixkey(const int *__restrict__ rk, int nfg,
@@ -291,17 +298,6 @@ __global__ void __launch_bounds__(256) k_det_copy(const float *a, float *b, long
 {
     const long k = (long)blockIdx.x * 256 + threadIdx.x;
     if (k < n) b[k] = a[k];
-}
-
-static int read_count(const int *d, hipStream_t s)
-{
-    int h = 0;
-    if (hipMemcpyAsync(&h, d, sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess ||
-        hipStreamSynchronize(s) != hipSuccess) {
-        sxg_set_error("run_detection: count readback failed");
-        return -1;
-    }
-    return h;
 }
 
 extern "C" void run_detection(float dthreshold, float thresh1, int ext_minarea,
@@ -338,8 +334,8 @@ extern "C" void run_detection(float dthreshold, float thresh1, int ext_minarea,
     int *cnt_d = sxg_take<int>("det.counts", 8);
     if (!rootpos || !cnt_d) return;
     const float *td = pd ? &pd->dthresh : nullptr;
-    int *nfg_d = pd ? &pd->nfg : cnt_d, *nraw_d = pd ? &pd->nraw : cnt_d;
-    int *npix_d = pd ? &pd->npix : cnt_d;
+    int *nfg_d = pd ? &pd->nfg : cnt_d, *nraw_d = pd ? &pd->nraw : cnt_d + 1;
+    int *npix_d = pd ? &pd->npix : cnt_d + 2;
     /* the device counts the kernels read (planned runs) */
     const int *nfg_k = pd ? nfg_d : nullptr, *nraw_k = pd ? nraw_d : nullptr;
     const int *npix_k = pd ? npix_d : nullptr;
@@ -367,8 +363,7 @@ extern "C" void run_detection(float dthreshold, float thresh1, int ext_minarea,
         nfg = (int)S.plan->cap[PL_NFG];
         sxg_plan_guard(nfg_d, nfg, PL_NFG);
     } else {
-        nfg = read_count(cnt_d, st);
-        if (nfg < 0) return;
+        if (!sxg_read_back({{nfg_d, &nfg, 1}})) return;
     }
     S.npix_above = nfg;
     const int gfg = sxg_div_up(nfg > 0 ? nfg : 1, 256);
@@ -402,41 +397,34 @@ extern "C" void run_detection(float dthreshold, float thresh1, int ext_minarea,
                            ext_minarea, keep, nfg_k);
     }
     sxg_compact_nonneg(keep, rawpos, nfg, nraw_d, st, nfg_k);
-    int nraw;
+    /* pixel keys, kept pixels: sized by nfg, so that the host waits once for both counts */
+    int *k0 = sxg_take<int>("det.k0", nfg), *v0 = sxg_take<int>("det.v0", nfg);
+    int *k1 = sxg_take<int>("det.k1", nfg), *v1 = sxg_take<int>("det.v1", nfg);
+    int *hist = sxg_take<int>("det.hist", 256 * (size_t)(sxg_div_up(nfg + 1, 4096) + 1) + 64);
+    int *idx = v1;   /* indices of kept pixels in the foreground list, until the sort */
+    if (!k0 || !v0 || !k1 || !v1 || !hist) return;
+    if (nfg > 0) {
+        hipLaunchKernelGGL(k_det_rawid, dim3(gfg), dim3(256), 0, st, rawpos, nraw_d,
+                           rawid_of_pos);
+        hipLaunchKernelGGL(k_det_pixkey, dim3(gfg), dim3(256), 0, st, rk, nfg, rawid_of_pos,
+                           keep, nfg_k);
+    }
+    sxg_compact_nonneg(keep, idx, nfg, npix_d, st, nfg_k);
+    int nraw, npix;
     if (pd) {
         nraw = (int)S.plan->cap[PL_NRAW];
         sxg_plan_guard(nraw_d, nraw, PL_NRAW);
-    } else {
-        nraw = read_count(cnt_d, st);
-        if (nraw < 0) return;
+        npix = (int)S.plan->cap[PL_NPIX];
+        sxg_plan_guard(npix_d, npix, PL_NPIX);
+    } else if (!sxg_read_back({{nraw_d, &nraw, 1}, {npix_d, &npix, 1}})) {
+        return;
     }
     S.nraw = nraw;
     RawObj ro;
     if (!sxg_raw_alloc(nraw, ro)) return;
-    if (nfg > 0) {
-        if (nraw > 0)
-            hipLaunchKernelGGL(k_det_rawinfo, dim3(sxg_div_up(nraw, 256)), dim3(256), 0, st, rawpos,
-                               nraw, fg, W, rs, rawid_of_pos, ro, dthreshold,
-                               (int)(wa.w && wa.rel),
-                               nraw_k, td);
-        /* pixel keys, kept pixels, stable sort by object */
-        hipLaunchKernelGGL(k_det_pixkey, dim3(gfg), dim3(256), 0, st, rk, nfg, rawid_of_pos,
-                           keep, nfg_k);
-    }
-    int *idx = rawpos;   /* reuse: indices of kept pixels in the foreground list */
-    int *k0 = sxg_take<int>("det.k0", nfg), *v0 = sxg_take<int>("det.v0", nfg);
-    int *k1 = sxg_take<int>("det.k1", nfg), *v1 = sxg_take<int>("det.v1", nfg);
-    int *hist = sxg_take<int>("det.hist", 256 * (size_t)(sxg_div_up(nfg + 1, 4096) + 1) + 64);
-    if (!k0 || !v0 || !k1 || !v1 || !hist) return;
-    sxg_compact_nonneg(keep, idx, nfg, npix_d, st, nfg_k);
-    int npix;
-    if (pd) {
-        npix = (int)S.plan->cap[PL_NPIX];
-        sxg_plan_guard(npix_d, npix, PL_NPIX);
-    } else {
-        npix = read_count(cnt_d, st);
-        if (npix < 0) return;
-    }
+    if (nraw > 0)
+        hipLaunchKernelGGL(k_det_rawinfo, dim3(sxg_div_up(nraw, 256)), dim3(256), 0, st, rawpos,
+                           nraw, fg, W, rs, ro, dthreshold, (int)(wa.w && wa.rel), nraw_k, td);
     S.npix_raw = npix;
     if (!pd) {
         S.seen.cap[PL_NFG] = nfg;

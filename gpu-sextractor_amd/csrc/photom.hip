@@ -712,7 +712,6 @@ extern "C" void endobject_gpu(void *prefs, void *brain, void *flagobj2, void *ob
     if (!vsum) return;
     hipLaunchKernelGGL(k_phot_sum, dim3(1), dim3(1024), 0, S.stream,
                        sxg_take<int>("phot.npix", (size_t)numobj), numobj, vsum);
-    SXG_HIP(hipMemcpyAsync(&visited, vsum, sizeof(visited), hipMemcpyDeviceToHost, S.stream));
     if (objlist) {
         PhotArgs A;
         A.nobj = numobj;
@@ -727,7 +726,7 @@ extern "C" void endobject_gpu(void *prefs, void *brain, void *flagobj2, void *ob
                                hipMemcpyDeviceToHost, S.stream));
     }
     SXG_HIP(hipGetLastError());
-    SXG_HIP(hipStreamSynchronize(S.stream));
+    if (!sxg_read_back({{vsum, &visited, 2}}, true)) return;
     S.phot_pixels = (int64_t)visited;
     S.phot_ready = true;
 }

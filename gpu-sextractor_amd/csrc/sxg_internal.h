@@ -8,6 +8,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <initializer_list>
 #include <map>
 #include <string>
 
@@ -239,6 +240,9 @@ struct SxgState {
     int *opix = nullptr;      /* int[P0]: raw pixels grouped by object, raster order inside */
     int *objoff = nullptr;    /* int[nobj + 1]: start of each object in opix */
     int nsurv = 0;
+    /* the survivors' ranks in "out.keep", "out.rank", "out.total" are those of the last
+       CLEAN; their number is in nsurv */
+    bool ranked = false, counted = false;
     bool cleaned = false;
     bool clean_enabled = true;
     float deb_base = 0.0f;
@@ -262,6 +266,9 @@ struct SxgState {
     int rw = 0, rh = 0;
     bool is_default = false;               /* the process-wide default context */
     bool single_stream = false;            /* no side streams (batch workers) */
+    unsigned *mail = nullptr;              /* pinned page of sxg_read_back: [0] the sequence
+                                              number, [16..] the words */
+    unsigned mail_seq = 0;
     /* MAP_WEIGHT map (sxg_set_weight) */
     DevBuf weight;
     int ww = 0, wh = 0;
@@ -309,9 +316,21 @@ SxgState *sxg_bound_state();
 void sxg_bind_state(SxgState *s);
 /* End of an entry point without a host output: the contexts of the batch workers
    (several sharing the device) wait for their stream there, which interleaves their
-   kernels on the hardware queues; the default context returns at once and keeps its
+   kernels on the hardware queues; every other context returns at once and keeps its
    queue full. */
 bool sxg_stage_wait();
+/* The host's copy of a few device words that the work queued on the context's stream
+   leaves behind (at most SXG_MAIL_WORDS together): a kernel writes them into the
+   context's page of pinned host memory and then their sequence number, which the host
+   polls for; drain: the host also waits for the stream to run dry, for entry points that
+   hand device memory to the caller.  Never in a planned run. */
+constexpr int SXG_MAIL_WORDS = 48;
+struct SxgRead {
+    const void *src;   /* device, 4-byte aligned */
+    void *dst;
+    int words;
+};
+bool sxg_read_back(std::initializer_list<SxgRead> what, bool drain = false);
 void sxg_stage_begin(StageId s);
 void sxg_stage_end(StageId s);
 

@@ -3,6 +3,7 @@
  * primitives, and the frame entry points init_device / clear_device (the reference's
  * src/cuda/cudainit.cu:16 and :160).
  */
+#include <chrono>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -205,8 +206,73 @@ extern "C" int sxg_stage_times(float *ms, int n)
 bool sxg_stage_wait()
 {
     SxgState &S = sxg_state();
-    if (S.is_default || S.plan) return true;
+    if (!S.single_stream || S.plan) return true;
     SXG_HIP_RET(hipStreamSynchronize(S.stream), false);
+    return true;
+}
+
+struct MailArgs {
+    const unsigned *src[SXG_MAIL_WORDS];   /* one word each */
+};
+
+__global__ void __launch_bounds__(64) k_mail(MailArgs a, int n, unsigned *mail, unsigned seq)
+{
+    const int i = threadIdx.x;
+    if (i < n) mail[16 + i] = *a.src[i];
+    __threadfence_system();   /* one wavefront: every lane's word before the number */
+    if (i == 0) __hip_atomic_store(mail, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+/* A copy of the words by the runtime and a wait for the stream left the GPU idle for 25 to
+   40 us at each count (the copy's own kernel, its signal, the host's wake-up, the next
+   launch); the words pushed by a kernel and seen by a polling host cost about 10. */
+bool sxg_read_back(std::initializer_list<SxgRead> what, bool drain)
+{
+    SxgState &S = sxg_state();
+    if (!S.mail) {
+        void *p = nullptr;
+        SXG_HIP_RET(hipHostMalloc(&p, 4096, hipHostMallocMapped | hipHostMallocCoherent), false);
+        memset(p, 0, 4096);
+        S.mail = static_cast<unsigned *>(p);
+    }
+    MailArgs a{};
+    int n = 0;
+    for (const SxgRead &r : what)
+        for (int w = 0; w < r.words; w++) {
+            if (n == SXG_MAIL_WORDS) {
+                sxg_set_error("sxg_read_back: too many words (internal error)");
+                return false;
+            }
+            a.src[n++] = static_cast<const unsigned *>(r.src) + w;
+        }
+    void *dev = nullptr;
+    SXG_HIP_RET(hipHostGetDevicePointer(&dev, S.mail, 0), false);
+    const unsigned seq = ++S.mail_seq;
+    hipLaunchKernelGGL(k_mail, dim3(1), dim3(64), 0, S.stream, a, n,
+                       static_cast<unsigned *>(dev), seq);
+    SXG_HIP_RET(hipGetLastError(), false);
+    auto seen = [&] { return __atomic_load_n(S.mail, __ATOMIC_ACQUIRE) == seq; };
+    /* polled for at most 2 ms: after that, and where the stream has failed, the runtime's
+       own wait decides */
+    bool got = false;
+    if (!drain) {
+        const auto t0 = std::chrono::steady_clock::now();
+        do {
+            for (int k = 0; k < 64 && !(got = seen()); k++) __builtin_ia32_pause();
+        } while (!got && std::chrono::steady_clock::now() - t0 < std::chrono::milliseconds(2));
+    }
+    if (!got) {
+        SXG_HIP_RET(hipStreamSynchronize(S.stream), false);
+        if (!seen()) {
+            sxg_set_error("sxg_read_back: the counts did not arrive");
+            return false;
+        }
+    }
+    n = 16;
+    for (const SxgRead &r : what) {
+        memcpy(r.dst, S.mail + n, sizeof(unsigned) * r.words);
+        n += r.words;
+    }
     return true;
 }
 
@@ -218,6 +284,9 @@ extern "C" void sxg_release(void)
                       &S.comps, &S.objs, &S.rootobj};
     for (DevBuf *b : bufs) b->release();
     sxg_release_named();
+    S.ranked = S.counted = false;
+    if (S.mail) (void)hipHostFree(S.mail);
+    S.mail = nullptr;
     S.dmask.release();
     S.mask_k = 0;
     S.back_W = S.back_H = 0;
