@@ -77,7 +77,8 @@ __device__ __forceinline__ void cv_load(float (*tile)[CV_TX + K], const float *_
     constexpr int NS = (K - 1) * LH;                     /* right-strip pixels */
     constexpr int NSU = (NS + CV_THREADS - 1) / CV_THREADS;
     constexpr bool SPL = MODE == TS_SPLINE;
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    /* the wavefront's number in a scalar register: rows and their addresses with it */
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nbx = sp.nbx;
     /* the lane's column of the main part and its spline segment */
     const int gxm = X0 + lane - HW;
@@ -169,6 +170,57 @@ __device__ __forceinline__ void cv_load(float (*tile)[CV_TX + K], const float *_
     }
 }
 
+/* The CV_R outputs of a lane, column tx of the tile's rows r0 .. r0 + CV_R - 1: each a sum
+   over the mask in raster order.  Mask row by mask row, with the CV_R tile rows that it
+   meets in registers: a step needs one mask row in scalar registers (the next one on its
+   way) and one new tile row, which takes the place of the one that has left.  Bound by its
+   arithmetic for the large masks: 2 K K multiplies and adds a pixel (the reference rounds
+   both, so no fused ones), 207 us at 8192 x 4096 and K = 11.  Tile row by tile row, with
+   the whole mask in scalars, k_subconv_det took 558 us there (weighted) and 86 us at
+   4096 x 4096, K = 7; mask row by mask row, 326 and 74. */
+template <int K>
+__device__ __forceinline__ void cv_taps(const float (*tile)[CV_TX + K], int r0, int tx,
+                                        const float *__restrict__ mask, float (&acc)[CV_R])
+{
+    float v[CV_R][K], m[2][K];
+    /* zeros that the compiler does not see through, new in each step: without them it
+       collects every load at the top, where they do not fit its registers (for K = 11 it
+       then moved 660 scalars to vector lanes and back) */
+    int mo = 0, to = 0;
+    asm volatile("" : "+s"(mo), "+v"(to));
+#pragma unroll
+    for (int j = 0; j < K; j++) m[0][j] = mask[mo + j];
+#pragma unroll
+    for (int r = 0; r < CV_R; r++) {
+        acc[r] = 0.0f;
+#pragma unroll
+        for (int j = 0; j < K; j++) v[r][j] = tile[r0 + r][tx + j];
+    }
+#pragma unroll
+    for (int i = 0; i < K; i++) {
+        if (i + 1 < K) {
+            asm volatile("" : "+s"(mo), "+v"(to));
+#pragma unroll
+            for (int j = 0; j < K; j++) m[(i + 1) & 1][j] = mask[mo + (i + 1) * K + j];
+        }
+#pragma unroll
+        for (int j = 0; j < K; j++) {
+#pragma unroll
+            for (int r = 0; r < CV_R; r++) {
+                const float prod = m[i & 1][j] * v[(i + r) % CV_R][j];
+                acc[r] = acc[r] + prod;
+            }
+        }
+        if (i + 1 < K) {
+#pragma unroll
+            for (int j = 0; j < K; j++) v[i % CV_R][j] = tile[r0 + i + CV_R][tx + j + to];
+        }
+        /* the sums stay here, and are not moved to where they are used */
+#pragma unroll
+        for (int r = 0; r < CV_R; r++) asm volatile("" : "+v"(acc[r]));
+    }
+}
+
 template <int K>
 __global__ void __launch_bounds__(CV_THREADS) k_convolve(const float *__restrict__ in,
                                                          float *__restrict__ out, int W, int H,
@@ -181,28 +233,10 @@ __global__ void __launch_bounds__(CV_THREADS) k_convolve(const float *__restrict
     cv_tile(X0, Y0);
     cv_load<K, TS_COPY>(tile, in, SplineArgs{}, W, H, X0, Y0);
     __syncthreads();
-    const int tx = threadIdx.x % CV_TX, ty = threadIdx.x / CV_TX;
-    const int r0 = ty * CV_R;
+    const int tx = threadIdx.x % CV_TX;
+    const int r0 = __builtin_amdgcn_readfirstlane(threadIdx.x / CV_TX) * CV_R;
     float acc[CV_R];
-#pragma unroll
-    for (int r = 0; r < CV_R; r++) acc[r] = 0.0f;
-#pragma unroll
-    for (int t = 0; t < CV_R + K - 1; t++) {
-        float v[K];
-#pragma unroll
-        for (int j = 0; j < K; j++) v[j] = tile[r0 + t][tx + j];
-#pragma unroll
-        for (int r = 0; r < CV_R; r++) {
-            const int i = t - r;
-            if (i >= 0 && i < K) {
-#pragma unroll
-                for (int j = 0; j < K; j++) {
-                    float prod = mask[i * K + j] * v[j];
-                    acc[r] = acc[r] + prod;
-                }
-            }
-        }
-    }
+    cv_taps<K>(tile, r0, tx, mask, acc);
     const int x = X0 + tx;
     if (x < W) {
 #pragma unroll
@@ -346,28 +380,10 @@ __global__ void __launch_bounds__(CV_THREADS) k_subconv_det(const float *__restr
     if (sp.nbx > 1) cv_load<K, TS_SPLINE>(tile, src, sp, W, H, X0, Y0);
     else cv_load<K, TS_NODE0>(tile, src, sp, W, H, X0, Y0);
     __syncthreads();
-    const int tx = threadIdx.x % CV_TX, ty = threadIdx.x / CV_TX;
-    const int r0 = ty * CV_R;
+    const int tx = threadIdx.x % CV_TX;
+    const int r0 = __builtin_amdgcn_readfirstlane(threadIdx.x / CV_TX) * CV_R;
     float acc[CV_R];
-#pragma unroll
-    for (int r = 0; r < CV_R; r++) acc[r] = 0.0f;
-#pragma unroll
-    for (int tt = 0; tt < CV_R + K - 1; tt++) {
-        float v[K];
-#pragma unroll
-        for (int j = 0; j < K; j++) v[j] = tile[r0 + tt][tx + j];
-#pragma unroll
-        for (int r = 0; r < CV_R; r++) {
-            const int i = tt - r;
-            if (i >= 0 && i < K) {
-#pragma unroll
-                for (int j = 0; j < K; j++) {
-                    float prod = mask[i * K + j] * v[j];
-                    acc[r] = acc[r] + prod;
-                }
-            }
-        }
-    }
+    cv_taps<K>(tile, r0, tx, mask, acc);
     const int x = X0 + tx, lane = tx;   /* X0 is a multiple of 64: lane = x mod 64 */
     const unsigned long long below = ~0ull >> (63 - lane);
 #pragma unroll
