@@ -20,13 +20,15 @@
  * computes in float: sqrt and log10 of a float are the float functions there).  The
  * transcendental functions are the canonical ones of sx_cmath.h.
  *
- * Layout: one 64-lane wavefront per object, objects with a large bounding box first.
- * The aperture boxes are walked in raster order 64 pixels at a time: the lanes compute
- * the per-pixel terms (oversampled area, masking and mirror, PHOTO-mode exponential), and
- * the sums are transposed ordered folds (sxg_wave.h), so every sum is the reference's
- * sequential raster-order sum bit for bit.  Counts are ballots.  The network runs one
- * neuron per lane.
+ * Layout: a 64-lane wavefront per object, a workgroup of four for the objects of the
+ * largest boxes, which come first.  The aperture boxes are walked in raster order 64 or 256
+ * pixels at a time, the next ones' values and labels on their way: the lanes compute the
+ * per-pixel terms (oversampled area, masking and mirror, PHOTO-mode exponential), and the
+ * sums are ordered folds, a row of 16 lanes to each (sxg_wave.h), so every sum is the
+ * reference's sequential raster-order sum bit for bit.  The network runs one neuron per
+ * lane.
  */
+#include <algorithm>
 #include <climits>
 #include <cstring>
 
@@ -39,7 +41,15 @@
 #define PH_OVERSAMP 5                 /* APER_OVERSAMP, src/define.h:172 */
 #define PH_KRON_NSIG (3 * 2.0)        /* KRON_NSIG = 3*MARGIN_SCALE, src/define.h:173 */
 #define PH_CROWD 0.1                  /* CROWD_THRESHOLD, src/define.h:177 */
-#define PH_BIG_BOX 256                /* objects with a larger bounding box go first */
+/* pixels of the first AUTO box from which an object takes a workgroup, and from which it goes
+   before the small ones.  k_endobject, 2048 x 2048 with about 5,000 objects: 189 us with one
+   wavefront an object and one lane a sum, 101 with a row of lanes a sum, then with PH_BIG
+   4096, 2048 and 1024: 69, 62 and 65 */
+#define PH_BIG 2048
+#define PH_MID 512
+/* workgroups for them at the most (further large ones take a wavefront): the grid is as much
+   larger, whatever the frame holds */
+#define PH_GROUPS 512
 
 struct PhotCols {
     float *flux_iso, *fluxerr_iso, *mag_iso, *magerr_iso, *flux_isocor, *fluxerr_isocor,
@@ -50,7 +60,7 @@ struct PhotCols {
 struct PhotArgs {
     const float *sub;          /* background-subtracted frame */
     const int *lab;            /* photometry labels */
-    const int *order;          /* objects in launch order */
+    const int *order, *cnt;    /* objects in launch order (k_phot_order) */
     int W, H, nobj;
     ObjCols o;
     PhotCols p;
@@ -96,25 +106,13 @@ __global__ void __launch_bounds__(256) k_phot_lab_scatter(const int *__restrict_
     lab[p] = (t > 0 && master[t] != 0xffffffffu) ? INT_MAX : t;
 }
 
-__global__ void __launch_bounds__(256) k_phot_order(ObjCols o, int nobj, int *cnt, int *order)
-{
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= nobj) return;
-    const long box = (long)(o.xmax[i] - o.xmin[i] + 1) * (o.ymax[i] - o.ymin[i] + 1);
-    if (box >= PH_BIG_BOX)
-        order[atomicAdd(&cnt[0], 1)] = i;
-    else
-        order[nobj - 1 - atomicAdd(&cnt[1], 1)] = i;
-}
-
 /* ---------------------------------------------------------------- per object ---- */
 /* the value used for pixel (x, y) of object obj's aperture: its own, or, when the pixel
    belongs to another object, the mirror pixel through the centroid if that one is free
    or the object's own (MASK_TYPE CORRECT), else 0 (cudaanalyse.cu:222-243, :523-545) */
 __device__ inline double ph_value(const PhotArgs &A, int obj, double mx, double my, int x,
-                                  int y, double pix, bool &masked)
+                                  int y, double pix, int t, bool &masked)
 {
-    int t = A.lab[(long)y * A.W + x];
     masked = t >= 0 && t != obj;
     if (!masked) return pix;
     int x2, y2;
@@ -154,21 +152,103 @@ __device__ inline void ph_ellipse(const PhotArgs &A, int obj, bool use_ellipse, 
     }
 }
 
-__global__ void __launch_bounds__(256) k_endobject(PhotArgs A)
+/* the pixels of a box in raster order, one of every STEP to a thread: its value and label,
+   read one step ahead (the box lies inside the frame) */
+template <int STEP> struct PhBox {
+    const PhotArgs &A;
+    int bw, x0, y0, nb, k, dx, dy, x, y;   /* x, y: pixel k in the box */
+    float pix_next = 0.0f;
+    int lab_next = -1;
+    __device__ PhBox(const PhotArgs &a, int first, int xmin, int xmax, int ymin, int ymax)
+        : A(a), bw(xmax - xmin), x0(xmin), y0(ymin), k(first)
+    {
+        const int bh = ymax - ymin;
+        nb = bw > 0 && bh > 0 ? bw * bh : 0;
+        if (!nb) return;
+        dy = STEP / bw;
+        dx = STEP - dy * bw;
+        y = first / bw;
+        x = first - y * bw;
+        load();
+    }
+    __device__ void load()
+    {
+        if (k >= nb) return;
+        const long p = (long)(y0 + y) * A.W + x0 + x;
+        pix_next = A.sub[p];
+        lab_next = A.lab[p];
+    }
+    /* the pixel of this step; false: past the box */
+    __device__ bool next(int &px, int &py, float &pix, int &lab)
+    {
+        const bool in = k < nb;
+        px = x0 + x;
+        py = y0 + y;
+        pix = pix_next;
+        lab = lab_next;
+        k += STEP;
+        x += dx;
+        y += dy;
+        if (x >= bw) {
+            x -= bw;
+            y++;
+        }
+        load();
+        return in;
+    }
+};
+
+/* the box of the first AUTO pass, which most of an object's time goes with */
+__device__ inline void ph_auto_box(const PhotArgs &A, int obj, float &cx2, float &cy2,
+                                   float &cxy, float &klim2, int &flag, int &xmin, int &xmax,
+                                   int &ymin, int &ymax)
 {
-    __shared__ double s_rows[4][3 * SXW_ROW];
-    const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int gw = blockIdx.x * 4 + wid;
-    if (gw >= A.nobj) return;            /* whole wavefronts only: no workgroup barrier */
-    const int obj = A.order[gw];
-    double *rows = s_rows[wid];
+    float dxlim, dylim;
+    const bool ell = PH_KRON_NSIG * sqrtf(A.o.a[obj] * A.o.b[obj]) > A.autoaper0 / 2.0;
+    ph_ellipse(A, obj, ell, A.autoaper0, cx2, cy2, cxy, dxlim, dylim);
+    if (ell) {
+        dxlim = dxlim > 0.0 ? (float)(PH_KRON_NSIG / sqrtf(dxlim)) : 0.0f;
+        dylim = dylim > 0.0 ? (float)(PH_KRON_NSIG / sqrtf(dylim)) : 0.0f;
+        klim2 = (float)(PH_KRON_NSIG * PH_KRON_NSIG);
+    } else {
+        klim2 = dxlim * dxlim;
+    }
+    ph_box(A.o.mx[obj], A.o.my[obj], dxlim, dylim, A.W, A.H, flag, xmin, xmax, ymin, ymax);
+}
+
+/* the objects in launch order: those of the large boxes at the front of order, the small
+   ones from its end, the others in order[nobj ..]; cnt: large, others, small */
+__global__ void __launch_bounds__(256) k_phot_order(PhotArgs A, int *cnt, int *order)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x, n = A.nobj;
+    long nb = 0;
+    if (i < n) {
+        float cx2, cy2, cxy, klim2;
+        int flag = 0, xmin, xmax, ymin, ymax;
+        ph_auto_box(A, i, cx2, cy2, cxy, klim2, flag, xmin, xmax, ymin, ymax);
+        nb = (long)max(xmax - xmin, 0) * max(ymax - ymin, 0);
+    }
+    const bool big = i < n && nb >= PH_BIG, mid = i < n && !big && nb >= PH_MID;
+    const bool small = i < n && nb < PH_MID;
+    const int kb = sxw_place(&cnt[0], big), km = sxw_place(&cnt[1], mid);
+    const int ks = sxw_place(&cnt[2], small);
+    if (big) order[kb] = i;
+    if (mid) order[n + km] = i;
+    if (small) order[n - 1 - ks] = i;
+}
+
+template <SxwSize Z> __device__ void phot_object(const PhotArgs &A, int obj, double *rows)
+{
+    using T = SxwTeam<Z>;
+    const int lane = threadIdx.x & 63;
+    const float none[1] = {};
     const ObjCols &o = A.o;
     const int W = A.W, H = A.H;
     const double mx = o.mx[obj], my = o.my[obj];
     const float a = o.a[obj], b = o.b[obj];
     int flag = o.flag[obj];
     double var = A.backsig * A.backsig;   /* float product, as the reference forms it */
-    int visited = 0;                      /* aperture pixels summed (wave-uniform) */
+    int visited = 0;                      /* aperture pixels summed by this thread */
 
     /* ---- APER (cudaanalyse.cu:104-287) */
     float flux_aper = 0.0f, fluxerr_aper = 0.0f, mag_aper = 0.0f, magerr_aper = 0.0f;
@@ -187,15 +267,14 @@ __global__ void __launch_bounds__(256) k_endobject(PhotArgs A)
         if (xmax > W) { xmax = W; flag |= PH_APERT_PB; }
         if (ymin < 0) { ymin = 0; flag |= PH_APERT_PB; }
         if (ymax > H) { ymax = H; flag |= PH_APERT_PB; }
-        const int bw = xmax - xmin, bh = ymax - ymin;
-        const int nb = (bw > 0 && bh > 0) ? bw * bh : 0;
-        double acc = 0.0;   /* lane 0: area, 1: tv, 2: sigtv */
-        for (int k0 = 0; k0 < nb; k0 += 64) {
-            const int k = k0 + lane;
+        PhBox<T::STEP> box(A, T::first(), xmin, xmax, ymin, ymax);
+        SxwSums<3, 0, Z> S;   /* area, tv, sigtv */
+        for (int k0 = 0; k0 < box.nb; k0 += T::STEP) {
             bool member = false;
             double t[3] = {0.0, 0.0, 0.0};
-            if (k < nb) {
-                const int y = ymin + k / bw, x = xmin + k % bw;
+            int x, y, lab;
+            float own;
+            if (box.next(x, y, own, lab)) {
                 float dx = (float)(x - mx), dy = (float)(y - my);
                 const float r2 = dx * dx + dy * dy;
                 if (r2 < rextlim2) {
@@ -215,8 +294,7 @@ __global__ void __launch_bounds__(256) k_endobject(PhotArgs A)
                         locarea = 1.0f;
                     }
                     bool masked;
-                    double pix = ph_value(A, obj, mx, my, x, y, (double)A.sub[(long)y * W + x],
-                                          masked);
+                    double pix = ph_value(A, obj, mx, my, x, y, (double)own, lab, masked);
                     double sig;
                     if (A.photo) {
                         pix = sx_exp(pix / A.ngamma);
@@ -229,11 +307,12 @@ __global__ void __launch_bounds__(256) k_endobject(PhotArgs A)
                     t[2] = sig;
                 }
             }
-            visited += __popcll(__ballot(member));
-            sxw_fold<3, double>(rows, t, member, acc);
+            visited += member;
+            S.add(rows, t, none, member);
         }
-        const double area = sxw_rl(acc, 0);
-        double tv = sxw_rl(acc, 1), sigtv = sxw_rl(acc, 2);
+        S.end(rows);
+        const double area = S.d[0];
+        double tv = S.d[1], sigtv = S.d[2];
         if (A.photo) {
             tv = A.ngamma * (tv - area * sx_exp(0.0 / A.ngamma));   /* dbkg = 0 (:2244) */
             sigtv /= A.ngamma * A.ngamma;
@@ -252,46 +331,35 @@ __global__ void __launch_bounds__(256) k_endobject(PhotArgs A)
     if (A.do_auto) {
         float cx2, cy2, cxy, klim2, dxlim, dylim;
         int xmin, xmax, ymin, ymax;
-        const bool ell1 = PH_KRON_NSIG * sqrtf(a * b) > A.autoaper0 / 2.0;
-        ph_ellipse(A, obj, ell1, A.autoaper0, cx2, cy2, cxy, dxlim, dylim);
-        if (ell1) {
-            dxlim = dxlim > 0.0 ? (float)(PH_KRON_NSIG / sqrtf(dxlim)) : 0.0f;
-            dylim = dylim > 0.0 ? (float)(PH_KRON_NSIG / sqrtf(dylim)) : 0.0f;
-            klim2 = (float)(PH_KRON_NSIG * PH_KRON_NSIG);
-        } else {
-            klim2 = dxlim * dxlim;
-        }
-        ph_box(mx, my, dxlim, dylim, W, H, flag, xmin, xmax, ymin, ymax);
-        int bw = xmax - xmin, bh = ymax - ymin;
-        int nb = (bw > 0 && bh > 0) ? bw * bh : 0;
+        ph_auto_box(A, obj, cx2, cy2, cxy, klim2, flag, xmin, xmax, ymin, ymax);
         int area = 0, areab = 0;
-        double acc = 0.0;   /* lane 0: r1, 1: v1 */
-        for (int k0 = 0; k0 < nb; k0 += 64) {
-            const int k = k0 + lane;
-            bool inside = false, good = false;
+        PhBox<T::STEP> box(A, T::first(), xmin, xmax, ymin, ymax);
+        SxwSums<2, 0, Z> R;   /* r1, v1 */
+        for (int k0 = 0; k0 < box.nb; k0 += T::STEP) {
+            bool good = false;
             double t[2] = {0.0, 0.0};
-            if (k < nb) {
-                const int y = ymin + k / bw, x = xmin + k % bw;
+            int x, y, tl;
+            float pix;
+            if (box.next(x, y, pix, tl)) {
                 const float dx = (float)(x - mx), dy = (float)(y - my);
                 const float r2 = cx2 * dx * dx + cy2 * dy * dy + cxy * dx * dy;
                 if (r2 <= klim2) {
-                    inside = true;
-                    const float pix = A.sub[(long)y * W + x];
-                    const int tl = A.lab[(long)y * W + x];
                     good = (tl == obj || tl == -1) && pix > -SXG_BIG;
+                    visited++;
+                    area += good;
+                    areab += !good;
                     if (good) {
                         t[0] = sqrtf(r2) * pix;
                         t[1] = pix;
                     }
                 }
             }
-            const unsigned long long bi = __ballot(inside), bg = __ballot(good);
-            area += __popcll(bg);
-            areab += __popcll(bi & ~bg);
-            visited += __popcll(bi);
-            sxw_fold<2, double>(rows, t, good, acc);
+            R.add(rows, t, none, good);
         }
-        const double r1 = sxw_rl(acc, 0), v1 = sxw_rl(acc, 1);
+        R.end(rows);
+        area = T::sum(area);
+        areab = T::sum(areab);
+        const double r1 = R.d[0], v1 = R.d[1];
         area += areab;
         double tv = 0.0, sigtv = 0.0;
         if (area) {
@@ -313,22 +381,20 @@ __global__ void __launch_bounds__(256) k_endobject(PhotArgs A)
                 kf = 0.0f;
             }
             ph_box(mx, my, dxlim, dylim, W, H, flag, xmin, xmax, ymin, ymax);
-            bw = xmax - xmin;
-            bh = ymax - ymin;
-            nb = (bw > 0 && bh > 0) ? bw * bh : 0;
             area = areab = 0;
-            acc = 0.0;      /* lane 0: tv, 1: sigtv */
-            for (int k0 = 0; k0 < nb; k0 += 64) {
-                const int k = k0 + lane;
+            PhBox<T::STEP> kbox(A, T::first(), xmin, xmax, ymin, ymax);
+            SxwSums<2, 0, Z> K;   /* tv, sigtv */
+            for (int k0 = 0; k0 < kbox.nb; k0 += T::STEP) {
                 bool inside = false, masked = false;
                 double t[2] = {0.0, 0.0};
-                if (k < nb) {
-                    const int y = ymin + k / bw, x = xmin + k % bw;
+                int x, y, lab;
+                float own;
+                if (kbox.next(x, y, own, lab)) {
                     const float dx = (float)(x - mx), dy = (float)(y - my);
                     if (cx2 * dx * dx + cy2 * dy * dy + cxy * dx * dy <= klim2) {
                         inside = true;
-                        float pix = (float)ph_value(A, obj, mx, my, x, y,
-                                                    (double)A.sub[(long)y * W + x], masked);
+                        float pix =
+                            (float)ph_value(A, obj, mx, my, x, y, (double)own, lab, masked);
                         double sig;
                         if (A.photo) {
                             pix = (float)sx_exp(pix / A.ngamma);
@@ -340,14 +406,16 @@ __global__ void __launch_bounds__(256) k_endobject(PhotArgs A)
                         t[1] = sig;
                     }
                 }
-                const unsigned long long bi = __ballot(inside), bm = __ballot(inside && masked);
-                area += __popcll(bi);
-                areab += __popcll(bm);
-                visited += __popcll(bi);
-                sxw_fold<2, double>(rows, t, inside, acc);
+                area += inside;
+                areab += inside && masked;
+                K.add(rows, t, none, inside);
             }
-            tv = sxw_rl(acc, 0);
-            sigtv = sxw_rl(acc, 1);
+            K.end(rows);
+            visited += area;
+            area = T::sum(area);
+            areab = T::sum(areab);
+            tv = K.d[0];
+            sigtv = K.d[1];
             if ((float)areab > PH_CROWD * area) flag |= PH_CROWDED;
             if (A.photo) {
                 tv = A.ngamma * (tv - area * sx_exp(0.0 / A.ngamma));
@@ -398,7 +466,8 @@ __global__ void __launch_bounds__(256) k_endobject(PhotArgs A)
         sprob = (float)((sxw_rl(cur, 0) - br->outbias[0]) / br->outscale[0]);
     }
 
-    if (lane == 0) {
+    visited = T::sum(visited);
+    if (T::first() == 0) {
         const PhotCols &p = A.p;
         p.elong[obj] = a / b;
         p.ellip[obj] = 1 - b / a;
@@ -438,6 +507,24 @@ __global__ void __launch_bounds__(256) k_endobject(PhotArgs A)
         o.flag[obj] = flag;
         A.npix[obj] = visited;
     }
+}
+
+/* The workgroups of the large boxes first, then the others, a wavefront each.  Bound by the
+   ordered sums (two or three adds a pixel, which no two lanes share) and by how long the
+   largest box takes alone. */
+__global__ void __launch_bounds__(256) k_endobject(PhotArgs A)
+{
+    __shared__ double s_rows[std::max(sxw_brows(3, 0), 4 * sxw_wrows(3, 0))];
+    const int n = A.nobj, wid = threadIdx.x >> 6, nbig = min(A.cnt[0], PH_GROUPS);
+    if ((int)blockIdx.x < nbig) {
+        phot_object<SXW_GROUP>(A, A.order[blockIdx.x], s_rows);
+        return;
+    }
+    const int i = nbig + ((int)blockIdx.x - nbig) * 4 + wid;
+    if (i >= n) return;                  /* whole wavefronts only: no workgroup barrier */
+    const int mid = i - A.cnt[0];        /* place among the others, then the small ones */
+    const int at = mid < 0 ? i : mid < A.cnt[1] ? n + mid : i;
+    phot_object<SXW_WAVE>(A, A.order[at], s_rows + wid * sxw_wrows(3, 0));
 }
 
 /* the total of the per-object aperture pixel counts (one workgroup) */
@@ -623,7 +710,7 @@ static bool run_photometry(const sxg_photom_params &pp, const sxg_brain *brain, 
         return false;
     }
     int *lab = sxg_take<int>("phot.lab", S.N);
-    int *order = sxg_take<int>("phot.order", (size_t)n + 2);
+    int *order = sxg_take<int>("phot.order", 2 * (size_t)n + 3);
     A.npix = sxg_take<int>("phot.npix", (size_t)n);
     if (!lab || !order || !A.npix) return false;
     A.brain = nullptr;
@@ -646,12 +733,10 @@ static bool run_photometry(const sxg_photom_params &pp, const sxg_brain *brain, 
         hipLaunchKernelGGL(k_phot_lab_scatter, dim3(sxg_div_up((long)S.npix_raw, 256)),
                            dim3(256), 0, st, S.fpia, (long)S.npix_raw,
                            sxg_take<int>("deb.alloc", S.N), A.o.master, lab);
-    SXG_HIP_RET(hipMemsetAsync(order + n, 0, 2 * sizeof(int), st), false);
-    hipLaunchKernelGGL(k_phot_order, dim3(sxg_div_up(n, 256)), dim3(256), 0, st, A.o, n,
-                       order + n, order);
     A.sub = S.img.as<float>();
     A.lab = lab;
     A.order = order;
+    A.cnt = order + 2 * (size_t)n;
     A.backsig = backsig;
     A.thresh = thresh;
     A.apert = pp.apert;
@@ -670,7 +755,11 @@ static bool run_photometry(const sxg_photom_params &pp, const sxg_brain *brain, 
     A.do_aper = pp.do_aper;
     A.do_auto = pp.do_auto;
     A.do_class = pp.do_class;
-    hipLaunchKernelGGL(k_endobject, dim3(sxg_div_up(n, 4)), dim3(256), 0, st, A);
+    SXG_HIP_RET(hipMemsetAsync(order + 2 * (size_t)n, 0, 3 * sizeof(int), st), false);
+    hipLaunchKernelGGL(k_phot_order, dim3(sxg_div_up(n, 256)), dim3(256), 0, st, A,
+                       order + 2 * (size_t)n, order);
+    hipLaunchKernelGGL(k_endobject, dim3(sxg_div_up(n, 4) + std::min(n, PH_GROUPS)), dim3(256), 0,
+                       st, A);
     sxg_kt_end(SXG_KT_PHOT);
     SXG_HIP_RET(hipGetLastError(), false);
     return true;

@@ -256,6 +256,42 @@ __device__ inline void sxw_fold2(double *drows, float *frows, const double (&td)
 }
 
 /*
+ * The same for up to four double sums, a row of 16 lanes for each (sxw_row_fold): 4.3 cycles
+ * a member for all of them where the reads and adds above take 13.  The members' terms go to
+ * LDS compacted, padded with +0 to a multiple of 16 (an identity: a sum that starts at +0 is
+ * never -0).  acc: the row's sum in each of its lanes.
+ */
+#define SXW_WROW 80   /* row stride: two rows of lanes on all banks */
+template <int ND>
+__device__ inline void sxw_wfold(double *rows, const double (&t)[ND], bool member, double &acc)
+{
+    static_assert(ND <= 4, "a row of lanes for each sum");
+    const int lane = threadIdx.x & 63;
+    const unsigned long long b = __ballot(member);
+    const int cnt = __popcll(b), n16 = (cnt + 15) >> 4;
+    const int pos = __popcll(b & sxw_lanes_below(lane));
+    const bool pad = lane >= cnt && lane < 16 * n16;
+#pragma unroll
+    for (int s = 0; s < ND; s++) {
+        if (member) rows[s * SXW_WROW + pos] = t[s];
+        if (pad) rows[s * SXW_WROW + lane] = 0.0;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const double *p = rows + min(lane >> 4, ND - 1) * SXW_WROW + (lane & 15);
+    double x[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) x[c] = p[16 * c];
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+        if (c < n16) acc = sxw_row_fold(acc, x[c]);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+/*
  * The same over a workgroup of four wavefronts, for the objects whose sums are the longest:
  * 256 pixels a step, one per thread.  All four compute terms, then each adds three of the
  * sums, a row of 16 lanes each (sxw_row_fold), so the longest chain is 256 adds of 4.3
@@ -405,7 +441,10 @@ template <SxwSize Z> struct SxwTeam {
 
 /* the ordered sums of an object: ND double and NF float ones; rows: LDS, for a workgroup
    sxw_brows(ND, NF) doubles, for a wavefront its own sxw_wrows(ND, NF), none for a row */
-constexpr int sxw_wrows(int nd, int nf) { return nd * SXW_ROW + (nf * SXW_ROW + 1) / 2; }
+constexpr int sxw_wrows(int nd, int nf)
+{
+    return nf == 0 && nd <= 4 ? nd * SXW_WROW : nd * SXW_ROW + (nf * SXW_ROW + 1) / 2;
+}
 template <int ND, int NF, SxwSize Z> struct SxwSums {
     double d[ND];
     float f[NF + 1];
@@ -427,6 +466,8 @@ template <int ND, int NF, SxwSize Z> struct SxwSums {
             for (int s = 0; s < NF; s++) t[s] = tf[s];
             sxw_fold2<ND, NF>(rows, reinterpret_cast<float *>(rows + ND * SXW_ROW), td, t, member,
                               d[0], f[0]);
+        } else if constexpr (Z == SXW_WAVE && ND <= 4) {
+            sxw_wfold<ND>(rows, td, member, d[0]);
         } else if constexpr (Z == SXW_WAVE) {
             sxw_fold<ND, double>(rows, td, member, d[0]);
         } else {
@@ -444,7 +485,7 @@ template <int ND, int NF, SxwSize Z> struct SxwSums {
             const double a = d[0];
             const float b = f[0];
 #pragma unroll
-            for (int s = 0; s < ND; s++) d[s] = sxw_rl(a, s);
+            for (int s = 0; s < ND; s++) d[s] = sxw_rl(a, NF == 0 && ND <= 4 ? 16 * s : s);
 #pragma unroll
             for (int s = 0; s < NF; s++) f[s] = sxw_rl(b, ND + s);
         }
