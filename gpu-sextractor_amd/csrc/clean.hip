@@ -259,9 +259,11 @@ static bool survivor_ranks(const ObjCols &o, int *&keep, int *&rank, int *&tot)
     if (!keep || !rank || !tot) return false;
     if (S.ranked && !S.plan) return true;
     const int *nd = S.plan ? &S.pdev->nobj : nullptr;
-    hipLaunchKernelGGL(k_keepflag, dim3(sxg_div_up(S.nobj, 256)), dim3(256), 0, S.stream,
-                       o.master, S.nobj, keep, nd);
-    sxg_scan_excl(keep, rank, S.nobj, tot, S.stream, nd);
+    if (!sxg_scan_kept(o.master, keep, rank, S.nobj, tot, S.stream, nd)) {
+        hipLaunchKernelGGL(k_keepflag, dim3(sxg_div_up(S.nobj, 256)), dim3(256), 0, S.stream,
+                           o.master, S.nobj, keep, nd);
+        sxg_scan_excl(keep, rank, S.nobj, tot, S.stream, nd);
+    }
     S.ranked = !S.plan;
     return true;
 }

@@ -231,17 +231,33 @@ __global__ void __launch_bounds__(256) k_det_rootstat(const int *__restrict__ fg
     if (perpix) atomicMin(&rs.t0[rk], tv);
 }
 
-/* keep[k] = k for kept roots (size >= minarea), -1 otherwise; entry k is a root when its
-   root entry rk[k] is itself */
-__global__ void __launch_bounds__(256) k_det_rootflag(const int *__restrict__ rk, int nfg,
-                                                      const int *__restrict__ cnt, int minarea,
-                                                      int *keep, const int *nd)
-{
-    const int k = blockIdx.x * 256 + threadIdx.x;
-    if (k >= sxg_dn(nd, nfg)) return;
-    const int r = rk[k], c = cnt[k];
-    keep[k] = (r == k && c >= minarea) ? k : -1;
-}
+/* the roots of the components of minarea pixels or more, as raw objects in raster order of
+   their first pixels: entry k is a root when its root entry rk[k] is itself */
+struct PickRoots {
+    const int *rk, *cnt;
+    int minarea;
+    int *rawpos, *rawid_of_pos;
+    __device__ int read(int k) const { return rk[k]; }
+    __device__ int take(int k, int r) const { return r == k && cnt[k] >= minarea ? k : -1; }
+    __device__ void put(int i, int k, int) const
+    {
+        rawpos[i] = k;
+        rawid_of_pos[k] = i;
+    }
+};
+
+/* the pixels of the raw objects, with the object's number, in raster order */
+struct PickPixels {
+    const int *rk, *rawid_of_pos, *fg;
+    int *key, *pos;
+    __device__ int read(int k) const { return rk[k]; }
+    __device__ int take(int, int r) const { return rawid_of_pos[r]; }
+    __device__ void put(int i, int k, int id) const
+    {
+        key[i] = id;
+        pos[i] = fg[k];
+    }
+};
 
 __global__ void __launch_bounds__(256) k_det_rawinfo(const int *__restrict__ rawpos, int nraw,
                                                      const int *__restrict__ fg, int W,
@@ -262,37 +278,6 @@ __global__ void __launch_bounds__(256) k_det_rawinfo(const int *__restrict__ raw
     ro.t0[i] = perpix ? ord2f(rs.t0[k]) : t;
 }
 
-
-/* the raw object number at each kept component's root entry */
-__global__ void __launch_bounds__(256) k_det_rawid(const int *__restrict__ rawpos,
-                                                   const int *__restrict__ nraw,
-                                                   int *rawid_of_pos)
-{
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < *nraw) rawid_of_pos[rawpos[i]] = i;
-}
-
-/* object id of each detected pixel (or -1 when its component is too small) */
-__global__ void __launch_bounds__(256) k_det_pixkey(const int *__restrict__ rk, int nfg,
-                                                    const int *__restrict__ rawid_of_pos,
-                                                    int *key, const int *nd)
-{
-    const int k = blockIdx.x * 256 + threadIdx.x;
-    if (k >= sxg_dn(nd, nfg)) return;
-    key[k] = rawid_of_pos[rk[k]];
-}
-
-__global__ void __launch_bounds__(256) k_det_gather(const int *__restrict__ idx, int n,
-                                                    const int *__restrict__ key,
-                                                    const int *__restrict__ fg, int *k0, int *v0,
-                                                    const int *nd)
-{
-    const int j = blockIdx.x * 256 + threadIdx.x;
-    if (j >= sxg_dn(nd, n)) return;
-    const int k = idx[j];
-    k0[j] = key[k];
-    v0[j] = fg[k];
-}
 
 __global__ void __launch_bounds__(256) k_det_copy(const float *a, float *b, long n)
 {
@@ -374,11 +359,10 @@ extern "C" void run_detection(float dthreshold, float thresh1, int ext_minarea,
     rs.xmax = sxg_take<int>("det.xmax", nfg);
     rs.ymax = sxg_take<int>("det.ymax", nfg);
     rs.t0 = sxg_take<int>("det.t0", nfg);
-    int *keep = sxg_take<int>("det.keep", nfg);
     int *rawpos = sxg_take<int>("det.rawpos", nfg);
     int *rawid_of_pos = sxg_take<int>("det.rawid", nfg);
     int *rk = sxg_take<int>("det.rk", nfg);
-    if (!rs.cnt || !rs.peak || !rs.xmin || !rs.xmax || !rs.ymax || !rs.t0 || !keep ||
+    if (!rs.cnt || !rs.peak || !rs.xmin || !rs.xmax || !rs.ymax || !rs.t0 ||
         !rawpos || !rawid_of_pos || !rk)
         return;
     if (nfg > 0) {
@@ -393,23 +377,16 @@ extern "C" void run_detection(float dthreshold, float thresh1, int ext_minarea,
         hipLaunchKernelGGL(k_det_rootstat, dim3(gfg), dim3(256), 0, st, fg, nfg, W, lab, rootpos,
                            S.cd.as<float>(), rs, rk, wa, nfg_k);
         sxg_kt_end(SXG_KT_DET_STAT);
-        hipLaunchKernelGGL(k_det_rootflag, dim3(gfg), dim3(256), 0, st, rk, nfg, rs.cnt,
-                           ext_minarea, keep, nfg_k);
     }
-    sxg_compact_nonneg(keep, rawpos, nfg, nraw_d, st, nfg_k);
-    /* pixel keys, kept pixels: sized by nfg, so that the host waits once for both counts */
+    /* pixel keys and kept pixels: sized by nfg, so that the host waits once for both counts */
     int *k0 = sxg_take<int>("det.k0", nfg), *v0 = sxg_take<int>("det.v0", nfg);
     int *k1 = sxg_take<int>("det.k1", nfg), *v1 = sxg_take<int>("det.v1", nfg);
-    int *hist = sxg_take<int>("det.hist", 256 * (size_t)(sxg_div_up(nfg + 1, 4096) + 1) + 64);
-    int *idx = v1;   /* indices of kept pixels in the foreground list, until the sort */
+    int *hist = sxg_take<int>("det.hist", sxg_radix_hist(nfg));
     if (!k0 || !v0 || !k1 || !v1 || !hist) return;
-    if (nfg > 0) {
-        hipLaunchKernelGGL(k_det_rawid, dim3(gfg), dim3(256), 0, st, rawpos, nraw_d,
-                           rawid_of_pos);
-        hipLaunchKernelGGL(k_det_pixkey, dim3(gfg), dim3(256), 0, st, rk, nfg, rawid_of_pos,
-                           keep, nfg_k);
-    }
-    sxg_compact_nonneg(keep, idx, nfg, npix_d, st, nfg_k);
+    if (!sxg_pick(PickRoots{rk, rs.cnt, ext_minarea, rawpos, rawid_of_pos}, nfg, nraw_d, st,
+                  nfg_k) ||
+        !sxg_pick(PickPixels{rk, rawid_of_pos, fg, k0, v0}, nfg, npix_d, st, nfg_k))
+        return;
     int nraw, npix;
     if (pd) {
         nraw = (int)S.plan->cap[PL_NRAW];
@@ -432,8 +409,6 @@ extern "C" void run_detection(float dthreshold, float thresh1, int ext_minarea,
         S.seen.cap[PL_NPIX] = npix;
     }
     if (npix > 0) {
-        hipLaunchKernelGGL(k_det_gather, dim3(sxg_div_up(npix, 256)), dim3(256), 0, st, idx, npix,
-                           keep, fg, k0, v0, npix_k);
         /* enough key bits for every object id (for the capacity in a planned run: more
            passes over zero digits leave a stable sort's order as it is) */
         int nbits = 0;

@@ -341,18 +341,18 @@ void sxg_stage_end(StageId s);
    on the device; the launches are sized for n. */
 void sxg_scan_excl(const int *in, int *out, int n, int *total, hipStream_t s,
                    const int *nd = nullptr);
-/* Stream compaction of the indices i in [0,n) with flag[i] != 0, in increasing order;
-   *count (device) receives the number kept. */
-void sxg_compact_index(const int *flag, int *out, int n, int *count, hipStream_t s,
-                       const int *nd = nullptr);
-/* Same, keeping the indices i with v[i] >= 0. */
+/* keep[i] = 1 for the objects that no other has taken (master[i] 0xffffffff), else 0, rank
+   their exclusive prefix sum and *total their number, in one launch; false (and nothing
+   done) for more of them than one workgroup scans */
+bool sxg_scan_kept(const unsigned *master, int *keep, int *rank, int n, int *total,
+                   hipStream_t s, const int *nd);
 /* the set bits of nw 64-bit window masks as positions 64 w + b, in increasing order */
 void sxg_compact_mask(const unsigned long long *m, long nw, int *out, int *count,
                       hipStream_t s);
-void sxg_compact_nonneg(const int *v, int *out, int n, int *count, hipStream_t s,
-                        const int *nd = nullptr);
 /* Stable LSD radix sort of (key, value) pairs on the low nbits of non-negative keys;
-   returns 0 when the result is in (k0, v0), 1 when in (k1, v1). */
+   returns 0 when the result is in (k0, v0), 1 when in (k1, v1).  hist: sxg_radix_hist(n)
+   ints. */
+size_t sxg_radix_hist(int n);
 int sxg_radix_sort(int *k0, int *v0, int *k1, int *v1, int n, int nbits, int *hist,
                    hipStream_t s, const int *nd = nullptr);
 /* Planned runs: queue the check of the device count *v against cap (bit: its PlanCap);

@@ -9,6 +9,7 @@
 #include <mutex>
 
 #include "sxg_internal.h"
+#include "sxg_wave.h"
 
 /* ---------------------------------------------------------------- errors ---- */
 /* per calling thread: contexts may run on several host threads at once */
@@ -303,6 +304,9 @@ extern "C" void sxg_release(void)
 /* counts up to this many are scanned by one workgroup in one launch */
 #define SCAN_SMALL 32768
 #define SCAN_SMALL_THREADS 1024
+/* survivors flagged by the scan itself: its workgroup's stores hold up its loads (20,000
+   objects: 15 us against 3 for the flags by a launch of their own and 8 for the scan) */
+#define SCAN_KEPT 4096
 
 /* workgroup-wide exclusive scan of one value per thread (NT threads): an inclusive scan
    inside each wavefront, then the wavefront totals through LDS; returns the total */
@@ -406,14 +410,26 @@ __global__ void __launch_bounds__(SCAN_BLOCK) k_scan_apply(const int *in, int *o
    stores), each thread scans a contiguous run of them.  The run length is odd (at most
    33), so the lanes of a wavefront, which read LDS words a run length apart, hit
    distinct banks. */
-__global__ void __launch_bounds__(SCAN_SMALL_THREADS) k_scan_small(const int *in, int *out, int n,
+struct ScanInts {
+    const int *in;
+    __device__ int operator()(int k) const { return in[k]; }
+};
+/* 1 for the objects that no other one has taken in CLEAN, which is also stored */
+struct ScanKept {
+    const unsigned *master;
+    int *keep;
+    __device__ int operator()(int k) const { return keep[k] = master[k] == 0xffffffffu; }
+};
+
+template <class In>
+__global__ void __launch_bounds__(SCAN_SMALL_THREADS) k_scan_small(In in, int *out, int n,
                                                                    int *total, const int *nd)
 {
     extern __shared__ int sv[];
     __shared__ int sm[SCAN_SMALL_THREADS / 64];
     n = sxg_dn(nd, n);
 #pragma unroll 8
-    for (int k = threadIdx.x; k < n; k += SCAN_SMALL_THREADS) sv[k] = in[k];
+    for (int k = threadIdx.x; k < n; k += SCAN_SMALL_THREADS) sv[k] = in(k);
     __syncthreads();
     const int per = ((n + SCAN_SMALL_THREADS - 1) / SCAN_SMALL_THREADS) | 1;
     const int b = threadIdx.x * per, e = min(b + per, n);
@@ -437,6 +453,44 @@ __global__ void k_set_int(int *p, int v)
     if (threadIdx.x == 0) *p = v;
 }
 
+void sxg_set_int(int *p, int v, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_set_int, dim3(1), dim3(64), 0, s, p, v);
+}
+
+int *sxg_block_sums(int nb)
+{
+    SxgState &S = sxg_state();
+    return S.scan_tmp.ensure(sizeof(int) * ((size_t)nb + 64)) ? S.scan_tmp.as<int>() : nullptr;
+}
+
+void sxg_scan_blocks(int *bsum, int nb, int *total, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(1024), 0, s, bsum, nb, total);
+}
+
+template <class In>
+static void scan_small(In in, int *out, int n, int *total, hipStream_t s, const int *nd)
+{
+    /* the attribute is per function: set once (thread-safe static initialisation) */
+    static const bool attr = [] {
+        return hipFuncSetAttribute(reinterpret_cast<const void *>(&k_scan_small<In>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   SCAN_SMALL * (int)sizeof(int)) == hipSuccess;
+    }();
+    (void)attr;
+    hipLaunchKernelGGL(k_scan_small<In>, dim3(1), dim3(SCAN_SMALL_THREADS),
+                       (size_t)n * sizeof(int), s, in, out, n, total, nd);
+}
+
+bool sxg_scan_kept(const unsigned *master, int *keep, int *rank, int n, int *total,
+                   hipStream_t s, const int *nd)
+{
+    if (n > SCAN_KEPT) return false;
+    scan_small(ScanKept{master, keep}, rank, n, total, s, nd);
+    return true;
+}
+
 /* exclusive prefix sum of n ints (in == out allowed); the total to *total (device) */
 void sxg_scan_excl(const int *in, int *out, int n, int *total, hipStream_t s, const int *nd)
 {
@@ -446,15 +500,7 @@ void sxg_scan_excl(const int *in, int *out, int n, int *total, hipStream_t s, co
         return;
     }
     if (n <= SCAN_SMALL) {
-        /* the attribute is per function: set once (thread-safe static initialisation) */
-        static const bool attr = [] {
-            return hipFuncSetAttribute(reinterpret_cast<const void *>(&k_scan_small),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       SCAN_SMALL * (int)sizeof(int)) == hipSuccess;
-        }();
-        (void)attr;
-        hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(SCAN_SMALL_THREADS),
-                           (size_t)n * sizeof(int), s, in, out, n, total, nd);
+        scan_small(ScanInts{in}, out, n, total, s, nd);
         return;
     }
     const int nb = sxg_div_up(n, SCAN_TILE);
@@ -467,83 +513,10 @@ void sxg_scan_excl(const int *in, int *out, int n, int *total, hipStream_t s, co
 }
 
 /* ------------------------------------------------------------ compaction ---- */
-/* Contiguous per-thread chunks keep the output in increasing index order. */
-struct PredNonzero { __device__ bool operator()(int v) const { return v != 0; } };
-struct PredNonneg { __device__ bool operator()(int v) const { return v >= 0; } };
-
-template <class P>
-__global__ void __launch_bounds__(SCAN_BLOCK) k_compact_count(const int *flag, int n, int *bsum,
-                                                              const int *nd)
-{
-    __shared__ int sm[SCAN_BLOCK / 64];
-    n = sxg_dn(nd, n);
-    const long base = (long)blockIdx.x * SCAN_TILE + (long)threadIdx.x * SCAN_ITEMS;
-    int v[SCAN_ITEMS], s = 0;
-    load16(flag, base, n, v);
-#pragma unroll
-    for (int i = 0; i < SCAN_ITEMS; i++) s += (base + i < n && P()(v[i])) ? 1 : 0;
-    int tot;
-    block_excl_scan(s, sm, &tot);
-    if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
-}
-
-template <class P>
-__global__ void __launch_bounds__(SCAN_BLOCK) k_compact_write(const int *flag, int n,
-                                                              const int *bsum, int *out,
-                                                              const int *nd)
-{
-    __shared__ int sm[SCAN_BLOCK / 64];
-    n = sxg_dn(nd, n);
-    const long base = (long)blockIdx.x * SCAN_TILE + (long)threadIdx.x * SCAN_ITEMS;
-    int v[SCAN_ITEMS], s = 0;
-    load16(flag, base, n, v);
-    unsigned f = 0;
-#pragma unroll
-    for (int i = 0; i < SCAN_ITEMS; i++)
-        if (base + i < n && P()(v[i])) {
-            f |= 1u << i;
-            s++;
-        }
-    int tot;
-    int pos = block_excl_scan(s, sm, &tot) + bsum[blockIdx.x];
-#pragma unroll
-    for (int i = 0; i < SCAN_ITEMS; i++)
-        if (f & (1u << i)) out[pos++] = (int)(base + i);
-}
-
-template <class P>
-static void compact_impl(const int *flag, int *out, int n, int *count, hipStream_t s,
-                         const int *nd)
-{
-    SxgState &S = sxg_state();
-    if (n <= 0) {
-        hipLaunchKernelGGL(k_set_int, dim3(1), dim3(64), 0, s, count, 0);
-        return;
-    }
-    const int nb = sxg_div_up(n, SCAN_TILE);
-    if (!S.scan_tmp.ensure(sizeof(int) * (nb + 64))) return;
-    int *bsum = S.scan_tmp.as<int>();
-    hipLaunchKernelGGL(k_compact_count<P>, dim3(nb), dim3(SCAN_BLOCK), 0, s, flag, n, bsum, nd);
-    hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(1024), 0, s, bsum, nb, count);
-    hipLaunchKernelGGL(k_compact_write<P>, dim3(nb), dim3(SCAN_BLOCK), 0, s, flag, n, bsum, out,
-                       nd);
-}
-
-void sxg_compact_index(const int *flag, int *out, int n, int *count, hipStream_t s,
-                       const int *nd)
-{
-    compact_impl<PredNonzero>(flag, out, n, count, s, nd);
-}
-
-void sxg_compact_nonneg(const int *v, int *out, int n, int *count, hipStream_t s, const int *nd)
-{
-    compact_impl<PredNonneg>(v, out, n, count, s, nd);
-}
-
 /* The positions of the set bits of nw 64-bit window masks (bit b of mask w: position
    64 w + b) in increasing order, and their number: one lane per window counts its bits;
-   after the scan of the workgroup sums each lane writes its window's positions in bit
-   order.  Reads the masks (8 bytes per 64 positions) instead of a flag per position. */
+   after the scan of the workgroup sums (sxg_block_offset) each lane writes its window's
+   positions in bit order.  Reads the masks (8 bytes per 64 positions) instead of a flag per position. */
 __global__ void __launch_bounds__(SCAN_BLOCK) k_fgm_count(const unsigned long long *m, long nw,
                                                           int *bsum)
 {
@@ -554,14 +527,16 @@ __global__ void __launch_bounds__(SCAN_BLOCK) k_fgm_count(const unsigned long lo
     if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
 }
 
+template <bool SCANNED>
 __global__ void __launch_bounds__(SCAN_BLOCK) k_fgm_write(const unsigned long long *m, long nw,
-                                                          const int *bsum, int *out)
+                                                          const int *bsum, int *out, int *count)
 {
     __shared__ int sm[SCAN_BLOCK / 64];
     const long w = (long)blockIdx.x * SCAN_BLOCK + threadIdx.x;
     unsigned long long b = w < nw ? m[w] : 0ull;
+    const int first = sxg_block_offset<SCANNED>(bsum, count);
     int tot;
-    int pos = block_excl_scan(__popcll(b), sm, &tot) + bsum[blockIdx.x];
+    int pos = first + block_excl_scan(__popcll(b), sm, &tot);
     const int base = (int)(w * 64);
     while (b) {
         out[pos++] = base + __builtin_ctzll(b);
@@ -571,13 +546,18 @@ __global__ void __launch_bounds__(SCAN_BLOCK) k_fgm_write(const unsigned long lo
 
 void sxg_compact_mask(const unsigned long long *m, long nw, int *out, int *count, hipStream_t s)
 {
-    SxgState &S = sxg_state();
     const int nb = (int)sxg_div_up(nw, SCAN_BLOCK);
-    if (nb < 1 || !S.scan_tmp.ensure(sizeof(int) * (nb + 64))) return;
-    int *bsum = S.scan_tmp.as<int>();
+    int *bsum = nb < 1 ? nullptr : sxg_block_sums(nb);
+    if (!bsum) return;
     hipLaunchKernelGGL(k_fgm_count, dim3(nb), dim3(SCAN_BLOCK), 0, s, m, nw, bsum);
-    hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(1024), 0, s, bsum, nb, count);
-    hipLaunchKernelGGL(k_fgm_write, dim3(nb), dim3(SCAN_BLOCK), 0, s, m, nw, bsum, out);
+    if (nb > SXG_BLOCK_SUMS) {
+        sxg_scan_blocks(bsum, nb, count, s);
+        hipLaunchKernelGGL(k_fgm_write<true>, dim3(nb), dim3(SCAN_BLOCK), 0, s, m, nw, bsum, out,
+                           count);
+    } else {
+        hipLaunchKernelGGL(k_fgm_write<false>, dim3(nb), dim3(SCAN_BLOCK), 0, s, m, nw, bsum, out,
+                           count);
+    }
 }
 
 /* ------------------------------------------------------------ plan guards ---- */

@@ -491,3 +491,142 @@ template <int ND, int NF, SxwSize Z> struct SxwSums {
         }
     }
 };
+
+/*
+ * The output offset of this workgroup (256 threads) of a two-launch compaction: the sum of the
+ * counts of the workgroups before it, which every workgroup adds up itself (a launch of one
+ * workgroup for the scan took longer, with its gap, than these reads), or, of more than
+ * SXG_BLOCK_SUMS workgroups, the sums as a launch between the two has scanned them.  The last
+ * workgroup stores the total.
+ */
+#define SXG_BLOCK_SUMS 4096
+template <bool SCANNED> __device__ inline int sxg_block_offset(const int *bsum, int *total)
+{
+    if (SCANNED) return bsum[blockIdx.x];
+    __shared__ int s_part[4];
+    const int b = blockIdx.x;
+    int s = 0;
+    for (int j = threadIdx.x; j < b; j += 256) s += bsum[j];
+    s = sxw_sum(s);
+    if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = s;
+    __syncthreads();
+    s = s_part[0] + s_part[1] + s_part[2] + s_part[3];
+    if (b == (int)gridDim.x - 1 && threadIdx.x == 0) *total = s + bsum[b];
+    return s;
+}
+
+/*
+ * Two-launch stable compaction of the indices 0 .. n - 1 that src keeps: src.read(k) is what
+ * decides, src.take(k, that) the kept value (>= 0) or -1, src.put(place, k, value) stores it.
+ * ITEMS indices a thread, 256 apart, so that loads and stores are coalesced; every first load
+ * is issued before one is used (crowded 4096 x 4096 frame: 14 us a count of 10^6 where each
+ * was waited for).
+ */
+template <class Src, int ITEMS>
+__device__ inline void sxg_pick_values(const Src &src, long base, int n, int (&v)[ITEMS])
+{
+#pragma unroll
+    for (int i = 0; i < ITEMS; i++) {
+        const long k = base + 256 * i;
+        v[i] = src.read(k < n ? (int)k : n - 1);
+    }
+#pragma unroll
+    for (int i = 0; i < ITEMS; i++) {
+        const long k = base + 256 * i;
+        const int t = src.take(k < n ? (int)k : n - 1, v[i]);
+        v[i] = k < n ? t : -1;
+    }
+}
+
+template <class Src, int ITEMS>
+__global__ void __launch_bounds__(256) k_pick_count(Src src, int n, int *bsum, const int *nd)
+{
+    __shared__ int s_part[4];
+    if (nd) n = min(*nd, n);
+    const long base = (long)blockIdx.x * (256 * ITEMS) + threadIdx.x;
+    int c = 0;
+    if (n > 0) {
+        int v[ITEMS];
+        sxg_pick_values(src, base, n, v);
+#pragma unroll
+        for (int i = 0; i < ITEMS; i++) c += __popcll(__ballot(v[i] >= 0));
+    }
+    if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) bsum[blockIdx.x] = s_part[0] + s_part[1] + s_part[2] + s_part[3];
+}
+
+template <class Src, int ITEMS, bool SCANNED>
+__global__ void __launch_bounds__(256) k_pick_write(Src src, int n, const int *bsum, int *total,
+                                                    const int *nd)
+{
+    __shared__ int s_at[64];   /* by item and wavefront: kept ones before it in the workgroup */
+    if (nd) n = min(*nd, n);
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const long base = (long)blockIdx.x * (256 * ITEMS) + threadIdx.x;
+    int v[ITEMS];
+#pragma unroll
+    for (int i = 0; i < ITEMS; i++) v[i] = -1;
+    if (n > 0) sxg_pick_values(src, base, n, v);
+#pragma unroll
+    for (int i = 0; i < ITEMS; i++) {
+        const int c = __popcll(__ballot(v[i] >= 0));
+        if (lane == 0) s_at[4 * i + wid] = c;
+    }
+    const int first = sxg_block_offset<SCANNED>(bsum, total);
+    __syncthreads();
+    if (wid == 0) {
+        const int own = lane < 4 * ITEMS ? s_at[lane] : 0;
+        int x = own;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(x, d);
+            if (lane >= d) x += o;
+        }
+        s_at[lane] = first + x - own;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ITEMS; i++) {
+        const unsigned long long b = __ballot(v[i] >= 0);
+        if (v[i] >= 0)
+            src.put(s_at[4 * i + wid] + __popcll(b & sxw_lanes_below(lane)),
+                    (int)(base + 256 * i), v[i]);
+    }
+}
+
+int *sxg_block_sums(int nb);   /* device: nb ints */
+void sxg_scan_blocks(int *bsum, int nb, int *total, hipStream_t s);
+void sxg_set_int(int *p, int v, hipStream_t s);
+
+/* With nd (planned runs) n is a capacity and the number of indices is *nd (<= n).  Up to
+   2^18 indices 1024 a workgroup, so that small frames have more than a few of them, else
+   4096: the sums that every workgroup adds up grow with their number. */
+template <class Src>
+bool sxg_pick(const Src &src, int n, int *count, hipStream_t s, const int *nd)
+{
+    if (n <= 0) {
+        sxg_set_int(count, 0, s);
+        return true;
+    }
+    const bool small = n <= 1 << 18;
+    const int nb = (int)(((long)n + (small ? 1023 : 4095)) / (small ? 1024 : 4096));
+    int *bsum = sxg_block_sums(nb);
+    if (!bsum) return false;
+    if (small) {
+        hipLaunchKernelGGL((k_pick_count<Src, 4>), dim3(nb), dim3(256), 0, s, src, n, bsum, nd);
+        hipLaunchKernelGGL((k_pick_write<Src, 4, false>), dim3(nb), dim3(256), 0, s, src, n, bsum,
+                           count, nd);
+        return true;
+    }
+    hipLaunchKernelGGL((k_pick_count<Src, 16>), dim3(nb), dim3(256), 0, s, src, n, bsum, nd);
+    if (nb > SXG_BLOCK_SUMS) {
+        sxg_scan_blocks(bsum, nb, count, s);
+        hipLaunchKernelGGL((k_pick_write<Src, 16, true>), dim3(nb), dim3(256), 0, s, src, n, bsum,
+                           count, nd);
+    } else {
+        hipLaunchKernelGGL((k_pick_write<Src, 16, false>), dim3(nb), dim3(256), 0, s, src, n,
+                           bsum, count, nd);
+    }
+    return true;
+}
