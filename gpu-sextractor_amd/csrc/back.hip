@@ -902,16 +902,15 @@ __device__ float wg_median(const float *a, int n, int cnt, bool positive, int *h
     return (float)((lo + hi) / 2.0);
 }
 
-/* global medians of the filtered maps (back.c:532-556): workgroup 0 the background,
-   workgroup 1 the sigma (with the median of the strictly positive sigmas when the median
-   is not positive, 1 when there is none) */
-__global__ void __launch_bounds__(FB_THREADS) k_fb_global(const float *back, const float *sigma,
-                                                          int np, float *out)
+/* global medians of the filtered maps (back.c:532-556): of the background, or of the sigma
+   (with the median of the strictly positive sigmas when the median is not positive, 1 when
+   there is none) */
+__device__ void fb_global(const float *back, const float *sigma, int np, float *out, bool sig)
 {
     __shared__ int hist[256];
     __shared__ int sel[2];
     __shared__ int s_npos;
-    if (blockIdx.x == 0) {
+    if (!sig) {
         const float m = wg_median(back, np, np, false, hist, sel);
         if (threadIdx.x == 0) out[0] = m;
         return;
@@ -930,31 +929,35 @@ __global__ void __launch_bounds__(FB_THREADS) k_fb_global(const float *back, con
     if (threadIdx.x == 0) out[1] = bsig;
 }
 
+/* (float)(v / 6.0): a float division gives the same.  v / 6 is either a float or its binary
+   digits end in a repeating 01, which lies a third of a unit from a tie at any precision, so
+   the rounding to double in between cannot make one. */
+__device__ inline float sixth(float v) { return v / 6.0f; }
+
+/* the loads of a recurrence: this many elements read before the first of them is used */
+#define SP_AHEAD 8
+
 /* y second derivatives of back and sigma, one lane per mesh column (back.c:739-780);
    the forward recurrence runs in registers and keeps its per-row values (the
    tridiagonal factors and uu) for the backward pass in LDS when ny rows of 64 lanes fit
-   (use_lds), else in uu_all (2 * ny floats per column) */
-__global__ void __launch_bounds__(64) k_fb_yderiv(const float *back, const float *sigma,
-                                                  float *dback, float *dsigma, int nx, int ny,
-                                                  int use_lds, float *uu_all)
+   (yd), else in uu_all (2 * ny floats per column) */
+__device__ void fb_yderiv(const float *back, const float *sigma, float *dback, float *dsigma,
+                          int nx, int ny, float *yd, float *uu_all, int c)
 {
-    extern __shared__ float yd[];
-    const int c = blockIdx.x * 64 + threadIdx.x;
-    const bool live = c < 2 * nx;
-    const int x = c % nx;
-    const float *map = c < nx ? back : sigma;
-    float *dmap = c < nx ? dback : dsigma;
-    if (!live) return;
+    if (c >= 2 * nx) return;
+    const int x = c % nx, lane = threadIdx.x & 63;
+    const float *map = (c < nx ? back : sigma) + x;
+    float *dmap = (c < nx ? dback : dsigma) + x;
     if (ny < 2) {
-        dmap[x] = 0.0f;
+        dmap[0] = 0.0f;
         return;
     }
     /* element y of this column's two scratch rows */
     float *ta, *tb;
     size_t st;
-    if (use_lds) {
-        ta = yd + threadIdx.x;
-        tb = yd + (size_t)ny * 64 + threadIdx.x;
+    if (yd) {
+        ta = yd + lane;
+        tb = yd + (size_t)ny * 64 + lane;
         st = 64;
     } else {
         ta = uu_all + (size_t)c * 2 * ny;
@@ -962,25 +965,99 @@ __global__ void __launch_bounds__(64) k_fb_yderiv(const float *back, const float
         st = 1;
     }
     float dprev = 0.0f, uprev = 0.0f;
-    float m0 = map[x], m1 = map[nx + x];
-    for (int y = 1; y < ny - 1; y++) {
-        const float m2 = map[(y + 1) * nx + x];
-        float temp = -1 / (dprev + 4);
-        ta[y * st] = temp;
-        dprev = temp;
-        temp *= uprev - 6 * (m2 + m0 - 2 * m1);
-        tb[y * st] = temp;
-        uprev = temp;
-        m0 = m1;
-        m1 = m2;
+    float m0 = map[0], m1 = map[nx];
+    for (int y0 = 1; y0 < ny - 1; y0 += SP_AHEAD) {
+        float m[SP_AHEAD];
+#pragma unroll
+        for (int k = 0; k < SP_AHEAD; k++) m[k] = map[(size_t)min(y0 + k + 1, ny - 1) * nx];
+#pragma unroll
+        for (int k = 0; k < SP_AHEAD; k++) {
+            const int y = y0 + k;
+            if (y < ny - 1) {
+                const float m2 = m[k];
+                float temp = -1 / (dprev + 4);
+                ta[y * st] = temp;
+                dprev = temp;
+                temp *= uprev - 6 * (m2 + m0 - 2 * m1);
+                tb[y * st] = temp;
+                uprev = temp;
+                m0 = m1;
+                m1 = m2;
+            }
+        }
     }
-    dmap[x] = 0.0f;
-    dmap[(ny - 1) * nx + x] = 0.0f;
+    dmap[0] = 0.0f;
+    dmap[(size_t)(ny - 1) * nx] = 0.0f;
     float dnext = 0.0f;
-    for (int y = ny - 2; y >= 1; y--) {
-        const float d = (float)((ta[y * st] * dnext + tb[y * st]) / 6.0);
-        dmap[y * nx + x] = d;
-        dnext = d;
+    for (int y0 = ny - 2; y0 >= 1; y0 -= SP_AHEAD) {
+        float p[SP_AHEAD], q[SP_AHEAD];
+#pragma unroll
+        for (int k = 0; k < SP_AHEAD; k++) {
+            const int y = max(y0 - k, 1);
+            p[k] = ta[y * st];
+            q[k] = tb[y * st];
+        }
+#pragma unroll
+        for (int k = 0; k < SP_AHEAD; k++)
+            if (y0 - k >= 1) {
+                dnext = sixth(p[k] * dnext + q[k]);
+                dmap[(size_t)(y0 - k) * nx] = dnext;
+            }
+    }
+}
+
+/* The column tables of the x loop of subbackline (back.c:880-908): for each column, the
+   index of its left node and the dx of the cumulative float recurrence dx += xstep,
+   which starts at (xstep - 1)/2 and restarts at dx0 at the half of every mesh t in
+   [1, nbx - 2] (the loop's pixel with i == bs/2, column t*bs + bs/2).  One lane per
+   restart segment performs that segment's additions in the loop's order, so every value
+   is the loop's own IEEE result. */
+__device__ void fb_coltables(int W, int nbx, int bs, int *colseg, float *coldx, int t,
+                             int nthreads)
+{
+    if (nbx <= 1) {
+        for (int j = t; j < W; j += nthreads) {
+            colseg[j] = 0;
+            coldx[j] = 0.0f;
+        }
+        return;
+    }
+    const int cp = bs / 2;
+    const int nseg = cp >= 1 && nbx > 2 ? nbx - 1 : 1;
+    if (t >= nseg) return;
+    const float xstep = (float)(1.0 / bs);
+    float dx = t == 0 ? (xstep - 1) / 2 : ((bs + 1) % 2) * xstep / 2;
+    const int j0 = t == 0 ? 0 : t * bs + cp;
+    const int j1 = t + 1 < nseg ? min((t + 1) * bs + cp, W) : W;
+    for (int j = j0; j < j1; j++) {
+        colseg[j] = t;
+        coldx[j] = dx;
+        dx = dx + xstep;
+    }
+}
+
+/* What follows the filtered mesh maps, in one launch, as none of its parts needs another's
+   result: workgroups 0 and 1 the global medians, then workgroups for the y derivatives (64
+   columns of the maps each, on one wavefront) and for the column tables.  Each part is a chain
+   of dependent steps on a few wavefronts: as launches of their own they took 18, 17 and 6 us
+   one after the other at 4096 x 4096 and 8, 6 and 5 at 1024 x 1024. */
+__global__ void __launch_bounds__(FB_THREADS) k_fb_tail(const float *back, const float *sigma,
+                                                        float *dback, float *dsigma, int nx,
+                                                        int ny, int use_lds, float *uu_all,
+                                                        float *out, int W, int bs, int *colseg,
+                                                        float *coldx)
+{
+    extern __shared__ float yd[];
+    const int ncol = (2 * nx + 63) / 64, b = (int)blockIdx.x - 2;
+    if (b < 0) {
+        fb_global(back, sigma, nx * ny, out, b + 1);
+    } else if (b < ncol) {
+        if (threadIdx.x < 64)
+            fb_yderiv(back, sigma, dback, dsigma, nx, ny, use_lds ? yd : nullptr, uu_all,
+                      b * 64 + threadIdx.x);
+    } else {
+        fb_coltables(W, nx, bs, colseg, coldx, (b - ncol) * FB_THREADS + threadIdx.x,
+                     ((int)gridDim.x - 2 - ncol) * FB_THREADS);
     }
 }
 
@@ -1034,17 +1111,22 @@ __global__ void __launch_bounds__(256) k_rownodes(const float *back, const float
 }
 
 /* the same for RN_ROWS consecutive rows per workgroup (one lane each) with the row
-   arrays in LDS, laid out [x][row] (no bank conflicts), and coalesced stores of the
-   finished rows; used when 3 * nbx * RN_ROWS floats fit in LDS */
+   arrays in LDS, laid out [x][row] with a stride of RN_ST (no bank conflicts along rows or
+   columns), and coalesced stores of the finished rows; used when 3 * nbx * RN_ST floats fit in
+   RN_LDS.  A chain of 2 nbx dependent divisions a lane, 64 nodes: 22 us with a stride of 64
+   (the stores' reads all on one bank, a division an element) and every element's reads waited
+   for in the recurrences, 15 us now. */
 #define RN_ROWS 64
+#define RN_ST 65
+#define RN_LDS (128 * 1024)
 __global__ void __launch_bounds__(RN_ROWS) k_rownodes_lds(const float *back, const float *dback,
                                                           int nbx, int nby, int bs, int H,
                                                           float *nodes, float *dnodes)
 {
     extern __shared__ float rn[];
     const int lane = threadIdx.x, y0 = blockIdx.x * RN_ROWS, y = y0 + lane;
-    float *node = rn, *dnode = rn + nbx * RN_ROWS, *u = dnode + nbx * RN_ROWS;
-#define RN(a, x) a[(x) * RN_ROWS + lane]
+    float *node = rn, *dnode = rn + nbx * RN_ST, *u = dnode + nbx * RN_ST;
+#define RN(a, x) a[(x) * RN_ST + lane]
     if (y < H) {
         if (nby > 1) {
             int yl;
@@ -1062,21 +1144,44 @@ __global__ void __launch_bounds__(RN_ROWS) k_rownodes_lds(const float *back, con
             const float cdy3 = (cdy * cdy * cdy - cdy);
             const float *blo = back + nbx * yl, *bhi = blo + nbx;
             const float *dblo = dback + nbx * yl, *dbhi = dblo + nbx;
+#pragma unroll 8
             for (int x = 0; x < nbx; x++)
                 RN(node, x) = cdy * blo[x] + dy * bhi[x] + cdy3 * dblo[x] + dy3 * dbhi[x];
             if (nbx > 1) {
                 float temp, dprev = 0.0f, uprev = 0.0f;
+                float n0 = RN(node, 0), n1 = RN(node, 1);
                 RN(dnode, 0) = RN(u, 0) = 0.0f;
-                for (int x = 1; x < nbx - 1; x++) {
-                    temp = -1 / (dprev + 4);
-                    RN(dnode, x) = dprev = temp;
-                    temp *= uprev - 6 * (RN(node, x + 1) + RN(node, x - 1) - 2 * RN(node, x));
-                    RN(u, x) = uprev = temp;
+                for (int x0 = 1; x0 < nbx - 1; x0 += SP_AHEAD) {
+                    float n[SP_AHEAD];
+#pragma unroll
+                    for (int k = 0; k < SP_AHEAD; k++) n[k] = RN(node, min(x0 + k + 1, nbx - 1));
+#pragma unroll
+                    for (int k = 0; k < SP_AHEAD; k++) {
+                        const int x = x0 + k;
+                        if (x < nbx - 1) {
+                            temp = -1 / (dprev + 4);
+                            RN(dnode, x) = dprev = temp;
+                            temp *= uprev - 6 * (n[k] + n0 - 2 * n1);
+                            RN(u, x) = uprev = temp;
+                            n0 = n1;
+                            n1 = n[k];
+                        }
+                    }
                 }
                 RN(dnode, nbx - 1) = 0.0f;
                 float dnext = 0.0f;
-                for (int x = nbx - 2; x >= 1; x--)
-                    RN(dnode, x) = dnext = (float)((RN(dnode, x) * dnext + RN(u, x)) / 6.0);
+                for (int x0 = nbx - 2; x0 >= 1; x0 -= SP_AHEAD) {
+                    float p[SP_AHEAD], q[SP_AHEAD];
+#pragma unroll
+                    for (int k = 0; k < SP_AHEAD; k++) {
+                        p[k] = RN(dnode, max(x0 - k, 1));
+                        q[k] = RN(u, max(x0 - k, 1));
+                    }
+#pragma unroll
+                    for (int k = 0; k < SP_AHEAD; k++)
+                        if (x0 - k >= 1)
+                            RN(dnode, x0 - k) = dnext = sixth(p[k] * dnext + q[k]);
+                }
             }
         } else {
             for (int x = 0; x < nbx; x++) {
@@ -1089,10 +1194,18 @@ __global__ void __launch_bounds__(RN_ROWS) k_rownodes_lds(const float *back, con
     __syncthreads();
     /* rows y0.. are contiguous in the node tables */
     const int nr = min(RN_ROWS, H - y0), tot = nr * nbx;
+    const int dr = RN_ROWS / nbx, dx = RN_ROWS - dr * nbx;
+    int r = lane / nbx, x = lane - r * nbx;
+#pragma unroll 4
     for (int e = lane; e < tot; e += RN_ROWS) {
-        const int r = e / nbx, x = e - r * nbx;
-        nodes[(size_t)y0 * nbx + e] = node[x * RN_ROWS + r];
-        dnodes[(size_t)y0 * nbx + e] = dnode[x * RN_ROWS + r];
+        nodes[(size_t)y0 * nbx + e] = node[x * RN_ST + r];
+        dnodes[(size_t)y0 * nbx + e] = dnode[x * RN_ST + r];
+        r += dr;
+        x += dx;
+        if (x >= nbx) {
+            x -= nbx;
+            r++;
+        }
     }
 }
 
@@ -1130,37 +1243,6 @@ __global__ void __launch_bounds__(256) k_subconst(const float *src, float *dst, 
 }
 
 __global__ void k_setval(float *p, float v) { *p = v; }
-
-/* The column tables of the x loop of subbackline (back.c:880-908): for each column, the
-   index of its left node and the dx of the cumulative float recurrence dx += xstep,
-   which starts at (xstep - 1)/2 and restarts at dx0 at the half of every mesh t in
-   [1, nbx - 2] (the loop's pixel with i == bs/2, column t*bs + bs/2).  One lane per
-   restart segment performs that segment's additions in the loop's order, so every value
-   is the loop's own IEEE result. */
-__global__ void __launch_bounds__(64) k_coltables(int W, int nbx, int bs, int *colseg,
-                                                  float *coldx)
-{
-    const int t = blockIdx.x * 64 + threadIdx.x;
-    if (nbx <= 1) {
-        for (int j = t; j < W; j += gridDim.x * 64) {
-            colseg[j] = 0;
-            coldx[j] = 0.0f;
-        }
-        return;
-    }
-    const int cp = bs / 2;
-    const int nseg = cp >= 1 && nbx > 2 ? nbx - 1 : 1;
-    if (t >= nseg) return;
-    const float xstep = (float)(1.0 / bs);
-    float dx = t == 0 ? (xstep - 1) / 2 : ((bs + 1) % 2) * xstep / 2;
-    const int j0 = t == 0 ? 0 : t * bs + cp;
-    const int j1 = t + 1 < nseg ? min((t + 1) * bs + cp, W) : W;
-    for (int j = j0; j < j1; j++) {
-        colseg[j] = t;
-        coldx[j] = dx;
-        dx = dx + xstep;
-    }
-}
 
 /* Byte layout of the device buffers of one background estimate of a W x H frame with
    nbx x nby meshes, each part 256-byte aligned: mesh statistics, work (4*n2 floats and
@@ -1209,8 +1291,11 @@ static BackBufs back_bufs(char *base, const BackLayout &L, int W, int H, int nbx
 static bool spline_rows(const BackGeom &g, const BackBufs &b, const float *map,
                         const float *dmap, hipStream_t st)
 {
-    const size_t rnlds = 3 * (size_t)g.nbx * RN_ROWS * sizeof(float);
-    if (rnlds <= 64 * 1024) {
+    const size_t rnlds = 3 * (size_t)g.nbx * RN_ST * sizeof(float);
+    static const bool attr =
+        hipFuncSetAttribute(reinterpret_cast<const void *>(&k_rownodes_lds),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, RN_LDS) == hipSuccess;
+    if (attr && rnlds <= RN_LDS) {
         hipLaunchKernelGGL(k_rownodes_lds, dim3(sxg_div_up(g.H, RN_ROWS)), dim3(RN_ROWS), rnlds,
                            st, map, dmap, g.nbx, g.nby, g.bs, g.H, b.nodes, b.dnodes);
     } else {
@@ -1300,24 +1385,22 @@ bool sxg_back_run(const BackGeom &g, const BackBufs &b, const float *src, float 
                            nbx, nby);
         hipLaunchKernelGGL(k_fb_median, dim3(gm), dim3(256), 0, st, back2, sigma2, b.back, b.sigma,
                            nbx, nby, g.nfx, g.nfy, backfthresh);
-        hipLaunchKernelGGL(k_fb_global, dim3(2), dim3(FB_THREADS), 0, st, b.back, b.sigma, nmesh,
-                           b.outv);
         /* scratch of 2*nby floats per column: LDS when it fits, else back2/sigma2 and the
            sort buffer (4*n2 >= 2 * 2*nbx*nby floats) */
         const size_t ylds = 2 * (size_t)nby * 64 * sizeof(float);
         const int ylds_ok = ylds <= 128 * 1024;
         static const bool yattr = [] {
-            return hipFuncSetAttribute(reinterpret_cast<const void *>(&k_fb_yderiv),
+            return hipFuncSetAttribute(reinterpret_cast<const void *>(&k_fb_tail),
                                        hipFuncAttributeMaxDynamicSharedMemorySize,
                                        128 * 1024) == hipSuccess;
         }();
         if (!yattr) {
-            sxg_set_error("back_estimate: cannot raise the LDS limit of k_fb_yderiv");
+            sxg_set_error("back_estimate: cannot raise the LDS limit of k_fb_tail");
             return false;
         }
-        hipLaunchKernelGGL(k_fb_yderiv, dim3(sxg_div_up(2 * nbx, 64)), dim3(64),
-                           ylds_ok ? ylds : 0, st, b.back, b.sigma, b.dback, b.dsigma, nbx, nby,
-                           ylds_ok, back2);
+        hipLaunchKernelGGL(k_fb_tail, dim3(2 + sxg_div_up(2 * nbx, 64) + sxg_div_up(nbx, FB_THREADS)),
+                           dim3(FB_THREADS), ylds_ok ? ylds : 0, st, b.back, b.sigma, b.dback,
+                           b.dsigma, nbx, nby, ylds_ok, back2, b.outv, W, bs, b.colseg, b.coldx);
     }
     if (timed) sxg_kt_end(SXG_KT_FILTERBACK);
     if (back_type == 1 || back_type == 2) {
@@ -1331,8 +1414,6 @@ bool sxg_back_run(const BackGeom &g, const BackBufs &b, const float *src, float 
                            dst, (long)W * H, back_value, back_type == 1 ? b.outv : nullptr);
     } else {
         if (timed) sxg_kt_begin(SXG_KT_ROWNODES);
-        hipLaunchKernelGGL(k_coltables, dim3(sxg_div_up(nbx, 64)), dim3(64), 0, st, W, nbx, bs,
-                           b.colseg, b.coldx);
         if (!spline_rows(g, b, b.back, b.dback, st)) return false;
         if (timed) sxg_kt_end(SXG_KT_ROWNODES);
         /* dst nullptr: the caller subtracts the spline itself (from the row and column
