@@ -18,13 +18,14 @@
  *   k_fb_*       bad-mesh interpolation and median filtering, one lane per mesh
  *                (back.c:434-530); global medians by radix selection, one workgroup
  *                per map (back.c:532-556); y second derivatives, one lane per mesh
- *                column with the recurrence in registers (back.c:739-780).
+ *                column with the recurrence in registers (back.c:739-780); the last
+ *                two in one launch (k_fb_tail).
  *   k_rownodes   one lane per frame row: node interpolation along y and the x
  *                tridiagonal solve of subbackline (back.c:790-880); 64 rows per
  *                workgroup with the row arrays in LDS when they fit (k_rownodes_lds).
  *   k_subback    one lane per pixel: bicubic evaluation with the column tables of the
- *                cumulative dx recurrence (back.c:880-908), computed once on the host
- *                with the same float additions, and in-place subtraction.
+ *                cumulative dx recurrence (back.c:880-908), computed with the
+ *                same float additions (fb_coltables), and in-place subtraction.
  */
 #include <algorithm>
 #include <cmath>
