@@ -62,17 +62,13 @@ __global__ void __launch_bounds__(256) k_obj_order(const int *objoff, int nobj, 
     const int obj = blockIdx.x * 256 + threadIdx.x;
     const int cap = nobj;
     if (pd) nobj = pd->nobj;
-    if (obj >= nobj) return;
-    const int n = objoff[obj + 1] - objoff[obj];
-    const int big = sxw_place(&cnt[0], n >= ANA_BIG);
-    const int mid = sxw_place(&cnt[1], n >= ANA_MID && n < ANA_BIG);
-    const int low = sxw_place(&cnt[2], n < ANA_MID);
-    if (n >= ANA_BIG)
-        order[big] = obj;
-    else if (n >= ANA_MID)
-        order[cap + mid] = obj;
-    else
-        order[nobj - 1 - low] = obj;
+    int cls = -1;
+    if (obj < nobj) {
+        const int n = objoff[obj + 1] - objoff[obj];
+        cls = n >= ANA_BIG ? 0 : n >= ANA_MID ? 1 : 2;
+    }
+    const int k = sxw_place<3>(cnt, cls);
+    if (cls >= 0) order[cls == 0 ? k : cls == 1 ? cap + k : nobj - 1 - k] = obj;
 }
 
 /* back.c:685-732 */

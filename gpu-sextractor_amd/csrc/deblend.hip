@@ -246,12 +246,18 @@ __global__ void __launch_bounds__(256) k_deb_nodecap(DebArgs a)
 
 /* single-peak objects are kept as they are (one node); the others go to a size class (0:
    up to cap0 pixels, 256 lanes in LDS; 1: up to cap1, 512 lanes in LDS; 2: up to cap2, 1024
-   lanes in LDS; 3: global memory).  The counters take one atomic per wavefront and
-   class; [4 + class] records the largest LDS need. */
+   lanes in LDS; 3: global memory).  The counters take one atomic per workgroup and
+   class (one per wavefront, as the order kernels had, took 19 us for 22,000 raw objects, 7
+   now); [4 + class] records the largest LDS need. */
 __global__ void __launch_bounds__(256) k_deb_classify(DebArgs a, int cap0, int cap1, int cap2)
 {
+    __shared__ int s_n[4], s_px[4], s_need[4], s_base[4];
+    __shared__ unsigned long long s_work[2];
     const int r = blockIdx.x * 256 + threadIdx.x;
     const int lane = threadIdx.x & 63;
+    if (threadIdx.x < 4) s_n[threadIdx.x] = s_px[threadIdx.x] = s_need[threadIdx.x] = 0;
+    if (threadIdx.x < 2) s_work[threadIdx.x] = 0;
+    __syncthreads();
     int cls = -1, n = 0, ls = 0, need = 0;
     if (r < deb_nraw(a)) {
         n = a.cnt[r];
@@ -271,25 +277,39 @@ __global__ void __launch_bounds__(256) k_deb_classify(DebArgs a, int cap0, int c
         w1 += __shfl_xor(w1, d);
     }
     if (lane == 0 && w0) {
-        atomicAdd(&a.dwork[0], w0);
-        atomicAdd(&a.dwork[1], w1);
+        atomicAdd(&s_work[0], w0);
+        atomicAdd(&s_work[1], w1);
     }
+    int slot = 0;
     for (int c = 0; c < 4; c++) {
         const unsigned long long b = __ballot(cls == c);
         if (!b) continue;
         const int lead = __builtin_ctzll(b);
         int base = 0;
-        if (lane == lead) base = atomicAdd(&a.ccount[c], __popcll(b));
+        if (lane == lead) base = atomicAdd(&s_n[c], __popcll(b));
         base = __shfl(base, lead);
         int mx = cls == c ? need : 0, px = cls == c ? n : 0;
         for (int d = 32; d > 0; d >>= 1) {
             mx = max(mx, __shfl_xor(mx, d));
             px += __shfl_xor(px, d);
         }
-        if (lane == lead && c < 3) atomicMax(&a.ccount[4 + c], mx);
-        if (lane == lead) atomicAdd(&a.ccount[7 + c], px);
-        if (cls == c) a.clist[(size_t)c * a.cstride + base + __popcll(b & sxw_lanes_below(lane))] = r;
+        if (lane == lead) {
+            atomicMax(&s_need[c], mx);
+            atomicAdd(&s_px[c], px);
+        }
+        if (cls == c) slot = base + __popcll(b & sxw_lanes_below(lane));
     }
+    __syncthreads();
+    if (threadIdx.x < 4 && s_n[threadIdx.x]) {
+        const int c = threadIdx.x;
+        s_base[c] = atomicAdd(&a.ccount[c], s_n[c]);
+        if (c < 3) atomicMax(&a.ccount[4 + c], s_need[c]);
+        atomicAdd(&a.ccount[7 + c], s_px[c]);
+    }
+    if (threadIdx.x >= 4 && threadIdx.x < 6 && s_work[threadIdx.x - 4])
+        atomicAdd(&a.dwork[threadIdx.x - 4], s_work[threadIdx.x - 4]);
+    __syncthreads();
+    if (cls >= 0) a.clist[(size_t)cls * a.cstride + s_base[cls] + slot] = r;
 }
 
 /*
@@ -1003,18 +1023,14 @@ __global__ void __launch_bounds__(256) k_pre_order(ObjArgs A, int *cnt, int *ord
 {
     const int obj = blockIdx.x * 256 + threadIdx.x;
     const int nobj = obj_n(A);
-    if (obj >= nobj) return;
-    const Comp c = A.d.comps[A.d.compoff[A.objraw[obj]] + A.objcomp[obj]];
-    const int n = c.hi - c.lo + 1;
-    const int big = sxw_place(&cnt[0], n >= PRE_BIG);
-    const int mid = sxw_place(&cnt[1], n >= PRE_MID && n < PRE_BIG);
-    const int low = sxw_place(&cnt[2], n < PRE_MID);
-    if (n >= PRE_BIG)
-        order[big] = obj;
-    else if (n >= PRE_MID)
-        order[A.nobj + mid] = obj;
-    else
-        order[nobj - 1 - low] = obj;
+    int cls = -1;
+    if (obj < nobj) {
+        const Comp c = A.d.comps[A.d.compoff[A.objraw[obj]] + A.objcomp[obj]];
+        const int n = c.hi - c.lo + 1;
+        cls = n >= PRE_BIG ? 0 : n >= PRE_MID ? 1 : 2;
+    }
+    const int k = sxw_place<3>(cnt, cls);
+    if (cls >= 0) order[cls == 0 ? k : cls == 1 ? A.nobj + k : nobj - 1 - k] = obj;
 }
 
 /* objects of each raw object, in component-table order (one wavefront per raw object) */

@@ -228,13 +228,9 @@ __global__ void __launch_bounds__(256) k_phot_order(PhotArgs A, int *cnt, int *o
         ph_auto_box(A, i, cx2, cy2, cxy, klim2, flag, xmin, xmax, ymin, ymax);
         nb = (long)max(xmax - xmin, 0) * max(ymax - ymin, 0);
     }
-    const bool big = i < n && nb >= PH_BIG, mid = i < n && !big && nb >= PH_MID;
-    const bool small = i < n && nb < PH_MID;
-    const int kb = sxw_place(&cnt[0], big), km = sxw_place(&cnt[1], mid);
-    const int ks = sxw_place(&cnt[2], small);
-    if (big) order[kb] = i;
-    if (mid) order[n + km] = i;
-    if (small) order[n - 1 - ks] = i;
+    const int cls = i >= n ? -1 : nb >= PH_BIG ? 0 : nb >= PH_MID ? 1 : 2;
+    const int k = sxw_place<3>(cnt, cls);
+    if (cls >= 0) order[cls == 0 ? k : cls == 1 ? n + k : n - 1 - k] = i;
 }
 
 template <SxwSize Z> __device__ void phot_object(const PhotArgs &A, int obj, double *rows)
