@@ -164,11 +164,19 @@ __global__ void k_plan_end(const PlanDev *pd, PlanRecord *rec)
     rec->t1 = wall_clock64();
 }
 
-/* resets the context's planned-run state when the frame's queueing ends, however it ends */
+/* resets the context's whole-frame state when the frame's queueing ends, however it ends */
 struct PlanScope {
     SxgState &S;
-    explicit PlanScope(SxgState &s, const FramePlan *plan) : S(s) { S.plan = plan; }
-    ~PlanScope() { S.plan = nullptr; }
+    explicit PlanScope(SxgState &s, const FramePlan *plan) : S(s)
+    {
+        S.plan = plan;
+        S.in_frame = true;
+    }
+    ~PlanScope()
+    {
+        S.plan = nullptr;
+        S.in_frame = false;
+    }
 };
 
 /* The whole path on a device frame (not modified), on the current context.  plan: a

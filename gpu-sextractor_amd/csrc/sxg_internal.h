@@ -269,6 +269,8 @@ struct SxgState {
     unsigned *mail = nullptr;              /* pinned page of sxg_read_back: [0] the sequence
                                               number, [16..] the words */
     unsigned mail_seq = 0;
+    bool exposed = false;                  /* sxg_device_frame handed out the frame's planes */
+    bool in_frame = false;                 /* inside a whole-frame run, which waits at its end */
     /* MAP_WEIGHT map (sxg_set_weight) */
     DevBuf weight;
     int ww = 0, wh = 0;
@@ -316,8 +318,9 @@ SxgState *sxg_bound_state();
 void sxg_bind_state(SxgState *s);
 /* End of an entry point without a host output: the contexts of the batch workers
    (several sharing the device) wait for their stream there, which interleaves their
-   kernels on the hardware queues; every other context returns at once and keeps its
-   queue full. */
+   kernels on the hardware queues; so do the contexts that callers create once they have
+   asked for device pointers, outside the whole-frame runs.  Every other context returns
+   at once and keeps its queue full. */
 bool sxg_stage_wait();
 /* The host's copy of a few device words that the work queued on the context's stream
    leaves behind (at most SXG_MAIL_WORDS together): a kernel writes them into the

@@ -207,7 +207,7 @@ extern "C" int sxg_stage_times(float *ms, int n)
 bool sxg_stage_wait()
 {
     SxgState &S = sxg_state();
-    if (!S.single_stream || S.plan) return true;
+    if (S.plan || (!S.single_stream && (S.is_default || S.in_frame || !S.exposed))) return true;
     SXG_HIP_RET(hipStreamSynchronize(S.stream), false);
     return true;
 }
@@ -285,7 +285,7 @@ extern "C" void sxg_release(void)
                       &S.comps, &S.objs, &S.rootobj};
     for (DevBuf *b : bufs) b->release();
     sxg_release_named();
-    S.ranked = S.counted = false;
+    S.ranked = S.counted = S.exposed = false;
     if (S.mail) (void)hipHostFree(S.mail);
     S.mail = nullptr;
     S.dmask.release();
@@ -669,6 +669,10 @@ extern "C" void *sxg_device_frame(int which)
 {
     SxgState &S = sxg_state();
     if (!S.have_frame) return nullptr;
+    /* the caller reads the planes on a stream of its own: what is queued is finished here,
+       and from now on at the end of the entry points (sxg_stage_wait) */
+    S.exposed = true;
+    if (S.stream) SXG_HIP_RET(hipStreamSynchronize(S.stream), nullptr);
     return which == 0 ? S.img.ptr : S.cd.ptr;
 }
 
