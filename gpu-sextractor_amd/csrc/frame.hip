@@ -112,6 +112,9 @@ extern "C" int sxg_set_resident_frame(const float *host, int width, int height)
         return -1;
     }
     const size_t n = (size_t)width * height;
+    /* a run that failed half-way leaves kernels queued that read the present frame, and
+       hipMemcpy does not wait for a non-blocking stream */
+    if (S.stream) SXG_HIP_RET(hipStreamSynchronize(S.stream), -1);
     if (!S.resident.ensure(n * sizeof(float))) return -1;
     SXG_HIP_RET(hipMemcpy(S.resident.ptr, host, n * sizeof(float), hipMemcpyHostToDevice), -1);
     S.rw = width;

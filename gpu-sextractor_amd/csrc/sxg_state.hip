@@ -710,6 +710,9 @@ extern "C" int sxg_set_weight_map(const float *map, int width, int height, int t
         return -1;
     }
     S.wrms_frame = false;
+    /* kernels that read the present map may still be queued (analyse_gpu, run_clean without a
+       host output), and neither hipMemcpy nor hipFree waits for a non-blocking stream */
+    if (S.stream) SXG_HIP_RET(hipStreamSynchronize(S.stream), -1);
     if (!map && type != SXG_WEIGHT_BACKGROUND) {
         S.weighted = false;
         S.weight.release();

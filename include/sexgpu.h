@@ -7,7 +7,10 @@
  * library instead.  Semantics follow the reference:
  *   - a stateful singleton: width, height and every device buffer live in the library;
  *     one frame at a time, calls in the order listed; not re-entrant, not thread-safe;
- *   - every call returns synchronously;
+ *   - a call returns when its host outputs are written and its host inputs are free again;
+ *     the kernels of a call without host outputs may still be queued then, ahead of what the
+ *     next calls queue on the context's stream, so every call sees the results of the calls
+ *     before it (sxg_sync waits for them; sxg_device_frame says what holds for its pointers);
  *   - the library owns device memory; init_device copies the caller's frame in and
  *     clear_device overwrites the caller's buffer with the background-subtracted frame;
  *   - run_clean fills the caller's masterIndex[numobj] (0xffffffff = kept).
