@@ -1539,6 +1539,8 @@ void sxg_back_estimate_from(const float *src, int back_size, float backfthresh, 
     }
     sxg_stage_end(ST_BACK);
     SXG_HIP(hipGetLastError());
+    /* the medians were polled for; planes by device pointer need the stream run dry */
+    if (S.exposed && !sxg_stage_wait()) return;
     if (backmean) *backmean = S.backmean;
     if (backsig) *backsig = S.backsig;
 }

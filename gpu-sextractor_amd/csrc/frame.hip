@@ -291,6 +291,9 @@ static int process_frame(const float *dframe, int W, int H, const sxg_params *p,
         SXG_HIP_RET(hipGetLastError(), -1);
         return 0;
     }
+    /* the wait at the end of the run came with the survivors' count; a frame without
+       objects has none to read */
+    if (nobj == 0) SXG_HIP_RET(hipStreamSynchronize(S.stream), -1);
     if (info) sxg_get_frame_info(info);
     return nobj;
 }

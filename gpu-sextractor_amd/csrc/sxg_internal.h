@@ -316,11 +316,11 @@ SxgState &sxg_state();
 /* the state bound to the calling thread (nullptr: the default context), and rebinding it */
 SxgState *sxg_bound_state();
 void sxg_bind_state(SxgState *s);
-/* End of an entry point without a host output: the contexts of the batch workers
-   (several sharing the device) wait for their stream there, which interleaves their
-   kernels on the hardware queues; so do the contexts that callers create once they have
-   asked for device pointers, outside the whole-frame runs.  Every other context returns
-   at once and keeps its queue full. */
+/* End of an entry point whose kernels may still be queued: the contexts of the batch
+   workers (several sharing the device) wait for their stream there, which interleaves their
+   kernels on the hardware queues; so does, outside the whole-frame runs, every context whose
+   planes the caller has by device pointer.  Every other context returns at once and keeps
+   its queue full. */
 bool sxg_stage_wait();
 /* The host's copy of a few device words that the work queued on the context's stream
    leaves behind (at most SXG_MAIL_WORDS together): a kernel writes them into the

@@ -207,7 +207,7 @@ extern "C" int sxg_stage_times(float *ms, int n)
 bool sxg_stage_wait()
 {
     SxgState &S = sxg_state();
-    if (S.plan || (!S.single_stream && (S.is_default || S.in_frame || !S.exposed))) return true;
+    if (S.plan || (!S.single_stream && (S.in_frame || !S.exposed))) return true;
     SXG_HIP_RET(hipStreamSynchronize(S.stream), false);
     return true;
 }
@@ -670,7 +670,8 @@ extern "C" void *sxg_device_frame(int which)
     SxgState &S = sxg_state();
     if (!S.have_frame) return nullptr;
     /* the caller reads the planes on a stream of its own: what is queued is finished here,
-       and from now on at the end of the entry points (sxg_stage_wait) */
+       and from now on at the end of every entry point, in the default context too
+       (sxg_stage_wait; a whole-frame run waits once, at its end) */
     S.exposed = true;
     if (S.stream) SXG_HIP_RET(hipStreamSynchronize(S.stream), nullptr);
     return which == 0 ? S.img.ptr : S.cd.ptr;

@@ -278,7 +278,9 @@ int sxg_get_filtered(float *out);
 int sxg_get_alloc_map(int32_t *out);
 
 /* Device pointers of the resident frame (for callers that keep data on the GPU):
-   background-subtracted frame and filtered frame.  Valid until clear_device. */
+   background-subtracted frame and filtered frame.  Valid until clear_device.  Once they
+   have been asked for, the entry points of the context return with their kernels finished,
+   so that the planes can be read on any stream. */
 void *sxg_device_frame(int which);
 
 /* Timing of the last frame's stages in milliseconds (HIP events): background, filter,
