@@ -84,6 +84,11 @@ __device__ inline void meshstat_pass2_end(const MeshAcc &a, MeshStat &o)
 }
 
 #define MS_LDS_BYTES (144 * 1024)
+/* larger meshes than the LDS: pixels in LDS at a time (a multiple of four) */
+#ifndef MS_PART
+#define MS_PART 16384
+#define MS_PARTW 4
+#endif
 /* the largest mesh (pixels) of the one-, two- and four-wavefront kernels */
 #define MS_PX1 2048
 #define MS_PX2 8192
@@ -109,25 +114,36 @@ __device__ inline void meshstat_pass2_end(const MeshAcc &a, MeshStat &o)
  *     is y2 plus the next run's y1, a multiple of u/2 below 2^52 u: a run costs the walk
  *     one dependent add.
  *   - |A - S| <= 2 n 2^-53 sum|x| (the rounding of two recursive sums, Higham, Accuracy and
- *     Stability of Numerical Algorithms, 2nd ed., eq. 4.4); the run's bounds are widened by
- *     delta = 8 times n 2^-53 sum|x|, and a run whose bounds do not lie in one binade, or are
- *     not finite, zero or subnormal, is flagged: its pixels are added one by one.  A sum of
- *     positive terms crosses log2(runs) + 1 binades after its first run, so few runs are.
+ *     Stability of Numerical Algorithms, 2nd ed., eq. 4.4); the run's bounds, A plus its lowest
+ *     and its highest partial sum, are widened by delta = 8 times n 2^-53 sum|x|, and a run
+ *     whose bounds do not lie in one binade, or are not finite, zero or subnormal, is flagged:
+ *     its pixels are added one by one.  A sum of positive terms crosses log2(runs) + 1 binades
+ *     after its first run, so few runs are; the sum of pix over a frame whose sky has been
+ *     subtracted stays within a few runs' reach of zero, and there up to a third of them are.
  *   - Where sum|pix| <= 2^53 times the unit of the smallest pixel's last bit, every partial
  *     sum is a multiple of that unit that a double holds: the order does not matter and the
  *     sum of pix is taken in any (true of almost all frames).
  *
  * The mesh sits in LDS between the two passes (run t at t*KS, KS a multiple of four floats
  * and KS/4 odd: a lane's float4 reads are conflict-free), so the frame is read once; the
- * runs' places past the last pixel hold NaN, which no pass takes.  G: a
- * mesh that does not fit stays in global memory.  One workgroup of NW wavefronts per mesh;
- * wavefront 0 walks the runs' increments.
+ * runs' places past the last pixel hold NaN, which no pass takes.  G: a mesh that does not fit
+ * goes through LDS in parts of MS_PART pixels, in both passes; each part starts from the sums
+ * that the one before left (A from S itself, |S| beside sum|x| in the bounds).  One workgroup of
+ * NW wavefronts per mesh; wavefront 0 walks the runs' increments.
  *
  * Bound: VALU instructions (about 20 a pixel and pass), then the walk (3 us a pass at two
  * wavefronts).  A 64 x 64 mesh takes 12 us; measured against the sequential chains fed from
  * an LDS ring (8,192 dependent adds a mesh): 1024^2 105 -> 15 us, 4096^2 119 -> 63 us (256
  * CUs, 16 meshes each, seven at a time by LDS), 2011 x 1533 (rows not aligned) 343 -> 21 us,
  * 8192 x 4096 with weights and 128 x 128 meshes 806 -> 140 us.
+ * Frames of zero mean are the slow ones (the whole background, in us, by chains, with bounds
+ * from the run's positive and negative parts and 16 pixels read at a time, and now): meshes of
+ * 64 at 512^2 171, 180, 140; of 96 at 1024^2 288, 315, 194; meshes beyond the LDS, which lanes
+ * read from global memory at a run's stride, of 256 at 4096^2 2,022, 3,317, 525 (with a sky of
+ * 200 sigma 2,020, 1,110, 228), of 1024 17,838, 41,082, 3,405.  Parts of 8,192 pixels and two
+ * wavefronts, 16,384 and four, 16,384 and eight, 32,768 and eight: meshes of 256 at 4096^2 266,
+ * 228, 222, 218 with a sky, 537, 525, 594, 535 without; of 192 at 8192^2 600, 640, 775, 782 and
+ * 787, 914, 1,294, 1,447; of 512 at 4096^2 629, 457, 450, 402 and 1,331, 1,502, 1,714, 1,409.
  */
 __host__ __device__ inline int ms_run(int npx, int runs)   /* pixels of a run: K */
 {
@@ -155,26 +171,31 @@ __global__ void __launch_bounds__(64 * NW) k_meshstat(const float *__restrict__ 
     __shared__ float s_fa[NW];
     __shared__ unsigned s_min[NW];
     __shared__ int s_cnt[NW];
-    __shared__ double s_res;
+    __shared__ double s_sum, s_sum2;         /* G: the sequential sums so far */
     __shared__ float s_cut[2];
     __shared__ int s_bad;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int m = blockIdx.x, x0 = (m % nbx) * bs, y0 = (m / nbx) * bs;
-    const int bw = min(bs, W - x0), bh = min(bs, H - y0), npx = bw * bh;
-    const int K = ms_run(npx, R), KS = ms_stride(K);
-    const int len = min(max(npx - tid * K, 0), K);      /* pixels of this lane's run */
+    const int bw = min(bs, W - x0), bh = min(bs, H - y0), mesh = bw * bh;
+    /* the pixels in LDS: all of the mesh, or a part at a time */
+    const int part = G ? MS_PART : mesh;
+    const int K = ms_run(part, R), KS = ms_stride(K);
     const float big = (float)-SXG_BIG;
     const float *const base = img + (size_t)y0 * W + x0;
     const float *const wbase = wmap ? wmap + (size_t)y0 * W + x0 : nullptr;
-    /* pixels of non-positive weight are left out: -BIG */
-    auto weigh = [&](float v, size_t o) { return wmap && !(wbase[o] > 0.0f) ? big : v; };
-    if constexpr (!G) {
-        /* pixel i of the mesh at i + (i / K) * (KS - K) */
-        const unsigned mk = 0xffffffffu / (unsigned)K + 1u;   /* i / K, i*K < 2^32 */
+    const unsigned mk = 0xffffffffu / (unsigned)K + 1u;   /* i / K, i*K < 2^32 */
+    /* pixels p0 .. p0 + npx - 1 of the mesh into LDS, pixel i of them at i + (i / K) * (KS - K),
+       those of non-positive weight as -BIG */
+    auto load = [&](int p0, int npx) {
+        const int ys = G ? p0 / bw : 0, xs = G ? p0 - ys * bw : 0;
+        const float *const src = base + (size_t)ys * W;
+        const float *const wsrc = wmap ? wbase + (size_t)ys * W : nullptr;
+        /* a row longer than a part is left at most once (and i*bw may pass 2^32) */
+        const bool longrow = G && bw >= MS_PART;
         const int pad = KS - K;
         if (((bw | W | bs) & 3) == 0) {
             constexpr int U = 8;
-            const int q4 = bw >> 2, tot = q4 * bh;
+            const int q4 = bw >> 2, x4 = xs >> 2, tot = npx >> 2;
             const unsigned mq = 0xffffffffu / (unsigned)q4 + 1u;
             for (int e0 = tid; e0 < tot; e0 += U * R) {
                 float4 v[U];
@@ -182,10 +203,10 @@ __global__ void __launch_bounds__(64 * NW) k_meshstat(const float *__restrict__ 
                 int at[U];
 #pragma unroll
                 for (int u = 0; u < U; u++) {
-                    const int e = min(e0 + u * R, tot - 1);
-                    const int y = q4 == 1 ? e : (int)__umulhi((unsigned)e, mq);
-                    const size_t o = (size_t)y * W + 4 * (e - y * q4);
-                    v[u] = *reinterpret_cast<const float4 *>(base + o);
+                    const int e = min(e0 + u * R, tot - 1), i = e + x4;
+                    const int y = longrow ? i >= q4 : q4 == 1 ? i : (int)__umulhi((unsigned)i, mq);
+                    const size_t o = (size_t)y * W + 4 * (i - y * q4);
+                    v[u] = *reinterpret_cast<const float4 *>(src + o);
                     of[u] = o;
                     at[u] = 4 * e + (int)__umulhi(4u * e, mk) * pad;
                 }
@@ -193,7 +214,7 @@ __global__ void __launch_bounds__(64 * NW) k_meshstat(const float *__restrict__ 
                     float4 wv[U];
 #pragma unroll
                     for (int u = 0; u < U; u++)
-                        wv[u] = *reinterpret_cast<const float4 *>(wbase + of[u]);
+                        wv[u] = *reinterpret_cast<const float4 *>(wsrc + of[u]);
 #pragma unroll
                     for (int u = 0; u < U; u++) {
                         if (!(wv[u].x > 0.0f)) v[u].x = big;
@@ -214,15 +235,15 @@ __global__ void __launch_bounds__(64 * NW) k_meshstat(const float *__restrict__ 
                 size_t of[U];
 #pragma unroll
                 for (int u = 0; u < U; u++) {
-                    const int e = min(e0 + u * R, npx - 1);
-                    const int y = bw == 1 ? e : (int)__umulhi((unsigned)e, mw);
-                    of[u] = (size_t)y * W + (e - y * bw);
-                    v[u] = base[of[u]];
+                    const int i = min(e0 + u * R, npx - 1) + xs;
+                    const int y = longrow ? i >= bw : bw == 1 ? i : (int)__umulhi((unsigned)i, mw);
+                    of[u] = (size_t)y * W + (i - y * bw);
+                    v[u] = src[of[u]];
                 }
                 if (wmap) {
                     float wv[U];
 #pragma unroll
-                    for (int u = 0; u < U; u++) wv[u] = wbase[of[u]];
+                    for (int u = 0; u < U; u++) wv[u] = wsrc[of[u]];
 #pragma unroll
                     for (int u = 0; u < U; u++)
                         if (!(wv[u] > 0.0f)) v[u] = big;
@@ -237,18 +258,8 @@ __global__ void __launch_bounds__(64 * NW) k_meshstat(const float *__restrict__ 
         for (int i = npx + tid; i < R * K; i += R)
             px[i + (int)__umulhi((unsigned)i, mk) * pad] = NAN;
         __syncthreads();
-    }
-    /* pixel j of run t (NaN past the mesh's last pixel) */
-    auto pix1 = [&](int t, int j) -> float {
-        const int i = t * K + j;
-        if (i >= npx) return NAN;
-        if constexpr (G) {
-            const size_t o = (size_t)(i / bw) * W + i % bw;
-            return weigh(base[o], o);
-        } else {
-            return px[t * KS + j];
-        }
     };
+    if constexpr (!G) load(0, mesh);
     /* the pixels that take part: those above -BIG, then those between the cuts */
     float lcut = ord2f(f2ord(big) + 1), hcut = INFINITY;
     auto sel = [&](float v, bool &in) {
@@ -257,182 +268,185 @@ __global__ void __launch_bounds__(64 * NW) k_meshstat(const float *__restrict__ 
     };
     /* f(the pixel or 0, takes part) over this lane's run */
     auto each = [&](auto f) {
-        if constexpr (G) {
-            int y = (tid * K) / bw, x = tid * K - y * bw;
-            for (int j = 0; j < len; j++) {
-                const size_t ofs = (size_t)y * W + x;
-                bool in;
-                const float q = sel(weigh(base[ofs], ofs), in);
-                f(q, in);
-                if (++x == bw) {
-                    x = 0;
-                    y++;
-                }
-            }
-        } else {
-            const float4 *rp = reinterpret_cast<const float4 *>(px + tid * KS);
+        const float4 *rp = reinterpret_cast<const float4 *>(px + tid * KS);
 #pragma unroll 4
-            for (int j = 0; j < K; j += 4) {
-                const float4 v = rp[j >> 2];
-                bool i0, i1, i2, i3;
-                const float q0 = sel(v.x, i0), q1 = sel(v.y, i1), q2 = sel(v.z, i2),
-                            q3 = sel(v.w, i3);
-                f(q0, i0);
-                f(q1, i1);
-                f(q2, i2);
-                f(q3, i3);
-            }
+        for (int j = 0; j < K; j += 4) {
+            const float4 v = rp[j >> 2];
+            bool i0, i1, i2, i3;
+            const float q0 = sel(v.x, i0), q1 = sel(v.y, i1), q2 = sel(v.z, i2),
+                        q3 = sel(v.w, i3);
+            f(q0, i0);
+            f(q1, i1);
+            f(q2, i2);
+            f(q3, i3);
         }
     };
     MeshStat o;
     for (int pass = 0; pass < 2; pass++) {
-        double s1 = 0.0, s2 = 0.0;
-        float fa = 0.0f;
-        /* bits of the smallest non-zero |pixel|, twice, less one */
-        unsigned um = 0xffffffffu;
-        int cnt = 0;
-        each([&](float q, bool in) {
-            const double p = q;
-            s1 += p;
-            s2 += p * p;
-            fa += fabsf(q);
-            um = min(um, 2u * (unsigned)__float_as_int(q) - 1u);
-            cnt += in;
-        });
-        const int mycnt = cnt;
-        double x2 = s2;                /* inclusive prefix in the wavefront */
-        for (int d = 1; d < 64; d <<= 1) {
-            const double t = __shfl_up(x2, d);
-            if (lane >= d) x2 += t;
-            s1 += __shfl_xor(s1, d);
-            fa += __shfl_xor(fa, d);
-        }
-        cnt = sxw_sum(cnt);
-        um = (unsigned)sxw_min((int)(um ^ 0x80000000u)) ^ 0x80000000u;
-        if (lane == 63) {
-            s_s1[wid] = s1;
-            s_s2[wid] = x2;
-            s_fa[wid] = fa;
-            s_min[wid] = um;
-            s_cnt[wid] = cnt;
-        }
-        __syncthreads();
-        double t1 = 0.0, t2 = 0.0, b2 = 0.0;
-        fa = 0.0f;
-        cnt = 0;
+        MeshAcc a;                     /* a.mean, a.sigma: the sums of pix and of pix*pix */
+        unsigned um = 0xffffffffu;     /* bits of the smallest non-zero |pixel|, twice, less one */
+        for (int left = mesh; left > 0; left -= min(left, part)) {
+            const int p0 = mesh - left, npx = min(left, part);
+            if constexpr (G) load(p0, npx);
+            double s1 = 0.0, s2 = 0.0;
+            float fa = 0.0f;
+            int cnt = 0;
+            each([&](float q, bool in) {
+                const double p = q;
+                s1 += p;
+                s2 += p * p;
+                fa += fabsf(q);
+                um = min(um, 2u * (unsigned)__float_as_int(q) - 1u);
+                cnt += in;
+            });
+            const int mycnt = cnt;
+            double x2 = s2;                /* inclusive prefix in the wavefront */
+            for (int d = 1; d < 64; d <<= 1) {
+                const double t = __shfl_up(x2, d);
+                if (lane >= d) x2 += t;
+                s1 += __shfl_xor(s1, d);
+                fa += __shfl_xor(fa, d);
+            }
+            cnt = sxw_sum(cnt);
+            um = (unsigned)sxw_min((int)(um ^ 0x80000000u)) ^ 0x80000000u;
+            if (lane == 63) {
+                s_s1[wid] = s1;
+                s_s2[wid] = x2;
+                s_fa[wid] = fa;
+                s_min[wid] = um;
+                s_cnt[wid] = cnt;
+            }
+            __syncthreads();
+            double t1 = 0.0, t2 = 0.0, b2 = 0.0;
+            fa = 0.0f;
 #pragma unroll
-        for (int w = 0; w < NW; w++) {
-            if (w == wid) b2 = t2;
-            t1 += s_s1[w];
-            t2 += s_s2[w];
-            fa += s_fa[w];
-            um = min(um, s_min[w]);
-            cnt += s_cnt[w];
-        }
-        /* wavefront 0: the sequential sum from the runs' increments, sixteen runs at a time
-           (the rows of the wavefront do the same); term: the summand of a pixel */
-        auto walk = [&](auto term) {
-            const int l16 = lane & 15;
-            double S = 0.0;
-#pragma unroll 1
             for (int w = 0; w < NW; w++) {
-                const unsigned long long f = s_flag[w];
-                const unsigned flo = (unsigned)__builtin_amdgcn_readfirstlane((int)f);
-                const unsigned fhi = (unsigned)__builtin_amdgcn_readfirstlane((int)(f >> 32));
-                double z[4];
-#pragma unroll
-                for (int g = 0; g < 4; g++)
-                    z[g] = s_y1[w * 64 + g * 16 + l16] + s_y2[w * 64 + g * 16 + l16];
-#pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    const int t0 = w * 64 + g * 16;
-                    unsigned fl = ((g < 2 ? flo : fhi) >> (16 * (g & 1))) & 0xffffu;
-                    int done = 0;      /* runs of the sixteen in S */
+                if (w == wid) b2 = t2;
+                t1 += s_s1[w];
+                t2 += s_s2[w];
+                fa += s_fa[w];
+                um = min(um, s_min[w]);
+                a.npix += s_cnt[w];
+            }
+            /* wavefront 0: the sequential sum from S on, from the runs' increments, sixteen
+               runs at a time (the rows of the wavefront do the same); term: the summand of a
+               pixel */
+            auto walk = [&](double S, auto term) {
+                const int l16 = lane & 15;
 #pragma unroll 1
-                    while (fl) {
-                        /* up to the next flagged run (its y1, y2 are 0), then its pixels
-                           one by one */
-                        const int r = __builtin_ctz(fl);
-                        fl &= fl - 1;
-                        S = sxw_row_fold(S, l16 >= done && l16 <= r ? z[g] : 0.0);
-                        for (int j = 0; j < K; j += 16) {
-                            bool in;
-                            const float v = j + l16 < K ? pix1(t0 + r, j + l16) : NAN;
-                            S = sxw_row_fold(S, term((double)sel(v, in)));
+                for (int w = 0; w < NW; w++) {
+                    const unsigned long long f = s_flag[w];
+                    const unsigned flo = (unsigned)__builtin_amdgcn_readfirstlane((int)f);
+                    const unsigned fhi = (unsigned)__builtin_amdgcn_readfirstlane((int)(f >> 32));
+                    double z[4];
+#pragma unroll
+                    for (int g = 0; g < 4; g++)
+                        z[g] = s_y1[w * 64 + g * 16 + l16] + s_y2[w * 64 + g * 16 + l16];
+#pragma unroll
+                    for (int g = 0; g < 4; g++) {
+                        const float *const rows = px + (w * 64 + g * 16) * KS;
+                        unsigned fl = ((g < 2 ? flo : fhi) >> (16 * (g & 1))) & 0xffffu;
+                        int done = 0;      /* runs of the sixteen in S */
+#pragma unroll 1
+                        while (fl) {
+                            /* up to the next flagged run (its y1, y2 are 0, and there is nothing
+                               between two that follow each other), then its pixels one by one,
+                               64 read at a time, a row of lanes each sixteen */
+                            const int r = __builtin_ctz(fl);
+                            fl &= fl - 1;
+                            if (done == 0 || r > done)
+                                S = sxw_row_fold(S, l16 >= done && l16 <= r ? z[g] : 0.0);
+                            done = r + 1;
+                            for (int j = 0; j < K; j += 64) {
+                                bool in;
+                                const float v = j + lane < K ? rows[r * KS + j + lane] : NAN;
+                                const double x = term((double)sel(v, in));
+#pragma unroll
+                                for (int c = 0; c < 4; c++)
+                                    if (j + 16 * c < K) S = sxw_rl(sxw_row_fold(S, x), 16 * c);
+                            }
                         }
-                        done = r + 1;
+                        S = sxw_row_fold(S, l16 >= done ? z[g] : 0.0);
                     }
-                    S = sxw_row_fold(S, l16 >= done ? z[g] : 0.0);
+                }
+                return S + s_y2[R];
+            };
+            /* every lane: its run's increments and flag.  A: the prefix before the run, A + lo,
+               A + hi: its lowest and highest partial sum, abs: |S| and sum|x| of what is in
+               LDS */
+            auto increments = [&](double A, double lo, double hi, double abs, auto term) {
+                const double delta = abs * (double)npx * 0x1p-50;
+                const bool flag = mycnt > 0 && !ms_binade(A + lo - delta, A + hi + delta);
+                double y1 = 0.0, y2 = 0.0;
+                if (mycnt > 0 && !flag) {
+                    const double B0 = __hiloint2double(__double2hiint(A), __double2loint(A) & ~1);
+                    const double B1 = __hiloint2double(__double2hiint(A), __double2loint(A) | 1);
+                    double a0 = B0, a1 = B1;
+                    each([&](float q, bool) {
+                        const double x = term((double)q);
+                        a0 += x;
+                        a1 += x;
+                    });
+                    const double d0 = a0 - B0, d1 = a1 - B1;
+                    const bool odd = d0 != d1 && (__double2loint(a0) & 1);
+                    y2 = odd ? B1 - B0 : 0.0;
+                    y1 = (d0 + d1) * 0.5 - y2;
+                }
+                s_y1[tid] = y1;
+                s_y2[tid + 1] = y2;
+                if (tid == 0) s_y2[0] = 0.0;
+                const unsigned long long b = __ballot(flag);
+                if (lane == 0) s_flag[wid] = b;
+            };
+            auto square = [](double p) { return p * p; };
+            auto same = [](double p) { return p; };
+            increments(a.sigma + b2 + x2 - s2, 0.0, s2, a.sigma + t2, square);
+            __syncthreads();
+            /* the unit of the last mantissa bit of the smallest pixel so far, of which the sum
+               so far is a multiple too */
+            const int ue = max((int)((um + 1u) >> 24), 1) - 150;
+            /* above |S| + sum|pix| */
+            const double abs1 = fabs(a.mean) * 1.001 + (double)fa * (1.001 + K * 0x1p-22);
+            const bool any = um == 0xffffffffu || abs1 <= ldexp(1.0, 53 + ue);
+            if (wid == 0) {
+                a.sigma = walk(a.sigma, square);
+                if (G && lane == 0) s_sum2 = a.sigma;
+            }
+            if (any) {
+                a.mean += t1;
+            } else {
+                /* the sum of pix along its order too: its prefix, and how far it goes either
+                   way */
+                __syncthreads();
+                double xs = 0.0, lo = 0.0, hi = 0.0;
+                each([&](float q, bool) {
+                    xs += (double)q;
+                    lo = fmin(lo, xs);
+                    hi = fmax(hi, xs);
+                });
+                const double own = xs;
+                for (int d = 1; d < 64; d <<= 1) {
+                    const double t = __shfl_up(xs, d);
+                    if (lane >= d) xs += t;
+                }
+                if (lane == 63) s_s1[wid] = xs;
+                __syncthreads();
+                double before = 0.0;
+#pragma unroll
+                for (int w = 0; w < NW; w++)
+                    if (w < wid) before += s_s1[w];
+                increments(a.mean + before + xs - own, lo, hi, abs1, same);
+                __syncthreads();
+                if (wid == 0) {
+                    a.mean = walk(a.mean, same);
+                    if (G && lane == 0) s_sum = a.mean;
                 }
             }
-            return S + s_y2[R];
-        };
-        /* every lane: its run's increments and flag.  A: the prefix before the run, [A -
-           neg, A + pos]: what the run can reach, abs: sum|x| of the mesh */
-        auto increments = [&](double A, double neg, double pos, double abs, auto term) {
-            const double delta = abs * (double)npx * 0x1p-50;
-            const bool flag = mycnt > 0 && !ms_binade(A - neg - delta, A + pos + delta);
-            double y1 = 0.0, y2 = 0.0;
-            if (mycnt > 0 && !flag) {
-                const double B0 = __hiloint2double(__double2hiint(A), __double2loint(A) & ~1);
-                const double B1 = __hiloint2double(__double2hiint(A), __double2loint(A) | 1);
-                double a0 = B0, a1 = B1;
-                each([&](float q, bool) {
-                    const double x = term((double)q);
-                    a0 += x;
-                    a1 += x;
-                });
-                const double d0 = a0 - B0, d1 = a1 - B1;
-                const bool odd = d0 != d1 && (__double2loint(a0) & 1);
-                y2 = odd ? B1 - B0 : 0.0;
-                y1 = (d0 + d1) * 0.5 - y2;
+            if constexpr (G) {
+                __syncthreads();
+                a.sigma = s_sum2;
+                if (!any) a.mean = s_sum;
             }
-            s_y1[tid] = y1;
-            s_y2[tid + 1] = y2;
-            if (tid == 0) s_y2[0] = 0.0;
-            const unsigned long long b = __ballot(flag);
-            if (lane == 0) s_flag[wid] = b;
-        };
-        auto square = [](double p) { return p * p; };
-        auto same = [](double p) { return p; };
-        increments(b2 + x2 - s2, 0.0, s2, t2, square);
-        __syncthreads();
-        /* the unit of the last mantissa bit of the smallest pixel */
-        const int ue = max((int)((um + 1u) >> 24), 1) - 150;
-        const bool any = um == 0xffffffffu || (double)fa * (1.001 + K * 0x1p-22) <= ldexp(1.0, 53 + ue);
-        MeshAcc a;
-        a.npix = cnt;
-        a.mean = t1;
-        if (wid == 0) a.sigma = walk(square);
-        if (!any) {
-            /* the sum of pix along its order too: prefix, and the parts of either sign */
-            __syncthreads();
-            double ps = 0.0, ng = 0.0;
-            each([&](float q, bool) {
-                ps += q > 0.0f ? (double)q : 0.0;
-                ng += q < 0.0f ? -(double)q : 0.0;
-            });
-            double xs = ps - ng, ab = ps + ng;
-            const double own = xs;
-            for (int d = 1; d < 64; d <<= 1) {
-                const double t = __shfl_up(xs, d);
-                if (lane >= d) xs += t;
-                ab += __shfl_xor(ab, d);
-            }
-            if (lane == 63) {
-                s_s1[wid] = xs;
-                s_s2[wid] = ab;
-            }
-            __syncthreads();
-            double before = 0.0, tab = 0.0;
-#pragma unroll
-            for (int w = 0; w < NW; w++) {
-                if (w < wid) before += s_s1[w];
-                tab += s_s2[w];
-            }
-            increments(before + xs - own, ng, ps, tab, same);
-            __syncthreads();
-            if (wid == 0) a.mean = walk(same);
         }
         if (tid == 0) {
             if (pass == 0) {
@@ -1340,7 +1354,7 @@ bool sxg_back_run(const BackGeom &g, const BackBufs &b, const float *src, float 
         /* wavefronts per mesh by its pixels: runs of 16 to 80 pixels.  Longer ones cost the
            flagged runs' one-by-one adds, shorter ones the walk.  Measured at 4096^2: meshes
            of 64 with 1, 2, 4 wavefronts 74, 63, 76 us, meshes of 128 with 2, 4, 8
-           wavefronts 92, 69, 93 us.  A mesh beyond the LDS stays in global memory */
+           wavefronts 92, 69, 93 us.  A mesh beyond the LDS goes through it in parts */
         const long px = (long)std::min(bs, W) * std::min(bs, H);
         auto bytes = [&](int nw) {
             return sizeof(float) * 64 * (size_t)nw * ms_stride(ms_run((int)px, 64 * nw));
@@ -1353,6 +1367,9 @@ bool sxg_back_run(const BackGeom &g, const BackBufs &b, const float *src, float 
            launch asks for */
         static const bool attr =
             hipFuncSetAttribute(reinterpret_cast<const void *>(&k_meshstat<4, false>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                MS_LDS_BYTES) == hipSuccess &&
+            hipFuncSetAttribute(reinterpret_cast<const void *>(&k_meshstat<MS_PARTW, true>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize,
                                 MS_LDS_BYTES) == hipSuccess &&
             hipFuncSetAttribute(reinterpret_cast<const void *>(&k_meshstat<8, false>),
@@ -1371,7 +1388,8 @@ bool sxg_back_run(const BackGeom &g, const BackBufs &b, const float *src, float 
         else if (bytes(8) <= MS_LDS_BYTES)
             launch(&k_meshstat<8, false>, 8, bytes(8));
         else
-            launch(&k_meshstat<16, true>, 16, 0);
+            launch(&k_meshstat<MS_PARTW, true>, MS_PARTW,
+                   sizeof(float) * 64 * MS_PARTW * ms_stride(ms_run(MS_PART, 64 * MS_PARTW)));
     }
     if (timed) sxg_kt_end(SXG_KT_MESHSTAT);
     if (timed) sxg_kt_begin(SXG_KT_MESHMODE);
