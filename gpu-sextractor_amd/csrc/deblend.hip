@@ -49,7 +49,9 @@
  *                    component tree as a max-tree (see deb_tree)
  *   k_deb_order      the objects too large for that, largest first
  *   k_deb_tree_glb   the same code for them, with only the parent words and level indices in
- *                    LDS, or none of it
+ *                    LDS
+ *   k_deb_wide_*     the same passes over the pixels of the objects above 29,696 pixels, a
+ *                    kernel each, all state in global memory
  *   k_deb_objlist    one wavefront per raw object: its kept nodes -> objects
  *   k_deb_pre        one wavefront per object: FULL preanalysis over the node's level
  *                    pixels (kcomp names them; lanes compute the terms, the raster-order
@@ -66,8 +68,15 @@
 #include "sxg_wave.h"
 
 #define DW 64
-/* words of the per-frame counter block (DebArgs::ccount) */
-#define DEB_NCOUNT 11
+/* size classes of the raw objects with a tree (k_deb_classify), and the words of the
+   per-frame counter block (DebArgs::ccount): objects per class, the largest LDS need of
+   classes 0..2, pixels per class (3 and 4 together) */
+#define DEB_NCLASS 5
+#define DEB_CLDS DEB_NCLASS
+#define DEB_CPIX (DEB_CLDS + 3)
+#define DEB_NCOUNT (DEB_CPIX + 4)
+/* pixels of the largest tree that one workgroup builds (class 3; above: class 4) */
+#define DEB_HALF 29696
 /* rounds of path shortening before the joins */
 #define DEB_JUMPS 3
 
@@ -134,15 +143,16 @@ struct DebArgs {
     unsigned char *lmflag;  /* per raw-list entry: 1 for a local maximum (first pass) */
     int *lstar;             /* first level above the second-highest maximum, then L* */
     int *clist;             /* objects of each size class: clist[cls * nraw + j] */
-    int *ccount;            /* [0..3] objects per class, [4..6] the largest LDS need of
-                               classes 0..2 (bytes), [7..10] pixels per class */
+    int *ccount;            /* DEB_NCOUNT counters */
     unsigned long long *dwork;  /* [0] pixels, [1] pixel-levels of the multi-peak objects,
                                    [2] node capacity of the frame */
-    /* global scratch for the objects built in global memory, by raw-list position */
+    /* global scratch for the objects built in global memory, by raw-list position, and a
+       record for each of class 4 */
     double *g_sum;
     unsigned long long *g_par, *g_cnt;
     int *g_list;
     unsigned char *g_m;
+    struct DebWide *wide;
 };
 
 /* the raw objects and their pixels: the device counts of a planned run */
@@ -246,16 +256,17 @@ __global__ void __launch_bounds__(256) k_deb_nodecap(DebArgs a)
 
 /* single-peak objects are kept as they are (one node); the others go to a size class (0:
    up to cap0 pixels, 256 lanes in LDS; 1: up to cap1, 512 lanes in LDS; 2: up to cap2, 1024
-   lanes in LDS; 3: global memory).  The counters take one atomic per workgroup and
-   class (one per wavefront, as the order kernels had, took 19 us for 22,000 raw objects, 7
-   now); [4 + class] records the largest LDS need. */
+   lanes in LDS; 3: up to DEB_HALF, one workgroup with its sums in global memory; 4: the whole
+   chip).  The counters take one atomic per workgroup and class (one per wavefront, as the
+   order kernels had, took 19 us for 22,000 raw objects, 7 now). */
 __global__ void __launch_bounds__(256) k_deb_classify(DebArgs a, int cap0, int cap1, int cap2)
 {
-    __shared__ int s_n[4], s_px[4], s_need[4], s_base[4];
+    __shared__ int s_n[DEB_NCLASS], s_px[DEB_NCLASS], s_need[DEB_NCLASS], s_base[DEB_NCLASS];
     __shared__ unsigned long long s_work[2];
     const int r = blockIdx.x * 256 + threadIdx.x;
     const int lane = threadIdx.x & 63;
-    if (threadIdx.x < 4) s_n[threadIdx.x] = s_px[threadIdx.x] = s_need[threadIdx.x] = 0;
+    if (threadIdx.x < DEB_NCLASS)
+        s_n[threadIdx.x] = s_px[threadIdx.x] = s_need[threadIdx.x] = 0;
     if (threadIdx.x < 2) s_work[threadIdx.x] = 0;
     __syncthreads();
     int cls = -1, n = 0, ls = 0, need = 0;
@@ -267,7 +278,7 @@ __global__ void __launch_bounds__(256) k_deb_classify(DebArgs a, int cap0, int c
             a.rootkept[r] = 1;
         } else {
             need = deb_lds_bytes(n);
-            cls = n <= cap0 ? 0 : n <= cap1 ? 1 : n <= cap2 ? 2 : 3;
+            cls = n <= cap0 ? 0 : n <= cap1 ? 1 : n <= cap2 ? 2 : n <= DEB_HALF ? 3 : 4;
         }
     }
     unsigned long long w0 = cls >= 0 ? (unsigned long long)n : 0ull;
@@ -281,7 +292,7 @@ __global__ void __launch_bounds__(256) k_deb_classify(DebArgs a, int cap0, int c
         atomicAdd(&s_work[1], w1);
     }
     int slot = 0;
-    for (int c = 0; c < 4; c++) {
+    for (int c = 0; c < DEB_NCLASS; c++) {
         const unsigned long long b = __ballot(cls == c);
         if (!b) continue;
         const int lead = __builtin_ctzll(b);
@@ -300,14 +311,14 @@ __global__ void __launch_bounds__(256) k_deb_classify(DebArgs a, int cap0, int c
         if (cls == c) slot = base + __popcll(b & sxw_lanes_below(lane));
     }
     __syncthreads();
-    if (threadIdx.x < 4 && s_n[threadIdx.x]) {
+    if (threadIdx.x < DEB_NCLASS && s_n[threadIdx.x]) {
         const int c = threadIdx.x;
         s_base[c] = atomicAdd(&a.ccount[c], s_n[c]);
-        if (c < 3) atomicMax(&a.ccount[4 + c], s_need[c]);
-        atomicAdd(&a.ccount[7 + c], s_px[c]);
+        if (c < 3) atomicMax(&a.ccount[DEB_CLDS + c], s_need[c]);
+        atomicAdd(&a.ccount[DEB_CPIX + min(c, 3)], s_px[c]);
     }
-    if (threadIdx.x >= 4 && threadIdx.x < 6 && s_work[threadIdx.x - 4])
-        atomicAdd(&a.dwork[threadIdx.x - 4], s_work[threadIdx.x - 4]);
+    if (threadIdx.x >= 64 && threadIdx.x < 66 && s_work[threadIdx.x - 64])
+        atomicAdd(&a.dwork[threadIdx.x - 64], s_work[threadIdx.x - 64]);
     __syncthreads();
     if (cls >= 0) a.clist[(size_t)cls * a.cstride + s_base[cls] + slot] = r;
 }
@@ -371,7 +382,8 @@ __device__ inline int deb_sig_bound(double s, double sabs, int n, float b, doubl
  * levels were walked one by one before, with five passes over all pixels each (13 us a level
  * for 4,370 pixels).  Measured, before and after: crowded 4096^2, classes 0, 1, 2: 276, 167,
  * 229 -> 76, 50, 46 us; dense 2048^2, class 3 (40 objects of 6,000 to 18,000 pixels) 2,617 ->
- * 472 us with par and m in LDS (1,470 with all state in global memory).  Lanes: class 0 with
+ * 472 us with par and m in LDS (1,470 with all state in global memory).  Objects of more
+ * pixels than that LDS holds (class 4) are built by the whole chip: k_deb_wide_levels.  Lanes: class 0 with
  * 64 lanes 138 us, class 1 with 256 lanes 73 us (more pixels a lane, one after the other).
  * Left out: the pixels entering level by level from the highest (each join is short then,
  * but a level costs two barriers and 3 us of contended joins whatever its size: class 2 46
@@ -491,97 +503,33 @@ __device__ inline float wave_ordered_sum(int n, Sel sel, Val val, int need)
     return f;
 }
 
-/* PG: par and m in global memory, else in LDS; G: the other arrays in global memory.
-   Per raw-list index of the object: sum (its cd, then the sum of a node; later two int
-   arrays of cap entries), par, cnt (G: par; the pixel list while the neighbours are found, then
-   count and flags of a node, later the order key of a kept node), list (the roots by
-   level, later the kept node of each pixel), m. */
-template <int NT, bool PG, bool G, class IT>
-__device__ __forceinline__ void deb_tree(const DebArgs &a, const int r, const int cap, double *sum,
-                                         typename DebWord<PG>::T *parw,
-                                         typename DebWord<PG>::T *cnt, IT *list,
-                                         unsigned char *m)
-{
-    typedef DebTree<PG> D;
-    const typename D::template Par<PG> par{parw};
+/*
+ * The passes over the pixels of one object.  WIDE: parent words of 64 bits and level indices in
+ * global memory, written by several workgroups in turn; else in LDS.  G: the other arrays in
+ * global memory.  Per raw-list index of the object: sum (its cd, then the sum of a node; later
+ * two int arrays), par, cnt (while the neighbours are found the pixel list, in LDS; then count
+ * and flags of a node, later the order key of a kept node), list (the neighbours, then the roots
+ * by level), m.
+ */
+template <bool WIDE, bool G, class IT> struct DebObj {
+    typedef DebTree<WIDE> D;
     typedef typename D::T T;
-    __shared__ int s_lev[SXG_MAXNTHRESH + 1], s_at[SXG_MAXNTHRESH + 1];
-    __shared__ float tthr[SXG_MAXNTHRESH + 1], ttau[SXG_MAXNTHRESH + 1];
-    __shared__ double s_rsum[NT / 64], s_rabs[NT / 64];
-    __shared__ T s_top;              /* flags of level 0, the whole object */
-    __shared__ int s_nk, s_nopen, s_open[256];
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const int n = a.cnt[r], off = a.off[r], ls = a.lstar[r];
-    const int W = a.W;
-    const int *const fp = a.fpia + off;
-    if (wid == 0) {
-        /* sub-thresholds 1..L* and their running maximum tau (L* <= 63: one lane each) */
-        const float v = lane < ls ? a.thr[(size_t)r * a.nthresh + lane + 1] : -INFINITY;
-        float tau = v;
-        for (int d = 1; d < 64; d <<= 1) {
-            const float o = __shfl_up(tau, d);
-            if (lane >= d) tau = fmaxf(tau, o);
-        }
-        if (lane < ls) {
-            tthr[lane + 1] = v;
-            ttau[lane + 1] = tau;
-        }
-        s_lev[lane] = 0;
-        if (lane == 0) {
-            s_lev[64] = 0;
-            s_top = 0;
-            s_nk = s_nopen = 0;
-        }
-    }
-    __syncthreads();
-    /* level index m = max{i <= L* : tau_i <= cd} (tau is non-decreasing), bounds of the
-       root's flux */
-    int *const pix = G ? reinterpret_cast<int *>(parw) : reinterpret_cast<int *>(cnt);
-    double rsum = 0.0, rabs = 0.0;
-    for (int k = tid; k < n; k += NT) {
-        const int p = fp[k];
-        const float v = a.cd[p];
-        rsum += v;
-        rabs += fabs(v);
-        int lo = 0, hi = ls;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (ttau[mid] <= v) lo = mid;
-            else hi = mid - 1;
-        }
-        if (!PG) pix[k] = p;
-        deb_st<G>(&sum[k], (double)v);
-        m[k] = (unsigned char)lo;
-    }
-    rsum = sxw_sum(rsum);
-    rabs = sxw_sum(rabs);
-    if (lane == 0) {
-        s_rsum[wid] = rsum;
-        s_rabs[wid] = rabs;
-    }
-    deb_sync<G || PG>();
-    rsum = rabs = 0.0;
-#pragma unroll
-    for (int w = 0; w < NT / 64; w++) {
-        rsum += s_rsum[w];
-        rabs += s_rabs[w];
-    }
-    /* First parents, one pair per pixel, without atomics: a pixel at the head of its run
-       (neighbours along the row on one level, inside the wavefront's 64 entries); a head at
-       a backward neighbour of its level, else at the one of the highest level below.  The
-       row above: its neighbours are consecutive list entries, searched for among the
-       entries that can lie between (a row of the object's width on either side of the
-       row's end).  Kept for the joins: their distance and which of them are there in list,
-       whether W is in bit 7 of m. */
-    const int *const pl = PG ? fp : pix;
-    const int span = 2 * (a.xmax[r] - a.xmin[r] + 1) + 1;
+    typename D::template Par<WIDE> par;
+    double *sum;
+    T *cnt;
+    IT *list;
+    unsigned char *m;
+    const int *pl;     /* the pixels */
+    int n, W, span;    /* span: list entries that may lie between a pixel and its row above */
+
     /* levels of the neighbours (0: none), their places, and which of them is the first
        parent: 1 W, 2 NW, 3 N, 4 NE, 0 none; same: W of the pixel's level */
     struct Nb {
         int mw, mnw, mn, mne, j0, jn, jne, first;
         bool same;
     };
-    auto around = [&](int k, int mk, int enc, bool west) {
+    __device__ Nb around(int k, int mk, int enc, bool west) const
+    {
         Nb q;
         q.j0 = k - (enc >> 3);
         q.jn = q.j0 + (enc & 1);
@@ -604,10 +552,15 @@ __device__ __forceinline__ void deb_tree(const DebArgs &a, const int r, const in
             if (q.mne < mk && q.mne > best) best = q.mne, q.first = 4;
         }
         return q;
-    };
-    for (int k = tid; k < n; k += NT) {
+    }
+    /* the neighbours of pixel k in the row above are consecutive list entries, searched for
+       among those that can lie between (a row of the object's width on either side of the row's
+       end): their distance and which of them are there into list, whether W is into bit 7 of
+       m */
+    __device__ void look(int k) const
+    {
         const int mk = m[k] & 63;
-        if (mk == 0) continue;
+        if (mk == 0) return;
         const int p = pl[k];
         const int y = p / W, x = p - y * W;
         int enc = 0, j0 = k;
@@ -627,10 +580,14 @@ __device__ __forceinline__ void deb_tree(const DebArgs &a, const int r, const in
         deb_st<G>(&list[k], (IT)(enc | (k - j0) << 3));
         if (x > 0 && k > 0 && pl[k - 1] == p - 1) m[k] = (unsigned char)(mk | 128);
     }
-    deb_sync<G || PG>();
-    for (int b0 = 0; b0 < n; b0 += NT) {
-        const int k = b0 + tid;
-        const int mk = k < n ? m[k] & 63 : 0;
+    /* first parents, one pair per pixel, without atomics: a pixel at the head of its run
+       (neighbours along the row on one level, inside the wavefront's 64 entries); a head at a
+       backward neighbour of its level, else at the one of the highest level below.  Every lane
+       of the wavefront calls, with consecutive entries; in: it has a pixel */
+    __device__ void first(int k, bool in) const
+    {
+        const int lane = threadIdx.x & 63;
+        const int mk = in ? m[k] & 63 : 0;
         bool same = false;
         Nb q{};
         if (mk > 0) {
@@ -646,27 +603,25 @@ __device__ __forceinline__ void deb_tree(const DebArgs &a, const int r, const in
                 w = q.first == 1 ? D::word(q.mw, k - 1) : q.first == 2 ? D::word(q.mnw, q.j0)
                     : q.first == 3 ? D::word(q.mn, q.jn) : D::word(q.mne, q.jne);
         }
-        if (k < n) par.st(k, w);
+        if (in) par.st(k, w);
     }
-    deb_sync<G || PG>();
     /* chains of a level cut short: a pixel at its parent's parent (only its own thread
        changes a word here, and every value read is above it on its level) */
-    for (int round = 0; round < DEB_JUMPS; round++) {
-        for (int k = tid; k < n; k += NT) {
-            const int mk = m[k] & 63;
-            if (mk == 0) continue;
-            const T w = par.ld(k);
-            if (D::lev(w) != mk) continue;
-            const T g = par.ld(D::idx(w));
-            if (D::lev(g) == mk) par.st(k, g);
-        }
-        deb_sync<G || PG>();
+    __device__ void shorten(int k) const
+    {
+        const int mk = m[k] & 63;
+        if (mk == 0) return;
+        const T w = par.ld(k);
+        if (D::lev(w) != mk) return;
+        const T g = par.ld(D::idx(w));
+        if (D::lev(g) == mk) par.st(k, g);
     }
     /* the other pairs.  One is left out where two others imply it at its level: N through W
        and NW; NW through W or N; NE through N. */
-    for (int k = tid; k < n; k += NT) {
+    __device__ void joins(int k) const
+    {
         const int mk = m[k] & 63;
-        if (mk == 0) continue;
+        if (mk == 0) return;
         const Nb q = around(k, mk, (int)deb_ld<G>(&list[k]), (m[k] & 128) != 0);
         const int en = min(mk, q.mn), enw = min(mk, q.mnw), ene = min(mk, q.mne);
         if (q.mw > 0 && q.first != 1) par.join(k, mk, k - 1, q.mw);
@@ -675,57 +630,78 @@ __device__ __forceinline__ void deb_tree(const DebArgs &a, const int r, const in
             par.join(k, mk, q.j0, q.mnw);
         if (ene > 0 && q.first != 4 && q.mn < ene) par.join(k, mk, q.jne, q.mne);
     }
-    deb_sync<G || PG>();
-    /* every pixel at the root of its level, every root at the root above it; the roots of
-       each level counted; a pixel of level 0 belongs to the whole object only */
-    for (int k = tid; k < n; k += NT) {
+    /* pixel k at the root of its level, a root at the root above it (a pixel of level 0
+       belongs to the whole object only); the level of a root, else 0 */
+    __device__ int settle(int k) const
+    {
         const int mk = m[k] & 63;
         m[k] = (unsigned char)mk;
-        deb_st<G>(&cnt[k], (T)1);
-        if (mk == 0) continue;
-        T w = par.ld(k);
+        if (mk == 0) return 0;
+        const T w = par.ld(k);
+        T pw;
         if (D::lev(w) == mk) {
-            T pw;
             const int q = par.root(D::idx(w), mk, pw);
             par.st(k, D::word(mk, q));
-        } else {
-            atomicAdd(&s_lev[mk], 1);
-            if (w) {
-                T pw;
-                const int q = par.root(D::idx(w), D::lev(w), pw);
-                par.st(k, D::word(D::lev(w), q));
-            }
+            return 0;
         }
-    }
-    deb_sync<G || PG>();
-    if (wid == 0) {
-        /* the list's places, the highest level first */
-        const int c = lane < 63 ? s_lev[63 - lane] : 0;
-        int x = c;
-        for (int d = 1; d < 64; d <<= 1) {
-            const int o = __shfl_up(x, d);
-            if (lane >= d) x += o;
+        if (w) {
+            const int q = par.root(D::idx(w), D::lev(w), pw);
+            par.st(k, D::word(D::lev(w), q));
         }
-        if (lane < 63) s_at[63 - lane] = x - c;
+        return mk;
     }
-    /* a pixel's count and cd to its root */
-    for (int k = tid; k < n; k += NT) {
-        const int mk = m[k];
-        if (mk == 0) continue;
-        const T w = par.ld(k);
-        if (D::lev(w) == mk) {
-            atomicAdd(&cnt[D::idx(w)], (T)1);
-            atomicAdd(&sum[D::idx(w)], deb_ld<G>(&sum[k]));
+    /* pixel k to the kept node that holds it (place: by node, see deb_nodes), and the last
+       pixel of each kept node from the last of every run of its pixels.  Every lane of the
+       wavefront calls, with consecutive entries; in: it has a pixel */
+    __device__ void assign(int k, bool in, const int *slot, const int *place, int *kcomp,
+                           Comp *C) const
+    {
+        const int lane = threadIdx.x & 63;
+        int c = -1;
+        const int mk = in ? m[k] : 0;
+        if (mk > 0) {
+            const T w = par.ld(k);
+            const int s = deb_ld<G>(&slot[D::lev(w) == mk ? D::idx(w) : k]);
+            if (s >= 0) c = deb_ld<G>(&place[s]);
         }
+        const int next = __shfl_down(c, 1);
+        if (!in) return;
+        kcomp[k] = c;
+        if (c >= 0 && (lane == 63 || k == n - 1 || next != c)) atomicMax(&C[c].hi, k);
     }
-    deb_sync<G || PG>();
-    for (int k = tid; k < n; k += NT) {
-        const int mk = m[k];
-        if (mk > 0 && D::lev(par.ld(k)) != mk)
-            deb_st<G>(&list[atomicAdd(&s_at[mk], 1)], (IT)k);
+};
+
+/*
+ * What follows when the pixels hang on their roots, by one workgroup: the node sums, the
+ * significance, A() and the kept nodes (into C, with lo = hi = the first pixel; their number,
+ * 0 where there is no split).  s_lev: roots of each level, s_at: where those of a level end in
+ * list (highest level first); tthr: sub-thresholds; rsum, rabs: bounds of the root's flux.
+ * Leaves in sum the slot of each node, that of its kept node or -1, and from cap on the place
+ * of each slot's kept node in C.
+ */
+template <int NT, bool WIDE, bool G, class IT>
+__device__ __forceinline__ int deb_nodes(const DebArgs &a, const DebObj<WIDE, G, IT> &t,
+                                         const int *const fp, int cap, int ls, const int *s_lev,
+                                         const int *s_at, const float *tthr, double rsum,
+                                         double rabs, Comp *C)
+{
+    typedef DebTree<WIDE> D;
+    typedef typename D::T T;
+    __shared__ T s_top;              /* flags of level 0, the whole object */
+    __shared__ int s_nk, s_nopen, s_open[256];
+    __shared__ float s_fr;
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const auto par = t.par;
+    T *const cnt = t.cnt;
+    double *const sum = t.sum;
+    IT *const list = t.list;
+    const unsigned char *const m = t.m;
+    const int n = t.n;
+    if (tid == 0) {
+        s_top = 0;
+        s_nk = s_nopen = 0;
     }
-    deb_sync<G || PG>();
-    /* now the roots of level i end at s_at[i]; those of level 1 are the last */
+    /* the roots of level i end at s_at[i]; those of level 1 are the last */
     const int nn = s_at[1];
     for (int i = ls; i >= 2; i--) {
         const int e = s_at[i], b = e - s_lev[i];
@@ -738,8 +714,9 @@ __device__ __forceinline__ void deb_tree(const DebArgs &a, const int r, const in
                 atomicAdd(&sum[D::idx(w)], deb_ld<G>(&sum[k]));
             }
         }
-        deb_sync<G || PG>();
+        deb_sync<G>();
     }
+    deb_sync<G>();
     /* children */
     auto mark = [&](T w, T f1, T f2) {
         T *q = w ? &cnt[D::idx(w)] : &s_top;
@@ -750,7 +727,7 @@ __device__ __forceinline__ void deb_tree(const DebArgs &a, const int r, const in
         const int k = deb_ld<G>(&list[c]);
         if ((int)(deb_ld<G>(&cnt[k]) & D::CM) >= a.debarea) mark(par.ld(k), D::CH1, D::CH2);
     }
-    deb_sync<G || PG>();
+    deb_sync<G>();
     /* significance of the nodes that have siblings */
     const bool nonneg = rabs == rsum;
     double v0lo, v0hi;
@@ -761,31 +738,51 @@ __device__ __forceinline__ void deb_tree(const DebArgs &a, const int r, const in
         v0lo = fmin(p, q) - fabs(fmin(p, q)) * 0x1p-50 - 1e-300;
         v0hi = fmax(p, q) + fabs(fmax(p, q)) * 0x1p-50 + 1e-300;
     }
-    bool fr_ok = false;
-    float fr = 0.0f;
+    bool exact = false;              /* the root's flux is known: v0lo = v0hi */
     auto val = [&](int k) { return a.cd[fp[k]]; };
+    auto test = [&](int k, int cc, T w) {
+        const double s = deb_ld<G>(&sum[k]);
+        const int sig = deb_sig_bound(s, nonneg ? s : rabs, cc, tthr[D::lev(w) + 1] * (float)cc,
+                                      v0lo, v0hi);
+        if (sig > 0) {
+            atomicOr(&cnt[k], D::SIG);
+            mark(w, D::SON1, D::SON2);
+        }
+        return sig;
+    };
     for (int c0 = 0; c0 < nn; c0 += 256) {
         const int c = c0 + tid;
         if (tid < 256 && c < nn) {
             const int k = deb_ld<G>(&list[c]);
             const int cc = (int)(deb_ld<G>(&cnt[k]) & D::CM);
             const T w = par.ld(k);
-            if (cc >= a.debarea && (flags(w) & D::CH2)) {
-                const double s = deb_ld<G>(&sum[k]);
-                const int sig = deb_sig_bound(s, nonneg ? s : rabs, cc,
-                                              tthr[D::lev(w) + 1] * (float)cc, v0lo, v0hi);
-                if (sig < 0) {
-                    s_open[atomicAdd(&s_nopen, 1)] = k;
-                } else if (sig > 0) {
-                    atomicOr(&cnt[k], D::SIG);
-                    mark(w, D::SON1, D::SON2);
-                }
-            }
+            if (cc >= a.debarea && (flags(w) & D::CH2) && test(k, cc, w) < 0)
+                s_open[atomicAdd(&s_nopen, 1)] = k;
         }
-        deb_sync<G || PG>();
-        /* the exact sequential float sums where the bounds cannot decide, a wavefront each */
-        for (int j = wid; j < s_nopen; j += NT / 64) {
-            const int node = s_open[j], mc = m[node];
+        deb_sync<G>();
+        const int nopen = s_nopen;
+        if (nopen > 0 && !exact) {
+            /* where the bounds cannot decide, first the exact sequential float sum of the whole
+               object: it leaves only the node's own rounding (an object of five million pixels
+               has a bound of 40 % on its flux) */
+            if (wid == 0) {
+                const float fr = wave_ordered_sum(n, [](int) { return true; }, val, n);
+                if (lane == 0) s_fr = fr;
+            }
+            __syncthreads();
+            v0lo = v0hi = (double)s_fr * a.mincont;
+            exact = true;
+            if (tid < nopen) {
+                const int k = s_open[tid];
+                if (test(k, (int)(deb_ld<G>(&cnt[k]) & D::CM), par.ld(k)) >= 0) s_open[tid] = -1;
+            }
+            deb_sync<G>();
+        }
+        /* then the node's, a wavefront each */
+        for (int j = wid; j < nopen; j += NT / 64) {
+            const int node = s_open[j];
+            if (node < 0) continue;
+            const int mc = m[node];
             const int cc = (int)(deb_ld<G>(&cnt[node]) & D::CM);
             const T w = par.ld(node);
             const float f = wave_ordered_sum(
@@ -804,19 +801,15 @@ __device__ __forceinline__ void deb_tree(const DebArgs &a, const int r, const in
                     return at == node;
                 },
                 val, cc);
-            if (!fr_ok) {
-                fr = wave_ordered_sum(n, [](int) { return true; }, val, n);
-                fr_ok = true;
-            }
             const float lhs = f - tthr[D::lev(w) + 1] * (float)cc;
-            if (lane == 0 && (double)lhs > (double)fr * a.mincont) {
+            if (lane == 0 && (double)lhs > v0lo) {
                 atomicOr(&cnt[node], D::SIG);
                 mark(w, D::SON1, D::SON2);
             }
         }
-        deb_sync<G || PG>();
+        deb_sync<G>();
         if (tid == 0) s_nopen = 0;
-        if (c0 + 256 < nn) deb_sync<G || PG>();
+        if (c0 + 256 < nn) deb_sync<G>();
     }
     /* A(): a node with two significant children voids its own and those above */
     int *const slot = reinterpret_cast<int *>(sum), *const kept = slot + cap;
@@ -833,17 +826,8 @@ __device__ __forceinline__ void deb_tree(const DebArgs &a, const int r, const in
         }
     }
     if (tid == 0 && (deb_ld<false>(&s_top) & D::SON2)) atomicOr(&s_top, D::NOTA);
-    deb_sync<G || PG>();
-    Comp *const C = a.comps + a.compoff[r];
-    if (!(deb_ld<false>(&s_top) & D::NOTA)) {
-        /* no split: the raw object is kept as it is */
-        if (tid == 0) {
-            C[0] = {0, fp[0], 0, n - 1};
-            a.rootnc[r] = 1;
-            a.rootkept[r] = 1;
-        }
-        return;
-    }
+    deb_sync<G>();
+    if (!(deb_ld<false>(&s_top) & D::NOTA)) return 0;
     for (int c = tid; c < nn; c += NT) {
         const int k = deb_ld<G>(&list[c]);
         const T f = deb_ld<G>(&cnt[k]);
@@ -853,36 +837,30 @@ __device__ __forceinline__ void deb_tree(const DebArgs &a, const int r, const in
             deb_st<G>(&kept[j], k);
         }
     }
-    deb_sync<G || PG>();
+    deb_sync<G>();
     const int nk = s_nk;
     for (int j = tid; j < nk; j += NT) deb_st<G>(&cnt[j], ~(T)0);
+    deb_sync<G>();
     /* each node's kept node (kept nodes never nest: one at most on its way up; a value that
-       another lane has put on the way is the same), then each pixel's, and the first pixel
-       of each kept node */
+       another lane has put on the way is the same), and the first pixel of each kept node: a
+       root is the first pixel of its level's component */
     for (int c = tid; c < nn; c += NT) {
         const int k = deb_ld<G>(&list[c]);
         int s = deb_ld<G>(&slot[k]);
-        if (s >= 0) continue;
-        for (T w = par.ld(k); w && s < 0; w = par.ld(D::idx(w))) s = deb_ld<G>(&slot[D::idx(w)]);
-        if (s >= 0) deb_st<G>(&slot[k], s);
-    }
-    deb_sync<G || PG>();
-    for (int k = tid; k < n; k += NT) {
-        int s = -1;
-        if (m[k] > 0) {
-            const T w = par.ld(k);
-            s = deb_ld<G>(&slot[D::lev(w) == m[k] ? D::idx(w) : k]);
-            if (s >= 0) atomicMin(&cnt[s], (T)k);
+        if (s < 0) {
+            for (T w = par.ld(k); w && s < 0; w = par.ld(D::idx(w)))
+                s = deb_ld<G>(&slot[D::idx(w)]);
+            if (s >= 0) deb_st<G>(&slot[k], s);
         }
-        deb_st<G>(&list[k], (IT)s);
+        if (s >= 0) atomicMin(&cnt[s], (T)k);
     }
-    deb_sync<G || PG>();
+    deb_sync<G>();
     /* the kept nodes ordered by level, then first pixel */
     for (int j = tid; j < nk; j += NT) {
         const T w = par.ld(deb_ld<G>(&kept[j]));
         deb_st<G>(&cnt[j], ((T)(D::lev(w) + 1) << D::SH) | deb_ld<G>(&cnt[j]));
     }
-    deb_sync<G || PG>();
+    deb_sync<G>();
     for (int j0 = wid * 64; j0 < nk; j0 += NT) {
         const int j = j0 + lane;
         const T key = j < nk ? deb_ld<G>(&cnt[j]) : 0;
@@ -892,34 +870,149 @@ __device__ __forceinline__ void deb_tree(const DebArgs &a, const int r, const in
             for (int u = 0; u < min(64, nk - i0); u++) {
                 const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)other, u);
                 const unsigned hi =
-                    PG ? (unsigned)__builtin_amdgcn_readlane((int)((unsigned long long)other >> 32), u)
-                       : 0u;
+                    WIDE ? (unsigned)__builtin_amdgcn_readlane((int)((unsigned long long)other >> 32), u)
+                         : 0u;
                 rank += (T)((unsigned long long)hi << 32 | lo) < key;
             }
         }
         if (j < nk) {
-            deb_st<G>(&slot[j], rank);
+            deb_st<G>(&kept[j], rank);
             const int lo = (int)(key & D::IM);
             C[rank] = {D::lev(key), fp[lo], lo, lo};
         }
     }
-    deb_sync<G || PG>();
-    /* the last pixel of each kept node: from the last of every run of its pixels */
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    return nk;
+}
+
+/* where the roots of level `lane` start in the list, the highest level first (lev: roots of
+   each level; one wavefront) */
+__device__ inline int deb_level_start(const int *lev)
+{
+    const int lane = threadIdx.x & 63;
+    const int c = lane < 63 ? lev[63 - lane] : 0;
+    int x = c;
+    for (int d = 1; d < 64; d <<= 1) {
+        const int o = __shfl_up(x, d);
+        if (lane >= d) x += o;
+    }
+    return __shfl(x - c, 63 - lane);
+}
+
+/* an object by one workgroup, with par and m in LDS (G: the rest in global memory) */
+template <int NT, bool G, class IT>
+__device__ __forceinline__ void deb_tree(const DebArgs &a, const int r, const int cap, double *sum,
+                                         unsigned *parw, unsigned *cnt, IT *list,
+                                         unsigned char *m)
+{
+    typedef DebTree<false> D;
+    typedef D::T T;
+    __shared__ int s_lev[SXG_MAXNTHRESH + 1], s_at[SXG_MAXNTHRESH + 1];
+    __shared__ float tthr[SXG_MAXNTHRESH + 1], ttau[SXG_MAXNTHRESH + 1];
+    __shared__ double s_rsum[NT / 64], s_rabs[NT / 64];
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int n = a.cnt[r], off = a.off[r], ls = a.lstar[r];
+    const int *const fp = a.fpia + off;
+    int *const pix = reinterpret_cast<int *>(G ? parw : cnt);
+    const DebObj<false, G, IT> t = {{parw}, sum, cnt, list, m, pix, n, a.W,
+                                    2 * (a.xmax[r] - a.xmin[r] + 1) + 1};
+    const auto &par = t.par;
+    if (wid == 0) {
+        /* sub-thresholds 1..L* and their running maximum tau (L* <= 63: one lane each) */
+        const float v = lane < ls ? a.thr[(size_t)r * a.nthresh + lane + 1] : -INFINITY;
+        float tau = v;
+        for (int d = 1; d < 64; d <<= 1) {
+            const float o = __shfl_up(tau, d);
+            if (lane >= d) tau = fmaxf(tau, o);
+        }
+        if (lane < ls) {
+            tthr[lane + 1] = v;
+            ttau[lane + 1] = tau;
+        }
+        s_lev[lane] = 0;
+        if (lane == 0) s_lev[64] = 0;
+    }
     __syncthreads();
-    for (int b0 = 0; b0 < n; b0 += NT) {
-        const int k = b0 + tid;
-        const IT s = k < n ? deb_ld<G>(&list[k]) : (IT)-1;
-        const int c = s == (IT)-1 ? -1 : deb_ld<G>(&slot[s]);
-        const int next = __shfl_down(c, 1);
-        if (k >= n) continue;
-        a.kcomp[off + k] = c;
-        if (c >= 0 && (lane == 63 || k == n - 1 || next != c)) atomicMax(&C[c].hi, k);
+    /* level index m = max{i <= L* : tau_i <= cd} (tau is non-decreasing), bounds of the
+       root's flux */
+    double rsum = 0.0, rabs = 0.0;
+    for (int k = tid; k < n; k += NT) {
+        const int p = fp[k];
+        const float v = a.cd[p];
+        rsum += v;
+        rabs += fabs(v);
+        int lo = 0, hi = ls;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (ttau[mid] <= v) lo = mid;
+            else hi = mid - 1;
+        }
+        pix[k] = p;
+        deb_st<G>(&sum[k], (double)v);
+        m[k] = (unsigned char)lo;
     }
+    rsum = sxw_sum(rsum);
+    rabs = sxw_sum(rabs);
+    if (lane == 0) {
+        s_rsum[wid] = rsum;
+        s_rabs[wid] = rabs;
+    }
+    deb_sync<G>();
+    rsum = rabs = 0.0;
+#pragma unroll
+    for (int w = 0; w < NT / 64; w++) {
+        rsum += s_rsum[w];
+        rabs += s_rabs[w];
+    }
+    for (int k = tid; k < n; k += NT) t.look(k);
+    deb_sync<G>();
+    for (int b0 = 0; b0 < n; b0 += NT) t.first(b0 + tid, b0 + tid < n);
+    deb_sync<G>();
+    for (int round = 0; round < DEB_JUMPS; round++) {
+        for (int k = tid; k < n; k += NT) t.shorten(k);
+        deb_sync<G>();
+    }
+    for (int k = tid; k < n; k += NT) t.joins(k);
+    deb_sync<G>();
+    for (int k = tid; k < n; k += NT) {
+        deb_st<G>(&cnt[k], (T)1);
+        const int l = t.settle(k);
+        if (l) atomicAdd(&s_lev[l], 1);
+    }
+    deb_sync<G>();
+    if (wid == 0) {
+        const int at = deb_level_start(s_lev);
+        if (lane > 0) s_at[lane] = at;
+    }
+    /* a pixel's count and cd to its root */
+    for (int k = tid; k < n; k += NT) {
+        const int mk = m[k];
+        if (mk == 0) continue;
+        const T w = par.ld(k);
+        if (D::lev(w) == mk) {
+            atomicAdd(&cnt[D::idx(w)], (T)1);
+            atomicAdd(&sum[D::idx(w)], deb_ld<G>(&sum[k]));
+        }
+    }
+    deb_sync<G>();
+    for (int k = tid; k < n; k += NT) {
+        const int mk = m[k];
+        if (mk > 0 && D::lev(par.ld(k)) != mk)
+            deb_st<G>(&list[atomicAdd(&s_at[mk], 1)], (IT)k);
+    }
+    deb_sync<G>();
+    Comp *const C = a.comps + a.compoff[r];
+    const int nk = deb_nodes<NT>(a, t, fp, cap, ls, s_lev, s_at, tthr, rsum, rabs, C);
     if (tid == 0) {
-        a.rootnc[r] = nk;
-        a.rootkept[r] = nk;
+        /* without a split the raw object is kept as it is */
+        if (nk == 0) C[0] = {0, fp[0], 0, n - 1};
+        a.rootnc[r] = a.rootkept[r] = max(nk, 1);
     }
+    if (nk == 0) return;
+    /* the kept nodes are in global memory */
+    deb_sync<true>();
+    const int *const slot = reinterpret_cast<const int *>(sum);
+    for (int b0 = 0; b0 < n; b0 += NT)
+        t.assign(b0 + tid, b0 + tid < n, slot, slot + cap, a.kcomp + off, C);
 }
 
 /* CLS names the size class in the kernel's symbol only (a kernel trace then times each
@@ -936,29 +1029,262 @@ template <int NT, int CLS> __global__ void __launch_bounds__(NT) k_deb_tree_lds(
     unsigned *cnt = par + cap;
     unsigned short *list = reinterpret_cast<unsigned short *>(cnt + cap);
     unsigned char *m = reinterpret_cast<unsigned char *>(list + cap);
-    deb_tree<NT, false, false, unsigned short>(a, r, cap, sum, par, cnt, list, m);
+    deb_tree<NT, false, unsigned short>(a, r, cap, sum, par, cnt, list, m);
 }
 
-/* raw objects too large for all of it: up to DEB_HALF pixels the parent words and level
-   indices, which the dependent accesses go to, still sit in LDS (5 bytes a pixel) and the
-   rest in global memory; above, everything does */
-#define DEB_HALF 29696
+/* raw objects too large for all of it, up to DEB_HALF pixels: the parent words and level
+   indices, which the dependent accesses go to, still sit in LDS (5 bytes a pixel) and the rest
+   in global memory */
 __global__ void __launch_bounds__(1024) k_deb_tree_glb(DebArgs a)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     if (a.pd && (int)blockIdx.x >= a.ccount[3]) return;
     const int r = a.clist[3 * (size_t)a.cstride + blockIdx.x];
     const int off = a.off[r], n = a.cnt[r];
-    if (n <= DEB_HALF) {
-        unsigned *par = reinterpret_cast<unsigned *>(smem);
-        deb_tree<1024, false, true, int>(a, r, n, a.g_sum + off, par,
-                                         reinterpret_cast<unsigned *>(a.g_cnt + off),
-                                         a.g_list + off,
-                                         reinterpret_cast<unsigned char *>(par + DEB_HALF));
-    } else {
-        deb_tree<1024, true, true, int>(a, r, n, a.g_sum + off, a.g_par + off, a.g_cnt + off,
-                                        a.g_list + off, a.g_m + off);
+    unsigned *par = reinterpret_cast<unsigned *>(smem);
+    deb_tree<1024, true, int>(a, r, n, a.g_sum + off, par,
+                              reinterpret_cast<unsigned *>(a.g_cnt + off), a.g_list + off,
+                              reinterpret_cast<unsigned char *>(par + DEB_HALF));
+}
+
+/*
+ * The trees of the larger raw objects, one pass a kernel: a lane for every pixel of the raw list
+ * that belongs to one of them, then a workgroup per object for the nodes, then the pixels again.  The same passes as in one workgroup, with all state in global
+ * memory; between kernels everything is there, and inside one the words that other workgroups
+ * change go through the device-coherent level.  Bound: latency of dependent accesses, in the
+ * nodes those of one CU.  In one workgroup per object the passes over the pixels were one CU's
+ * too; before, a workgroup per level walked them.  Trees of one frame, in us, by levels, in one
+ * workgroup, and now: 300 x 291 pixels 2,070, 4,800, 530; 512 x 512 5,860, 15,850, 3,440;
+ * 1024 x 1024 24,800, 73,800, 13,300; five million pixels in a 4096^2 frame 288,000, 817,000,
+ * 220,000 (of which the exact flux of the whole object, and those of the nodes that need it, are
+ * nearly all).
+ */
+struct DebWide {
+    double rsum, rabs;              /* sums of cd and |cd| */
+    int lev[SXG_MAXNTHRESH], at[SXG_MAXNTHRESH];   /* roots of each level; taken places of each */
+};
+typedef DebObj<true, true, int> DebWideObj;
+
+__device__ inline DebWideObj deb_wide_obj(const DebArgs &a, int r)
+{
+    const int off = a.off[r];
+    return {{a.g_par + off}, a.g_sum + off, a.g_cnt + off, a.g_list + off, a.g_m + off,
+            a.fpia + off, a.cnt[r], a.W, 2 * (a.xmax[r] - a.xmin[r] + 1) + 1};
+}
+/* the object of raw-list entry g, or -1 where it is none of class 4 */
+__device__ inline int deb_wide_root(const DebArgs &a, long g)
+{
+    if (g >= deb_P0(a)) return -1;
+    const int r = a.rawkey[g];
+    return a.cnt[r] > DEB_HALF && a.lstar[r] > 0 ? r : -1;
+}
+/* whether all entries of this workgroup belong to object r (the list is grouped by object) */
+__device__ inline bool deb_wide_one(const DebArgs &a, int r)
+{
+    const long b = (long)blockIdx.x * 256;
+    return r >= 0 && b + 255 < deb_P0(a) && a.rawkey[b] == r && a.rawkey[b + 255] == r;
+}
+
+/* the record of each object, whose number is in rootnc until the nodes are done */
+__global__ void __launch_bounds__(64) k_deb_wide_start(DebArgs a)
+{
+    const int j = blockIdx.x;
+    if (a.pd && j >= a.ccount[4]) return;
+    if (threadIdx.x == 0) {
+        a.rootnc[a.clist[4 * (size_t)a.cstride + j]] = j;
+        a.wide[j].rsum = a.wide[j].rabs = 0.0;
     }
+    a.wide[j].lev[threadIdx.x] = a.wide[j].at[threadIdx.x] = 0;
+}
+
+/* level index, count and sum of each pixel, its neighbours, and the bounds of the root's flux.
+   A level is the number of leading sub-thresholds at or below cd: tau_i <= cd where all up to
+   i are */
+__global__ void __launch_bounds__(256) k_deb_wide_levels(DebArgs a)
+{
+    const long g = (long)blockIdx.x * 256 + threadIdx.x;
+    const int r = deb_wide_root(a, g);
+    double rs = 0.0, ra = 0.0;
+    if (r >= 0) {
+        const DebWideObj t = deb_wide_obj(a, r);
+        const int k = (int)(g - a.off[r]), ls = a.lstar[r];
+        const float *const thr = a.thr + (size_t)r * a.nthresh;
+        const float v = a.cd[t.pl[k]];
+        rs = v;
+        ra = fabs(v);
+        int lo = 0;
+        while (lo < ls && thr[lo + 1] <= v) lo++;
+        t.sum[k] = v;
+        t.cnt[k] = 1;
+        t.m[k] = (unsigned char)lo;
+        t.look(k);
+    }
+    if (deb_wide_one(a, r)) {
+        rs = sxw_sum(rs);
+        ra = sxw_sum(ra);
+        if (threadIdx.x & 63) return;
+    } else if (r < 0) {
+        return;
+    }
+    DebWide &w = a.wide[a.rootnc[r]];
+    atomicAdd(&w.rsum, rs);
+    atomicAdd(&w.rabs, ra);
+}
+
+__global__ void __launch_bounds__(256) k_deb_wide_first(DebArgs a)
+{
+    const long g = (long)blockIdx.x * 256 + threadIdx.x;
+    const int r = deb_wide_root(a, g);
+    if (!__ballot(r >= 0)) return;
+    const DebWideObj t = r >= 0 ? deb_wide_obj(a, r) : DebWideObj{};
+    t.first(r >= 0 ? (int)(g - a.off[r]) : 0, r >= 0);
+}
+
+__global__ void __launch_bounds__(256) k_deb_wide_shorten(DebArgs a)
+{
+    const long g = (long)blockIdx.x * 256 + threadIdx.x;
+    const int r = deb_wide_root(a, g);
+    if (r < 0) return;
+    const DebWideObj t = deb_wide_obj(a, r);
+    for (int round = 0; round < DEB_JUMPS; round++) t.shorten((int)(g - a.off[r]));
+}
+
+__global__ void __launch_bounds__(256) k_deb_wide_join(DebArgs a)
+{
+    const long g = (long)blockIdx.x * 256 + threadIdx.x;
+    const int r = deb_wide_root(a, g);
+    if (r >= 0) deb_wide_obj(a, r).joins((int)(g - a.off[r]));
+}
+
+__global__ void __launch_bounds__(256) k_deb_wide_settle(DebArgs a)
+{
+    __shared__ int s_n[SXG_MAXNTHRESH];
+    const long g = (long)blockIdx.x * 256 + threadIdx.x;
+    const int r = deb_wide_root(a, g);
+    const bool one = deb_wide_one(a, r);   /* the same in every thread */
+    if (one) {
+        if (threadIdx.x < SXG_MAXNTHRESH) s_n[threadIdx.x] = 0;
+        __syncthreads();
+    }
+    if (r < 0) return;
+    int *const lev = a.wide[a.rootnc[r]].lev;
+    const int l = deb_wide_obj(a, r).settle((int)(g - a.off[r]));
+    if (!one) {
+        if (l) atomicAdd(&lev[l], 1);
+        return;
+    }
+    if (l) atomicAdd(&s_n[l], 1);
+    __syncthreads();
+    if (threadIdx.x < SXG_MAXNTHRESH && s_n[threadIdx.x])
+        atomicAdd(&lev[threadIdx.x], s_n[threadIdx.x]);
+}
+
+/* a pixel's count and cd to its root, together for the lanes of a wavefront that share the
+   root of one (four rounds: the roots that many share come up first); the roots into the list */
+__global__ void __launch_bounds__(256) k_deb_wide_sums(DebArgs a)
+{
+    typedef DebTree<true> D;
+    __shared__ int s_n[SXG_MAXNTHRESH], s_b[SXG_MAXNTHRESH];
+    const long g = (long)blockIdx.x * 256 + threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int r = deb_wide_root(a, g);
+    const bool one = deb_wide_one(a, r);
+    if (one) {
+        if (threadIdx.x < SXG_MAXNTHRESH) s_n[threadIdx.x] = 0;
+        __syncthreads();
+    }
+    long root = -1;      /* of another pixel, by raw-list entry */
+    int lev = 0, k = 0;  /* a root's level */
+    double v = 0.0;
+    if (r >= 0) {
+        const DebWideObj t = deb_wide_obj(a, r);
+        k = (int)(g - a.off[r]);
+        const int mk = t.m[k];
+        if (mk > 0) {
+            const D::T w = t.par.ld(k);
+            if (D::lev(w) == mk) {
+                root = a.off[r] + D::idx(w);
+                v = t.sum[k];
+            } else {
+                lev = mk;
+            }
+        }
+    }
+#pragma unroll 1
+    for (int round = 0; round < 4; round++) {
+        const unsigned long long b = __ballot(root >= 0);
+        if (!b) break;
+        const int lead = __builtin_ctzll(b);
+        const long key = __shfl(root, lead);
+        const bool mine = root == key;
+        const int c = __popcll(__ballot(mine));
+        const double s = sxw_sum(mine ? v : 0.0);
+        if (lane == lead) {
+            atomicAdd(&a.g_cnt[key], (D::T)c);
+            atomicAdd(&a.g_sum[key], s);
+        }
+        if (mine) root = -1;
+    }
+    if (root >= 0) {
+        atomicAdd(&a.g_cnt[root], (D::T)1);
+        atomicAdd(&a.g_sum[root], v);
+    }
+    if (r < 0) return;
+    DebWide &w = a.wide[a.rootnc[r]];
+    int *const list = a.g_list + a.off[r];
+    if (!one) {
+        if (!lev) return;
+        int at = atomicAdd(&w.at[lev], 1);
+        for (int l = SXG_MAXNTHRESH - 1; l > lev; l--) at += w.lev[l];
+        list[at] = k;
+        return;
+    }
+    const int place = lev ? atomicAdd(&s_n[lev], 1) : 0;
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        const int at = deb_level_start(w.lev), c = s_n[lane];
+        s_b[lane] = c ? at + atomicAdd(&w.at[lane], c) : 0;
+    }
+    __syncthreads();
+    if (lev) list[s_b[lev] + place] = k;
+}
+
+__global__ void __launch_bounds__(1024) k_deb_wide_nodes(DebArgs a)
+{
+    __shared__ int s_lev[SXG_MAXNTHRESH], s_at[SXG_MAXNTHRESH];
+    __shared__ float tthr[SXG_MAXNTHRESH + 1];
+    const int j = blockIdx.x, tid = threadIdx.x;
+    if (a.pd && j >= a.ccount[4]) return;
+    const int r = a.clist[4 * (size_t)a.cstride + j];
+    const DebWideObj t = deb_wide_obj(a, r);
+    const DebWide &w = a.wide[j];
+    const int ls = a.lstar[r];
+    if (tid < 64) {
+        const int at = deb_level_start(w.lev);
+        s_lev[tid] = w.lev[tid];
+        s_at[tid] = at + w.lev[tid];
+        if (tid < ls) tthr[tid + 1] = a.thr[(size_t)r * a.nthresh + tid + 1];
+    }
+    __syncthreads();
+    Comp *const C = a.comps + a.compoff[r];
+    const int nk = deb_nodes<1024>(a, t, t.pl, t.n, ls, s_lev, s_at, tthr, w.rsum, w.rabs, C);
+    if (tid == 0) {
+        if (nk == 0) C[0] = {0, t.pl[0], 0, t.n - 1};
+        a.rootnc[r] = a.rootkept[r] = max(nk, 1);
+    }
+}
+
+__global__ void __launch_bounds__(256) k_deb_wide_assign(DebArgs a)
+{
+    const long g = (long)blockIdx.x * 256 + threadIdx.x;
+    int r = deb_wide_root(a, g);
+    if (r >= 0 && a.rootkept[r] < 2) r = -1;
+    if (!__ballot(r >= 0)) return;
+    const DebWideObj t = r >= 0 ? deb_wide_obj(a, r) : DebWideObj{};
+    const int *const slot = reinterpret_cast<const int *>(t.sum);
+    const int off = r >= 0 ? a.off[r] : 0;
+    t.assign((int)(g - off), r >= 0, slot, slot + t.n, a.kcomp + off,
+             r >= 0 ? a.comps + a.compoff[r] : nullptr);
 }
 
 /* the objects of class 3 into out, largest first (ties in list order), so that the longest
@@ -1309,7 +1635,7 @@ __global__ void __launch_bounds__(256) k_deb_zero(int *v, long n)
    2^31 is an overflow) and the class words of the counter block against theirs; on any
    overflow of the frame the class counts are zeroed so that no tree kernel has work */
 struct DebGuardCaps {
-    long long lds[3], cls[4];   /* LDS bytes of classes 0..2, objects of classes 0..3 */
+    long long lds[3], cls[DEB_NCLASS];   /* LDS bytes of classes 0..2, objects of each class */
 };
 
 __global__ void k_deb_plan_guard(const unsigned long long *dw, PlanDev *pd, int *cc,
@@ -1319,12 +1645,13 @@ __global__ void k_deb_plan_guard(const unsigned long long *dw, PlanDev *pd, int 
     if (dw[2] > (unsigned long long)cap_tot || (long long)*ntot > cap_tot || *ntot < 0)
         pd->ovf |= 1 << PL_NTOT;
     for (int c = 0; c < 3; c++)
-        if (cc[4 + c] < 0 || (long long)cc[4 + c] > gc.lds[c]) pd->ovf |= 1 << (PL_LDS0 + c);
-    for (int c = 0; c < 4; c++)
+        if (cc[DEB_CLDS + c] < 0 || (long long)cc[DEB_CLDS + c] > gc.lds[c])
+            pd->ovf |= 1 << (PL_LDS0 + c);
+    for (int c = 0; c < DEB_NCLASS; c++)
         if (cc[c] < 0 || (long long)cc[c] > gc.cls[c]) pd->ovf |= 1 << (PL_C0 + c);
     if (pd->ovf) {
         pd->nfg = pd->nraw = pd->npix = pd->nobj = pd->nsurv = 0;
-        for (int c = 0; c < 7; c++) cc[c] = 0;
+        for (int c = 0; c < DEB_CPIX; c++) cc[c] = 0;
     }
 }
 
@@ -1334,7 +1661,7 @@ __global__ void k_deb_plan_info(const unsigned long long *dw, const int *cc, Pla
     if (threadIdx.x != 0) return;
     pd->deb_pixels = (long long)dw[0];
     pd->deb_labels = (long long)dw[1];
-    for (int c = 0; c < 4; c++) pd->class_pixels[c] = cc[7 + c];
+    for (int c = 0; c < 4; c++) pd->class_pixels[c] = cc[DEB_CPIX + c];
 }
 
 /* --------------------------------------------------------------- host side ---- */
@@ -1405,7 +1732,7 @@ extern "C" int parcel_out(float basethresh, int n_thresh, int deb_minarea, size_
     auto *top2 = sxg_take<unsigned>("deb.top2", nr);
     int *nmax = sxg_take<int>("deb.nmax", nr);
     int *lstar = sxg_take<int>("deb.lstar", nr);
-    int *clist = sxg_take<int>("deb.clist", 4 * nr);
+    int *clist = sxg_take<int>("deb.clist", DEB_NCLASS * nr);
     int *ccount = sxg_take<int>("deb.ccount", DEB_NCOUNT);
     auto *dwork = sxg_take<unsigned long long>("deb.dwork", 3);
     int *kcomp = sxg_take<int>("deb.kcomp", (size_t)(P0 > 0 ? P0 : 1));
@@ -1451,15 +1778,15 @@ extern "C" int parcel_out(float basethresh, int n_thresh, int deb_minarea, size_
             /* the capacities stand for the counts; the guards check the device counts
                against them (the node total first, then every class) */
             ntot = (int)pl->cap[PL_NTOT];
-            for (int c = 0; c < 4; c++) cc[c] = (int)pl->cap[PL_C0 + c];
+            for (int c = 0; c < DEB_NCLASS; c++) cc[c] = (int)pl->cap[PL_C0 + c];
             /* the class's LDS: what its largest object may need, or less when the plan asks
                less */
             const int caps[3] = {cap0, cap1, cap2};
             DebGuardCaps gc;
             for (int c = 0; c < 3; c++)
-                gc.lds[c] = cc[4 + c] =
+                gc.lds[c] = cc[DEB_CLDS + c] =
                     (int)std::min<int64_t>(pl->cap[PL_LDS0 + c], deb_lds_bytes(caps[c]));
-            for (int c = 0; c < 4; c++) gc.cls[c] = cc[c];
+            for (int c = 0; c < DEB_NCLASS; c++) gc.cls[c] = cc[c];
             hipLaunchKernelGGL(k_deb_plan_guard, dim3(1), dim3(64), 0, st, dwork, pd, ccount,
                                dtot, (long long)pl->cap[PL_NTOT], gc);
         } else {
@@ -1470,11 +1797,11 @@ extern "C" int parcel_out(float basethresh, int n_thresh, int deb_minarea, size_
                 return -1;
             }
             S.deb_pixels = (int64_t)dw[0];
-            for (int c = 0; c < 4; c++) S.deb_class_pixels[c] = cc[7 + c];
+            for (int c = 0; c < 4; c++) S.deb_class_pixels[c] = cc[DEB_CPIX + c];
             S.deb_labels = (int64_t)dw[1];
             S.seen.cap[PL_NTOT] = ntot;
-            for (int c = 0; c < 4; c++) S.seen.cap[PL_C0 + c] = cc[c];
-            for (int c = 0; c < 3; c++) S.seen.cap[PL_LDS0 + c] = cc[4 + c];
+            for (int c = 0; c < DEB_NCLASS; c++) S.seen.cap[PL_C0 + c] = cc[c];
+            for (int c = 0; c < 3; c++) S.seen.cap[PL_LDS0 + c] = cc[DEB_CLDS + c];
         }
         a.comps = sxg_take<Comp>("deb.comps", (size_t)ntot + 1);
         if (!a.comps) return -1;
@@ -1485,6 +1812,7 @@ extern "C" int parcel_out(float basethresh, int n_thresh, int deb_minarea, size_
            Everything they read was finished by the synchronisation above. */
         int nside = 0;
         const bool use_side = !S.single_stream && !pl && sxg_option(SXG_OPT_SIDE_STREAMS) != 0;
+        static_assert(SXG_NSIDE >= DEB_NCLASS - 1, "a side stream for each class but the first");
         /* the dynamic-LDS limit is an attribute of the function, shared by every context:
            it is raised once, to the most any class asks for (DEB_LDS_LIMIT), never per
            launch (batch workers launch these kernels from several host threads) */
@@ -1507,7 +1835,7 @@ extern "C" int parcel_out(float basethresh, int n_thresh, int deb_minarea, size_
             return -1;
         }
         auto launch_lds = [&](const void *fn, int cls, int nt) -> bool {
-            const size_t lds = (size_t)cc[4 + cls];
+            const size_t lds = (size_t)cc[DEB_CLDS + cls];
             if (lds > DEB_LDS_LIMIT) {
                 sxg_set_error("parcel_out: LDS request above the limit (internal error)");
                 return false;
@@ -1522,15 +1850,36 @@ extern "C" int parcel_out(float basethresh, int n_thresh, int deb_minarea, size_
             if (side) SXG_HIP_RET(hipEventRecord(S.side_ev[nside++], ks), false);
             return true;
         };
-        if (cc[3] > 0) {
+        if (cc[3] > 0 || cc[4] > 0) {
             a.g_sum = sxg_take<double>("deb.g_sum", (size_t)P0);
-            a.g_par = sxg_take<unsigned long long>("deb.g_par", (size_t)P0);
             a.g_cnt = sxg_take<unsigned long long>("deb.g_cnt", (size_t)P0);
             a.g_list = sxg_take<int>("deb.g_list", (size_t)P0);
+            if (!a.g_sum || !a.g_cnt || !a.g_list) return -1;
+        }
+        if (cc[4] > 0) {
+            a.g_par = sxg_take<unsigned long long>("deb.g_par", (size_t)P0);
             a.g_m = sxg_take<unsigned char>("deb.g_m", (size_t)P0);
+            a.wide = sxg_take<DebWide>("deb.wide", (size_t)cc[4]);
+            if (!a.g_par || !a.g_m || !a.wide) return -1;
+            hipStream_t ks = use_side ? S.side[nside] : st;
+            const dim3 gp(sxg_div_up(P0, 256)), gw(cc[4]);
+            sxg_kt_begin_on(SXG_KT_DEB_LVPAR, ks);
+            hipLaunchKernelGGL(k_deb_wide_start, gw, dim3(64), 0, ks, a);
+            hipLaunchKernelGGL(k_deb_wide_levels, gp, dim3(256), 0, ks, a);
+            hipLaunchKernelGGL(k_deb_wide_first, gp, dim3(256), 0, ks, a);
+            hipLaunchKernelGGL(k_deb_wide_shorten, gp, dim3(256), 0, ks, a);
+            hipLaunchKernelGGL(k_deb_wide_join, gp, dim3(256), 0, ks, a);
+            hipLaunchKernelGGL(k_deb_wide_settle, gp, dim3(256), 0, ks, a);
+            hipLaunchKernelGGL(k_deb_wide_sums, gp, dim3(256), 0, ks, a);
+            hipLaunchKernelGGL(k_deb_wide_nodes, gw, dim3(1024), 0, ks, a);
+            hipLaunchKernelGGL(k_deb_wide_assign, gp, dim3(256), 0, ks, a);
+            sxg_kt_end_on(SXG_KT_DEB_LVPAR, ks);
+            if (use_side) SXG_HIP_RET(hipEventRecord(S.side_ev[nside++], ks), -1);
+        }
+        if (cc[3] > 0) {
             /* class 3 largest first */
             int *clist3 = sxg_take<int>("deb.clist3", 4 * nr);
-            if (!a.g_sum || !a.g_par || !a.g_cnt || !a.g_list || !a.g_m || !clist3) return -1;
+            if (!clist3) return -1;
             DebArgs a3 = a;
             a3.clist = clist3;
             hipStream_t ks = use_side ? S.side[nside] : st;

@@ -574,7 +574,9 @@ static void graph_release()
 /* capacity of a count seen in calibration: the margin, and a few units of slack */
 static FramePlan plan_from(const FramePlan &seen, int margin)
 {
-    static const int64_t slack[PL_N] = {4096, 64, 1024, 256, 16, 8, 4, 4, 0, 0, 0, 128};
+    /* the trees that the whole chip builds have none: where the calibration saw no such blend,
+       its nine launches are left out, and a frame that has one runs again eagerly */
+    static const int64_t slack[PL_N] = {4096, 64, 1024, 256, 16, 8, 4, 4, 0, 0, 0, 0, 128};
     FramePlan pl;
     for (int k = 0; k < PL_N; k++) {
         if (k >= PL_LDS0 && k <= PL_LDS2) continue;

@@ -156,7 +156,7 @@ enum PlanCap {
     PL_NRAW,      /* raw objects */
     PL_NPIX,      /* pixels of raw objects */
     PL_NTOT,      /* node capacity of the deblending trees */
-    PL_C0, PL_C1, PL_C2, PL_C3,     /* raw objects per deblending size class */
+    PL_C0, PL_C1, PL_C2, PL_C3, PL_C4,   /* raw objects per deblending size class */
     PL_LDS0, PL_LDS1, PL_LDS2,      /* LDS bytes of the tree workgroups of classes 0..2 */
     PL_NOBJ,      /* deblended objects */
     PL_N

@@ -263,7 +263,7 @@ typedef struct {
        the APER outer radius, inside both AUTO ellipses) */
     int64_t phot_pixels;
     /* pixels of the multi-peak raw objects in each deblending size class (0, 1, 2: trees in
-       LDS with 256, 512 and 1024 lanes, 3: global-memory trees) */
+       LDS with 256, 512 and 1024 lanes, 3: trees with state in global memory) */
     int64_t deb_class_pixels[4];
 } sxg_frame_info;
 int sxg_get_frame_info(sxg_frame_info *info);
@@ -414,8 +414,8 @@ enum sxg_kernel_id {
     SXG_KT_DEB_LEVELS, SXG_KT_DEB_OBJECTS, SXG_KT_ANALYSE, SXG_KT_CLEAN, SXG_KT_SEG,
     SXG_KT_DEB_LMAX, SXG_KT_OBJ_SORT, SXG_KT_PHOT,
     /* the deblending tree kernels one by one, each timed on the stream it runs on: size
-       classes 0, 1, 2 (k_deb_tree_lds) and the global-memory trees (k_deb_tree_glb);
-       SXG_KT_DEB_LVPAR times nothing any more */
+       classes 0, 1, 2 (k_deb_tree_lds), the larger ones of up to 29,696 pixels
+       (k_deb_tree_glb), and the chain of kernels for those beyond (k_deb_wide_*) */
     SXG_KT_DEB_TREE0, SXG_KT_DEB_TREE1, SXG_KT_DEB_TREE2, SXG_KT_DEB_TREE_GLB, SXG_KT_DEB_LVPAR,
     SXG_NKT
 };
