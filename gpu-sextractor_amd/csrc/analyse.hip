@@ -401,7 +401,7 @@ __global__ void __launch_bounds__(256) k_analyse(AnaArgs A)
     if (slot < nobj) ana_object<SXW_ROWS>(A, A.order[slot], s_rows);
 }
 
-__global__ void k_ana_zero2(int *p)
+__global__ void k_ana_zero(int *p)
 {
     if (threadIdx.x < 3) p[threadIdx.x] = 0;
 }
@@ -463,7 +463,7 @@ extern "C" void analyse_gpu(double flagobj_poserr_mx2, int flagobj_peakx, int fl
     A.pd = S.plan ? S.pdev : nullptr;
     sxg_stage_begin(ST_ANALYSE);
     /* the counters of k_obj_order (a fill kernel: no memset node in a graph) */
-    hipLaunchKernelGGL(k_ana_zero2, dim3(1), dim3(64), 0, S.stream, order + 2 * numobj);
+    hipLaunchKernelGGL(k_ana_zero, dim3(1), dim3(64), 0, S.stream, order + 2 * numobj);
     hipLaunchKernelGGL(k_obj_order, dim3(sxg_div_up(numobj, 256)), dim3(256), 0, S.stream,
                        S.objoff, numobj, order + 2 * (size_t)numobj, order, A.pd);
     sxg_kt_begin(SXG_KT_ANALYSE);

@@ -53,9 +53,9 @@
  *   k_deb_wide_*     the same passes over the pixels of the objects above 29,696 pixels, a
  *                    kernel each, all state in global memory
  *   k_deb_objlist    one wavefront per raw object: its kept nodes -> objects
- *   k_deb_pre        one wavefront per object: FULL preanalysis over the node's level
- *                    pixels (kcomp names them; lanes compute the terms, the raster-order
- *                    sums are transposed folds: sxg_wave.h)
+ *   k_deb_pre        a row of 16 lanes, a wavefront or a workgroup per object: FULL
+ *                    preanalysis over the node's level pixels (kcomp names them; lanes compute
+ *                    the terms, the sums are folded in raster order: sxg_wave.h)
  *   k_deb_gather     one lane per raw pixel: gatherup of the pixels no kept node holds
  *   then the raw pixels are regrouped by object, stably (opix, objoff): every later
  *   per-object pass reads one contiguous raster-ordered range
@@ -67,7 +67,6 @@
 #include "sxg_objects.h"
 #include "sxg_wave.h"
 
-#define DW 64
 /* size classes of the raw objects with a tree (k_deb_classify), and the words of the
    per-frame counter block (DebArgs::ccount): objects per class, the largest LDS need of
    classes 0..2, pixels per class (3 and 4 together) */
@@ -1327,7 +1326,7 @@ struct ObjArgs {
     int *objraw, *objcomp;  /* raw object and component of each object */
     int *alloc;             /* frame-wide object index of each raw pixel */
     const float *sub;       /* background-subtracted frame */
-    int *okey, *oval;       /* object index / pixel of each raw-list entry (sort input) */
+    int *okey;              /* object index of each raw-list entry */
     ObjCols o;
     int nobj;
     const int *order;       /* objects in launch order: those of large raw objects first */
@@ -1508,7 +1507,7 @@ __global__ void __launch_bounds__(256) k_deb_pre(ObjArgs A)
 }
 
 /* gatherup: every unassigned pixel goes to the nearest kept object of its raw object
-   in the ellipse metric (first minimum in object order); then the sort keys */
+   in the ellipse metric (first minimum in object order); then the object of every entry */
 __global__ void __launch_bounds__(256) k_deb_gather(ObjArgs A, int *objcnt, int2 *objspan, long nz)
 {
     const long g = (long)blockIdx.x * 256 + threadIdx.x;
@@ -1545,7 +1544,6 @@ __global__ void __launch_bounds__(256) k_deb_gather(ObjArgs A, int *objcnt, int2
         a = A.alloc[p];
     }
     A.okey[g] = a;
-    A.oval[g] = p;
 }
 
 /* pixels per object, and for those of split raw objects the first and last list entry of
@@ -1806,10 +1804,10 @@ extern "C" int parcel_out(float basethresh, int n_thresh, int deb_minarea, size_
         a.comps = sxg_take<Comp>("deb.comps", (size_t)ntot + 1);
         if (!a.comps) return -1;
         sxg_kt_begin(SXG_KT_DEB_LEVELS);
-        /* one launch per class; LDS: the class's node table, then its largest object's
-           pixels */
-        /* the classes run side by side: each kernel lasts as long as its slowest tree.
-           Everything they read was finished by the synchronisation above. */
+        /* one launch per class (LDS: the words of its largest object's pixels), side by side:
+           each kernel lasts as long as its slowest tree.  What they read was written on the
+           context's stream ahead of the kernel that sent the counts, and the host has seen the
+           number that this kernel stores last, so a launch on a side stream comes after it. */
         int nside = 0;
         const bool use_side = !S.single_stream && !pl && sxg_option(SXG_OPT_SIDE_STREAMS) != 0;
         static_assert(SXG_NSIDE >= DEB_NCLASS - 1, "a side stream for each class but the first");
@@ -1934,15 +1932,12 @@ extern "C" int parcel_out(float basethresh, int n_thresh, int deb_minarea, size_
         A.nobj = nobj;
         A.objraw = sxg_take<int>("obj.raw", nobj);
         A.objcomp = sxg_take<int>("obj.comp", nobj);
-        int *k0 = sxg_take<int>("opix.k0", P0), *v0 = sxg_take<int>("opix.v0", P0);
-        int *v1 = sxg_take<int>("opix.v1", P0);
+        int *okey = sxg_take<int>("opix.key", P0), *opix = sxg_take<int>("opix.pix", P0);
         int2 *objspan = sxg_take<int2>("obj.pixspan", (size_t)nobj + 1);
         int *objcnt = sxg_take<int>("obj.pixcount", (size_t)nobj + 1);
         int *objoff = sxg_take<int>("obj.pixoff", (size_t)nobj + 1);
-        if (!A.objraw || !A.objcomp || !k0 || !v0 || !v1 || !objspan || !objcnt || !objoff)
-            return -1;
-        A.okey = k0;
-        A.oval = v0;
+        if (!A.objraw || !A.objcomp || !okey || !opix || !objspan || !objcnt || !objoff) return -1;
+        A.okey = okey;
         const int gp = sxg_div_up(P0, 256);
         sxg_kt_begin(SXG_KT_DEB_OBJECTS);
         int *order = sxg_take<int>("pre.order", 2 * (size_t)nobj + 3);
@@ -1974,11 +1969,11 @@ extern "C" int parcel_out(float basethresh, int n_thresh, int deb_minarea, size_
             sxg_scan_excl(objcnt, objoff, nobj + 1, nullptr, st);
         else
             sxg_scan_excl(objcnt, objoff, nobj, objoff + nobj, st);
-        hipLaunchKernelGGL(k_obj_place1, dim3(gp), dim3(256), 0, st, A, (const int *)objoff, v1);
+        hipLaunchKernelGGL(k_obj_place1, dim3(gp), dim3(256), 0, st, A, (const int *)objoff, opix);
         hipLaunchKernelGGL(k_obj_place_multi, dim3(sxg_div_up(nobj, 4)), dim3(256), 0, st, A,
-                           (const int *)objoff, (const int2 *)objspan, v1);
+                           (const int *)objoff, (const int2 *)objspan, opix);
         sxg_kt_end(SXG_KT_OBJ_SORT);
-        S.opix = v1;
+        S.opix = opix;
         S.objoff = objoff;
     }
     sxg_stage_end(ST_DEBLEND);

@@ -232,11 +232,6 @@ struct SxgState {
     /* deblending and objects */
     int nthresh = 0;
     int nobj = 0;
-    DevBuf thr;      /* float[nraw * nthresh] sub-thresholds */
-    DevBuf lvl;      /* int[nthresh * P0] component of each raw pixel per level */
-    DevBuf comps;    /* component table */
-    DevBuf objs;     /* object columns (SoA) */
-    DevBuf rootobj;  /* per root: first object, object count */
     int *opix = nullptr;      /* int[P0]: raw pixels grouped by object, raster order inside */
     int *objoff = nullptr;    /* int[nobj + 1]: start of each object in opix */
     int nsurv = 0;
@@ -359,9 +354,8 @@ size_t sxg_radix_hist(int n);
 int sxg_radix_sort(int *k0, int *v0, int *k1, int *v1, int n, int nbits, int *hist,
                    hipStream_t s, const int *nd = nullptr);
 /* Planned runs: queue the check of the device count *v against cap (bit: its PlanCap);
-   above it, or after an earlier overflow of the frame, the frame's counts are zeroed
-   (also the deblending class counts ccount[0..3] and [8] when ccount is given). */
-void sxg_plan_guard(int *v, int64_t cap, int bit, int *ccount = nullptr);
+   above it, or after an earlier overflow of the frame, the frame's counts are zeroed. */
+void sxg_plan_guard(int *v, int64_t cap, int bit);
 /* the capacity of count k in a planned run, else n itself */
 inline int64_t sxg_plan_cap(const SxgState &S, int k, int64_t n)
 {

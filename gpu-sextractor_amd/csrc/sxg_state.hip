@@ -281,8 +281,7 @@ extern "C" void sxg_release(void)
 {
     SxgState &S = sxg_state();
     if (S.stream) (void)hipStreamSynchronize(S.stream);
-    DevBuf *bufs[] = {&S.img, &S.cd, &S.aux, &S.backbuf, &S.scan_tmp, &S.thr, &S.lvl,
-                      &S.comps, &S.objs, &S.rootobj};
+    DevBuf *bufs[] = {&S.img, &S.cd, &S.aux, &S.backbuf, &S.scan_tmp};
     for (DevBuf *b : bufs) b->release();
     sxg_release_named();
     S.ranked = S.counted = S.exposed = false;
@@ -561,7 +560,7 @@ void sxg_compact_mask(const unsigned long long *m, long nw, int *out, int *count
 }
 
 /* ------------------------------------------------------------ plan guards ---- */
-__global__ void k_plan_guard(int *v, long long cap, int bit, PlanDev *pd, int *cc)
+__global__ void k_plan_guard(int *v, long long cap, int bit, PlanDev *pd)
 {
     if (threadIdx.x != 0) return;
     const int x = *v;
@@ -570,19 +569,15 @@ __global__ void k_plan_guard(int *v, long long cap, int bit, PlanDev *pd, int *c
         /* the frame is run again eagerly: nothing after this point has work to do */
         *v = 0;
         pd->nfg = pd->nraw = pd->npix = pd->nobj = pd->nsurv = 0;
-        if (cc) {
-            for (int c = 0; c < 4; c++) cc[c] = 0;
-            cc[8] = 0;
-        }
     }
 }
 
-void sxg_plan_guard(int *v, int64_t cap, int bit, int *ccount)
+void sxg_plan_guard(int *v, int64_t cap, int bit)
 {
     SxgState &S = sxg_state();
     if (!S.plan) return;
     hipLaunchKernelGGL(k_plan_guard, dim3(1), dim3(64), 0, S.stream, v, (long long)cap, bit,
-                       S.pdev, ccount);
+                       S.pdev);
 }
 
 /* ------------------------------------------------------- named buffers ---- */
