@@ -1,6 +1,7 @@
 """The spline tables over the numbers of mesh columns and rows where their kernels change: the
-recurrences' groups of eight, 64 columns a workgroup, the row tables' LDS limit (163 columns)
-and the column recurrences' (256 rows), against the oracle bit for bit."""
+recurrences' groups of eight, 64 columns a workgroup, the row tables' LDS limit (168 columns:
+131,072 bytes of three tables with a stride of 65 floats) and the column recurrences' (256 rows),
+against the oracle bit for bit."""
 import numpy as np
 import pytest
 
@@ -12,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("nbx,nby", [(1, 1), (1, 9), (2, 2), (3, 11), (9, 3), (10, 10), (11, 18),
-                                     (32, 5), (33, 2), (65, 7), (85, 3), (163, 3), (164, 2),
+                                     (32, 5), (33, 2), (65, 7), (85, 3), (168, 3), (169, 2),
+                                     (169, 1), (300, 4),
                                      (4, 256), (3, 257)])
 @pytest.mark.parametrize("bs", [4, 7])
 def test_spline_tables(nbx, nby, bs):
