@@ -73,6 +73,18 @@ def test_several_large_objects(coarse, holes):
         compare(sexgpu.run_frame(img, sexgpu.Params(**KW)), o)
 
 
+@pytest.mark.parametrize("kw", [dict(ext_minarea=1), dict(deblend_nthresh=64),
+                                dict(deblend_mincont=0.0)])
+def test_large_objects_parameter_variants(kw):
+    """One-pixel nodes, 64 levels, every node significant."""
+    kw = dict(KW, **kw)
+    img = blends((260, 330), [(2, 1, 182, 173), (190, 0, 60, 330)], False, 0.05)
+    print("large object, %s" % kw, flush=True)
+    o = sxo.run(img, **kw)
+    assert np.asarray(o["raw_count"]).max() > 29696
+    compare(sexgpu.run_frame(img, sexgpu.Params(**kw)), o)
+
+
 def test_large_objects_in_a_graph():
     """Planned runs: a graph whose calibration had such objects, and one whose had none and
     whose frame then gets one (it runs again eagerly)."""

@@ -108,73 +108,77 @@ def test_catalog_rows_match_columns(frame1024, masks):
     assert np.array_equal(fe, np.sqrt(g["fluxerr"].astype(np.float64)).astype(np.float32))
 
 
-KNOBS = ("deb_lds_tiny", "deb_lds_small", "deb_lds_large", "deb_table", "deb_glb_levels",
-         "deb_order_full")
+KNOBS = ("deb_lds_tiny", "deb_lds_small", "deb_lds_large", "deb_order_full")
+# every object with a tree in one class: 256, 512 and 1024 lanes in LDS, and one workgroup
+# with its sums in global memory
+ONE_CLASS = [(6400, 6400, 6400, 4096), (0, 6400, 6400, 4096), (0, 0, 6400, 4096),
+             (0, 0, 0, 4096)]
 
 
-@pytest.mark.parametrize("caps", [(0, 0, 0, 0, 1, 4096), (0, 0, 0, 0, 0, 4096),
-                                  (0, 64, 256, 0, 1, 4096), (0, 6400, 6400, 0, 1, 4096),
-                                  (256, 1024, 6144, 0, 1, 4096), (6400, 6400, 6400, 0, 1, 4096),
-                                  (256, 1024, 6144, 1, 1, 4096), (256, 1024, 6144, 5, 1, 4096),
-                                  (0, 0, 0, 3, 1, 4096), (0, 0, 0, 3, 0, 4096),
-                                  (0, 64, 256, 0, 2000, 4096), (0, 64, 256, 0, 2000, 0),
-                                  (0, 0, 0, 0, 1, 0), (0, 0, 0, 0, 0, 0)])
+def run_with(knobs, values, img, p):
+    old = [sexgpu.get_option(k) for k in knobs]
+    try:
+        for k, v in zip(knobs, values):
+            sexgpu.set_option(k, v)
+        return sexgpu.run_frame(img, p)
+    finally:
+        for k, v in zip(knobs, old):
+            sexgpu.set_option(k, v)
+
+
+@pytest.mark.parametrize("caps", ONE_CLASS + [(0, 0, 0, 0), (0, 64, 256, 4096), (0, 64, 256, 0),
+                                              (64, 256, 6144, 4096)])
 def test_deblend_kernel_variants(masks, caps):
-    """Every deblending kernel variant (LDS 256- and 1024-lane workgroups, global
-    scratch with the level components built level by level or, from a size on, all
-    levels in parallel, launched largest first or only the level-parallel ones ordered;
-    the tree's node table in LDS or moved to global memory when it outgrows its LDS
-    share) gives the oracle's result: the options move raw objects between them."""
+    """Every deblending size class (LDS workgroups of 256, 512 and 1024 lanes, one workgroup
+    with its sums in global memory, the objects of that class launched largest first or in any
+    order) gives the oracle's result: the options move raw objects between them."""
     img = sexgpu.synth("crowded4096", width=1024, height=1024, nsrc=167000 // 16, seed=1201)
     m = masks["gauss_3p0_7x7"]
-    old = [sexgpu.get_option(k) for k in KNOBS]
-    try:
-        for k, v in zip(KNOBS, caps):
-            sexgpu.set_option(k, v)
-        g = sexgpu.run_frame(img, _params(m))
-    finally:
-        for k, v in zip(KNOBS, old):
-            sexgpu.set_option(k, v)
+    g = run_with(KNOBS, caps, img, _params(m))
     compare(g, _oracle(img, m))
     assert (g["level"] > 0).sum() > 20
 
 
+@pytest.mark.parametrize("caps", ONE_CLASS)
 @pytest.mark.parametrize("kw", [dict(ext_minarea=1), dict(deblend_nthresh=64),
                                 dict(deblend_mincont=0.0)])
-def test_level_parallel_parameter_variants(frame1024, masks, kw):
-    """Every multi-peak object built level-parallel (one workgroup per object and level)
-    under the parameters that stress that build: one-pixel nodes (as many node records
-    as pixels per level), 64 levels, every node significant."""
+def test_tree_parameter_variants(frame1024, masks, kw, caps):
+    """Every class under the parameters that stress its max-trees: one-pixel nodes, 64 levels,
+    every node significant."""
     m = masks["default"]
-    old = [sexgpu.get_option(k) for k in KNOBS]
-    try:
-        for k, v in zip(KNOBS, (0, 0, 0, 0, 1, 4096)):
-            sexgpu.set_option(k, v)
-        g = sexgpu.run_frame(frame1024, _params(m, **kw))
-    finally:
-        for k, v in zip(KNOBS, old):
-            sexgpu.set_option(k, v)
-    compare(g, _oracle(frame1024, m, **kw))
+    compare(run_with(KNOBS, caps, frame1024, _params(m, **kw)), _oracle(frame1024, m, **kw))
 
 
 def test_dense_blends_default_paths(masks):
-    """A 2048^2 frame of the dense regime (fluxes from 3000 ADU; blends of 10k-20k pixels)
-    gives the oracle's result with the default options, where the largest trees are built
-    one workgroup per level and the other global-memory trees one workgroup each, and
-    with every global-memory tree built one workgroup each."""
+    """A 2048^2 frame of the dense regime (fluxes from 3000 ADU; blends of up to 20,000 pixels)
+    gives the oracle's result with the default options, where its largest trees are those of one
+    workgroup with its sums in global memory, in both launch orders."""
     img = sexgpu.synth("crowded4096", width=2048, height=2048, nsrc=167000 // 4, seed=1301,
                        fmin=3000.0)
     m = masks["gauss_3p0_7x7"]
     ref = _oracle(img, m)
-    lvmin = sexgpu.get_option("deb_glb_levels")
     sizes = np.asarray(ref["raw_count"])
-    assert (sizes >= lvmin).sum() >= 4 and ((sizes > 6144) & (sizes < lvmin)).sum() >= 10
-    try:
-        for v in (lvmin, 0):
-            sexgpu.set_option("deb_glb_levels", v)
-            compare(sexgpu.run_frame(img, _params(m)), ref)
-    finally:
-        sexgpu.set_option("deb_glb_levels", lvmin)
+    assert (sizes > 6144).sum() >= 14 and sizes.max() <= 29696
+    for full in (sexgpu.get_option("deb_order_full"), 0):
+        compare(run_with(("deb_order_full",), (full,), img, _params(m)), ref)
+
+
+def test_options_without_effect(frame1024, masks):
+    """Options whose kernels are gone are still taken, in their ranges, and change nothing."""
+    p = _params(masks["default"])
+    ref = _oracle(frame1024, masks["default"])
+    for name, values in (("deb_table", (0, 1, 2048)), ("deb_glb_levels", (0, 2000, 1 << 30)),
+                         ("mesh_rows", (0, 1, 8))):
+        old = sexgpu.get_option(name)
+        try:
+            for v in values:
+                sexgpu.set_option(name, v)
+                assert sexgpu.get_option(name) == v
+            compare(sexgpu.run_frame(frame1024, p), ref)
+            with pytest.raises(ValueError):
+                sexgpu.set_option(name, values[-1] + 1)
+        finally:
+            sexgpu.set_option(name, old)
 
 
 def test_option_range():
