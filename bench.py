@@ -120,8 +120,8 @@ SINGLE_KERNELS = {
 # figure).  "conv_fused" is the whole-frame runs' k_subconv_det<7>, the kernel the conv
 # timer brackets when no subback runs.
 MEASURED_TRAFFIC_CROWDED4096 = {
-    "meshstat": 6.748e7, "meshmode": 6.858e7, "analyse": 6.982e7, "conv_fused": 2.749e8,
-    "deb_tree0": 1.067e7, "deb_tree1": 1.136e6, "deb_tree2": 9.297e5,
+    "meshstat": 6.750e7, "meshmode": 6.859e7, "analyse": 6.983e7, "conv_fused": 2.749e8,
+    "deb_tree0": 1.069e7, "deb_tree1": 1.146e6, "deb_tree2": 9.445e5,
 }
 
 
@@ -517,7 +517,7 @@ def wide8192(args):
 
 # HBM bytes per frame of the photometry kernels (label map, labels of the raw pixels,
 # order, k_endobject, count), from profiles/photometry_crowded4096_trace_and_traffic.md
-PHOT_TRAFFIC_CROWDED4096 = 3.895e8
+PHOT_TRAFFIC_CROWDED4096 = 3.896e8
 
 PHOT_ORACLE = {"flux_isocor": "flux_isocor", "flux_aper": "flux_aper",
                "fluxerr_aper": "fluxerr_aper", "mag_aper": "mag_aper",

@@ -945,7 +945,8 @@ __device__ void fb_global(const float *back, const float *sigma, int np, float *
 }
 
 /* (float)(v / 6.0): a float division gives the same.  v / 6 is either a float or its binary
-   digits end in a repeating 01, which lies a third of a unit from a tie at any precision, so
+   digits end in a repeating 01 or 10: cut at any precision, what is left is a third or two
+   thirds of a unit, a sixth of one from a tie, so
    the rounding to double in between cannot make one. */
 __device__ inline float sixth(float v) { return v / 6.0f; }
 

@@ -363,7 +363,10 @@ __device__ inline int deb_sig_bound(double s, double sabs, int n, float b, doubl
  * is the whole object, level 0).  A word holds the parent's level over its complemented
  * index: of two candidates for the same pixel the larger word is the closer one, so
  * atomicMax keeps it and returns what it replaced, and joining two pixels (deb_join) is
- * lock-free: climb both to the roots of the lower pixel's level, hang the deeper root below
+ * lock-free (the merge of two root paths of Wilkinson et al., Concurrent computation of
+ * attribute filters on shared memory parallel machines, IEEE TPAMI 30(10), 2008, by atomicMax
+ * instead of under locks or phases): climb both to the roots of the lower pixel's level, hang
+ * the deeper root below
  * the other, go on with the other root and the parent that was replaced (or kept).  Every
  * step keeps, for each level, the components that the pairs joined so far (and the pairs in
  * hand) make up, so at the end the parents are the tree whatever the order.
@@ -380,8 +383,9 @@ __device__ inline int deb_sig_bound(double s, double sabs, int n, float b, doubl
  * pixels in 1024 lanes, 55 us for 6,000 in a dense frame), then one barrier per level.  The
  * levels were walked one by one before, with five passes over all pixels each (13 us a level
  * for 4,370 pixels).  Measured, before and after: crowded 4096^2, classes 0, 1, 2: 276, 167,
- * 229 -> 76, 50, 46 us; dense 2048^2, class 3 (40 objects of 6,000 to 18,000 pixels) 2,617 ->
- * 472 us with par and m in LDS (1,470 with all state in global memory).  Objects of more
+ * 229 -> 76, 50, 46 us; dense 2048^2, class 3 (40 objects of 6,000 to 20,000 pixels) 2,617 ->
+ * 472 us with par and m in LDS (1,470 with all state in global memory), 380 with the exact
+ * flux of the object ahead of those of its nodes.  Objects of more
  * pixels than that LDS holds (class 4) are built by the whole chip: k_deb_wide_levels.  Lanes: class 0 with
  * 64 lanes 138 us, class 1 with 256 lanes 73 us (more pixels a lane, one after the other).
  * Left out: the pixels entering level by level from the highest (each join is short then,
